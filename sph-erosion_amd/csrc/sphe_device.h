@@ -8,10 +8,11 @@
 //              scene's pad cell and is skipped by every physics kernel.
 //   cells      dense uniform grid per scene, x fastest, global keys
 //              [cell_off, cell_off + ncell) plus one pad cell at
-//              cell_off + ncell; start[] is the exclusive prefix of counts.
+//              cell_off + ncell; cells[].x is the exclusive prefix of counts.
 //   terrain    cells [t_off, t_off + tcap) per scene, row = z.
 #pragma once
 
+#include <hip/hip_runtime.h>
 #include <stdint.h>
 
 #define SPHE_WAVE 64
@@ -80,25 +81,27 @@ struct DevState {
     void* rho; void* posa;              // density; (x, y, z, p / rho^2) per sorted slot
     int32_t* key; uint32_t* arank;      // cell key << sub_log2 | x slab, arrival rank in the cell
     uint64_t* tmp_kid; int32_t* tmp_src;  // scatter output: (key, id) packed, previous slot
-    uint32_t* cnt; uint32_t* start; uint32_t* partial; int64_t npartial;
+    uint32_t* cnt; uint32_t* partial; int64_t npartial;
     // one word per scan tile of cnt (2^scan_log2 cells): set when a count
     // in the tile is taken, cleared by the scan that consumes the tile; the
     // scan reads the counts of flagged tiles only (the rest are zero)
     uint32_t* tocc;
-    // one word per scan tile of start: the value every start of the tile
+    // one word per scan tile of cells: the value every start of the tile
     // holds when the tile was last written empty, ~0 otherwise; the scan
     // leaves an empty tile unwritten when that value is still right
     uint32_t* tfill;
     int32_t scan_log2;  // cells per scan tile: 2^scan_log2
-    // cells are split into 2^sub_log2 slabs along x (sub_log2 <= 2); subw
-    // holds each cell's slab offsets (10 bits per inner boundary; bit 31:
-    // more than 1023 particles, no offsets), rewritten every step for the
-    // occupied cells (an empty cell's word may be stale: readers clamp the
-    // offsets to the cell)
-    uint32_t* subw; int32_t sub_log2;
+    // cell records (x: start, y: slab offsets): the scan writes (start, 0) and
+    // the reorder the offsets of the occupied cells.  Cells are split into
+    // 2^sub_log2 slabs along x (sub_log2 <= 2); y has 10 bits per inner
+    // boundary (bit 31: more than 1023 particles, no offsets).  One record
+    // beside the next, so a stencil row takes what it needs of a cell and of
+    // the next one's start with one load.
+    uint2* cells; int32_t sub_log2;
     // cells are 1/yz of the x edge along y and z (yz = 1, 2 or 3): the stencil
     // has (2 yz + 1)^2 rows
     int32_t yz;
+    int32_t h_unit;  // every scene's smoothing length is at most 1
     int64_t* vol; float* height;
     int64_t* dq; int32_t* tcell;        // two-phase erosion records
     uint32_t* tcnt; uint32_t* tstart; uint32_t* tpartial; int64_t ntpartial;
@@ -107,8 +110,9 @@ struct DevState {
     double* red;                        // reduction scratch
     int64_t nred;
     // neighbour lists written by the density pass for the force pass: the
-    // neighbours of sorted slot i (self excluded) in canonical order at
-    // nbl[i * maxn + m], m < min(nbc[i], maxn); a particle whose count
+    // neighbours of sorted slot i (self excluded) in canonical order from
+    // nbl[i * maxn] on, in chunks of 16 laid out by the lanes that read them
+    // (entry l + G u of a chunk at word l 16 / G + u); a particle whose count
     // exceeds maxn walks its stencil again in the force pass
     uint32_t* nbl;
     uint32_t* nbc;

@@ -25,10 +25,11 @@
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
-#include <map>
-#include <tuple>
 #include <algorithm>
+#include <map>
 #include <mutex>
+#include <tuple>
+#include <type_traits>
 
 #include "sphe_device.h"
 #include "sphe_launch.h"
@@ -343,9 +344,9 @@ __device__ __forceinline__ T gap_of(int d, int yz, T l1, T l2, T l3, T h1, T h2,
 
 // Slot range [j0, j1) of the row at (dy, dz); false when the row is outside
 // the grid or out of the sphere's reach.  roff = (dz ny + dy) nx, the row's
-// cell offset from the particle's own row (mod 2^32), kept by the callers.  The six table words a row may need
-// are loaded unconditionally (a skipped row reads the particle's own row),
-// so a row costs one memory round trip.
+// cell offset from the particle's own row (mod 2^32), kept by the callers.
+// The cell records a row may need are loaded unconditionally (a skipped row
+// reads the particle's own row), so a row costs one memory round trip.
 template <typename T>
 __device__ __forceinline__ bool row_range(const DevState& D, const SceneDev& S, const RowProbe<T>& P, int dyc,
                                           int dzc, uint32_t roff, uint32_t& j0, uint32_t& j1)
@@ -361,25 +362,21 @@ __device__ __forceinline__ bool row_range(const DevState& D, const SceneDev& S, 
     int fhi = cidx<T>(d_floor((P.gx + w) * P.scale), P.fmax);
     flo = max(flo, P.flo_min);
     fhi = min(fhi, P.fhi_max);
-    // cell indices are below 2^30 (the layout's limit): 32-bit offsets
     const uint32_t rk = on ? P.rbase + roff : P.rbase;
     const int sl = P.sl, smax = P.smax;
     const uint32_t clo = rk + (uint32_t)(flo >> sl), chi = rk + (uint32_t)(fhi >> sl);
-    const uint32_t s_lo = at(D.start, clo), s_lo1 = at(D.start, clo + 1);
-    const uint32_t s_hi = at(D.start, chi), s_hi1 = at(D.start, chi + 1);
-    const uint32_t w0 = at(D.subw, clo), w1 = at(D.subw, chi);
-    // slab offsets (none with one slab: slo = 0, shi = smax), clamped to the
-    // cell: an empty cell's word is not rewritten each step, and any value
-    // then gives its empty range; starts never decrease, so min(s_lo, s_lo1)
-    // is s_lo when there is no offset
+    const uint2 rlo = D.cells[clo], rhi = D.cells[chi];
+    const uint32_t s_hi1 = D.cells[(size_t)chi + 1].x;
+    // slab offsets (none with one slab: slo = 0, shi = smax); an empty cell's
+    // word is 0
     const int slo = flo & smax, shi = fhi & smax;
     // field shifts from byte tables: 10 (slo - 1) for slo = 1..3, 10 shi
     const uint32_t sh0 = (0x140A0000u >> ((uint32_t)slo << 3)) & 0xFFu;
     const uint32_t sh1 = (0x1E140A00u >> ((uint32_t)shi << 3)) & 0xFFu;
-    const uint32_t f0 = (slo != 0 && !(w0 >> 31)) ? (w0 >> sh0) & 1023u : 0u;
-    const bool use1 = shi != smax && !(w1 >> 31);
-    const uint32_t a = min(s_lo + f0, s_lo1);
-    const uint32_t b = use1 ? min(s_hi + ((w1 >> sh1) & 1023u), s_hi1) : s_hi1;
+    const uint32_t f0 = (slo != 0 && !(rlo.y >> 31)) ? (rlo.y >> sh0) & 1023u : 0u;
+    const bool use1 = shi != smax && !(rhi.y >> 31);
+    const uint32_t a = rlo.x + f0;
+    const uint32_t b = use1 ? rhi.x + ((rhi.y >> sh1) & 1023u) : s_hi1;
     // rows of real cells lie inside [p_begin, p_begin + n); the clamp only
     // matters if the counts were inconsistent
     const uint32_t lo = (uint32_t)S.p_begin, hi = (uint32_t)(S.p_begin + S.n);
@@ -528,6 +525,21 @@ __device__ __forceinline__ void load_run(const uint32_t* __restrict__ p, int64_t
     }
 }
 
+// The same as cell records (start, 0).
+template <int ITEMS>
+__device__ __forceinline__ void store_run(uint2* __restrict__ p, int64_t base, int64_t n, const uint32_t* v)
+{
+    if (base + ITEMS <= n) {
+        uint4* q = (uint4*)(p + base);
+#pragma unroll
+        for (int k = 0; k < ITEMS / 2; ++k) q[k] = make_uint4(v[2 * k], 0u, v[2 * k + 1], 0u);
+    } else {
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i)
+            if (base + i < n) p[base + i] = make_uint2(v[i], 0u);
+    }
+}
+
 template <int ITEMS>
 __device__ __forceinline__ void store_run(uint32_t* __restrict__ p, int64_t base, int64_t n, const uint32_t* v)
 {
@@ -628,8 +640,9 @@ __global__ __launch_bounds__(1024) void k_scan_tiles(uint32_t* __restrict__ part
 // fill (optional, with occ): per tile, the value all of an empty tile's
 // starts hold since the tile was last written empty (~0: not known); an
 // empty tile whose prefix equals it is not written again.
-template <int ITEMS>
-__global__ __launch_bounds__(256) void k_scan_down(uint32_t* __restrict__ cnt, uint32_t* __restrict__ start,
+// S: what a start is written as, a plain word or a cell record (start, 0).
+template <int ITEMS, typename S>
+__global__ __launch_bounds__(256) void k_scan_down(uint32_t* __restrict__ cnt, S* __restrict__ start,
                                                    int64_t n, const uint32_t* __restrict__ partial,
                                                    int zero_counts, unsigned long long* __restrict__ zero,
                                                    unsigned long long zero_to,
@@ -689,7 +702,7 @@ __global__ __launch_bounds__(256) void k_scatter(DevState D)
         return;
     }
     const uint32_t r = D.arank[p];
-    const uint32_t d = D.start[c] + r;
+    const uint32_t d = D.cells[c].x + r;
     // the cell's count is used up: its first arrival (one per counted cell)
     // resets it for the next step's arrivals
     if (r == 0u) D.cnt[c] = 0u;
@@ -732,8 +745,9 @@ __global__ __launch_bounds__(256) void k_reorder(DevState D)
         c = fk >> sl;
         ok = fk >= 0 && (int64_t)c < D.C;
         if (ok) {
-            s0 = D.start[c];
-            s1 = (int64_t)D.start[c + 1] <= D.P ? D.start[c + 1] : (uint32_t)D.P;
+            s0 = D.cells[c].x;
+            s1 = D.cells[(size_t)c + 1].x;
+            if ((int64_t)s1 > D.P) s1 = (uint32_t)D.P;
         }
     }
     if (threadIdx.x == 0) {
@@ -806,7 +820,7 @@ __global__ __launch_bounds__(256) void k_reorder(DevState D)
         atomicOr(D.status, 2u);
         return;
     }
-    if (rank == 0) D.subw[c] = s1 - s0 > 1023u ? 0x80000000u : below;
+    if (rank == 0) D.cells[c].y = s1 - s0 > 1023u ? 0x80000000u : below;
     ((V4<T>*)D.s_pos)[f] = pv;
     ((V4<T>*)D.s_vel)[f] = vv;
     D.s_sed[f] = sed;
@@ -879,15 +893,76 @@ __host__ __device__ constexpr int density_lds_bytes(int W, int ngroups, int ring
     return density_ring_offset(W, ngroups, ring) + ngroups * ring * 4;
 }
 
+// Where list positions c0 .. c0+15 (c0 a multiple of 16) of a particle go: its
+// list of cap entries, then the group's pool chunk of ocap entries, claimed by
+// the first call past cap (one 64-bit atomic; none left: null, the claim
+// failure is counted and the force pass walks the stencil).  Called by all G
+// lanes of the group; lane l == 0 is lane gfirst of the wave.
+struct ListOut {
+    uint32_t* nbl;
+    uint32_t cap, pb = ~0u;  // pb: the group's chunk in the pool (none yet)
+    bool claimed = false;    // the group asked for a chunk (at most once)
+    __device__ __forceinline__ uint32_t* chunk(const DevState& D, uint32_t c0, int l, int gfirst)
+    {
+        if (c0 < cap) return nbl + c0;
+        const uint32_t ocap = (uint32_t)D.ocap;
+        if (!claimed) {
+            claimed = true;
+            uint32_t b0 = ~0u;
+            if (l == 0) {
+                const unsigned long long t = atomicAdd(D.ptop, (unsigned long long)ocap);
+                b0 = t + ocap <= (unsigned long long)D.pool_cap ? (uint32_t)(t / SPHE_POOL_UNIT) : ~0u;
+                if (b0 == ~0u) atomicAdd(&D.ovf[1], 1u);
+            }
+            pb = __shfl(b0, gfirst, SPHE_WAVE);
+        }
+        return pb != ~0u && c0 - cap < ocap ? D.pool + (size_t)pb * SPHE_POOL_UNIT + (c0 - cap) : nullptr;
+    }
+};
+
+// The end of the density pass: the largest count past the lists (one atomic
+// per wave: the lanes still here; the loop over the overflowing groups is
+// wave-uniform), then lane 0 of the group writes the particle's outputs.
+template <typename T>
+__device__ __forceinline__ void density_out(const DevState& D, const SceneConsts<T>& K, int64_t slot, int l,
+                                            const V4<T>& pi, T sum, uint32_t cnt, uint32_t cap, uint32_t pb)
+{
+    uint64_t over = __ballot(cnt > cap);
+    if (over) {
+        uint32_t mx = 0;
+        for (; over; over &= over - 1) {
+            const uint32_t c = (uint32_t)__shfl(cnt, __ffsll((unsigned long long)over) - 1, SPHE_WAVE);
+            mx = c > mx ? c : mx;
+        }
+        const uint64_t here = __ballot(1);
+        if ((int)(threadIdx.x & (SPHE_WAVE - 1)) == __ffsll((unsigned long long)here) - 1) atomicMax(D.ovf, mx);
+    }
+    if (l != 0) return;
+    D.nbc[slot] = cnt;
+    D.pbase[slot] = pb;
+    const T rho = sum * K.mc6;
+    const T p = K.k * (rho - K.rho0);
+    ((T*)D.rho)[slot] = rho;
+    // (x, y, z, p / rho^2) and vel.w = m / rho: what the force pass gathers
+    // per neighbour, in two 16-byte loads
+    V4<T> pa = pi;
+    pa.w = p / (rho * rho);
+    ((V4<T>*)D.posa)[slot] = pa;
+    ((T*)D.s_vel)[4 * slot + 3] = K.mass / rho;
+}
+
 // One G-lane group per particle (lane l = thread index mod G).  The clipped
 // stencil rows form one stream of candidates; lane l takes stream positions
 // l, l+G, ... (U = SPHE_DENSITY_UNROLL per iteration) for its share of the
 // density sum.
 // The group writes one neighbour list per particle (self left out) in
-// canonical order, nbl[slot * maxn + m], m < maxn, count in nbc[slot]; a
-// byte-wise prefix sum over the group places each lane's entries in a ring
-// in LDS, and every completed chunk of 16 entries goes out with one 16-byte
-// store per lane (64-byte aligned: one cache line per group).  List
+// canonical order, in chunks of 16 entries from nbl[slot * maxn] on, count in
+// nbc[slot]; a byte-wise prefix sum over the group places each lane's entries
+// in a ring in LDS, and every completed chunk goes out with one 16-byte store
+// per lane (64-byte aligned: one cache line per group).  A chunk is stored by
+// the lane that will read it: its entry e = l + G u lies at word l (16 / G)
+// + u, so a force lane takes its four neighbours of an iteration
+// with one 16-byte load.  List
 // entries are byte offsets of the neighbours' slots in the per-slot vectors
 // of V4<T> (slot * sizeof(V4<T>), below 2^32 by the layout's limits).  The
 // group then merges the partial sums and lane 0 writes rho and
@@ -907,13 +982,11 @@ __device__ __forceinline__ void density_body(const DevState& D, int b)
     Acc<T, SM != SUM_PLAIN> sum;
     const T h2 = K.h2, thr = K.thr;
     const uint32_t cap = (uint32_t)D.maxn;
-    uint32_t* __restrict__ nbl = D.nbl + slot * (int64_t)D.maxn;
+    ListOut out{D.nbl + slot * (int64_t)D.maxn, cap};
     constexpr uint32_t VB = (uint32_t)sizeof(V4<T>);  // bytes per slot of a V4<T> vector
     const uint32_t self = (uint32_t)slot * VB;          // as a byte offset
     const int gfirst = (int)(threadIdx.x & (SPHE_WAVE - 1)) & ~(G - 1);  // the group's first lane in the wave
     uint32_t cnt = 0;      // the same in every lane of the group
-    uint32_t pb = ~0u;     // the group's overflow chunk in the pool (none yet)
-    bool claimed = false;  // the group asked for a chunk (at most once)
     uint32_t stream_total = 0;
     // The particle's clipped rows as one stream of candidates, t = 0 ..
     // total-1 in canonical order.  Lane l computes rows l, l+G, ... (the
@@ -983,51 +1056,28 @@ __device__ __forceinline__ void density_body(const DevState& D, int b)
         const uint2* cur = tab - 1;         // the current row's entry (none yet)
         uint32_t cur_end = 0, cur_off = 0;  // its stream end and slot offset
         const uint32_t lane_b = (uint32_t)l * VB;
-        // Writes list positions c0 .. c0+n-1 (c0 a multiple of 16, n <= 16)
-        // from the ring: lane l copies positions c0 + l PER .. + PER-1, as
-        // 16-byte (G = 8: 8-byte) stores of whole chunks.  The list (capacity
-        // cap, a multiple of 16) continues in the group's pool chunk of ocap
-        // entries (a multiple of 16), claimed when the first chunk past cap is
-        // written (one 64-bit atomic; none left: the rest is not stored, the
-        // claim failure is counted and the force pass walks the stencil); the
-        // list rows and pool chunks are 64-byte aligned.  Called by all lanes
-        // of the group.
-        const uint32_t ocap = (uint32_t)D.ocap;
-        auto flush = [&](uint32_t c0, uint32_t n) {
+        // Writes the chunk of 16 list positions from c0 (a multiple of 16) on
+        // from the ring: lane l copies positions c0 + l, c0 + l + G, ... to
+        // words l PER .. of the chunk, with 16-byte (G = 8: 8-byte) stores.  Of
+        // the last, partial chunk the words past the count are written with
+        // whatever the ring holds and never read.  The list rows and pool
+        // chunks are 64-byte aligned.  Called by all lanes of the group.
+        auto flush = [&](uint32_t c0) {
             constexpr int PER = 16 / G;
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-            uint32_t* dst = nullptr;
-            if (c0 < cap) {
-                dst = nbl + c0;
-            } else {
-                if (!claimed) {
-                    claimed = true;
-                    uint32_t b0 = ~0u;
-                    if (l == 0) {
-                        const unsigned long long t = atomicAdd(D.ptop, (unsigned long long)ocap);
-                        b0 = t + ocap <= (unsigned long long)D.pool_cap ? (uint32_t)(t / SPHE_POOL_UNIT) : ~0u;
-                        if (b0 == ~0u) atomicAdd(&D.ovf[1], 1u);
-                    }
-                    pb = __shfl(b0, gfirst, SPHE_WAVE);
-                }
-                if (pb != ~0u && c0 - cap < ocap) dst = D.pool + (size_t)pb * SPHE_POOL_UNIT + (c0 - cap);
-            }
+            uint32_t* dst = out.chunk(D, c0, l, gfirst);
             if (dst) {
-                const uint32_t* src = (const uint32_t*)((char*)rowtab + (ring_rel | ((c0 * 4u) & RMASK))) + l * PER;
-                uint32_t* out = dst + l * PER;
-                if (n == 16u) {
-                    if constexpr (PER >= 4) {
+                const uint32_t* src = (const uint32_t*)((char*)rowtab + (ring_rel | ((c0 * 4u) & RMASK))) + l;
+                dst += l * PER;
+                if constexpr (PER >= 4) {
 #pragma unroll
-                        for (int k = 0; k < PER; k += 4) *(uint4*)(out + k) = *(const uint4*)(src + k);
-                    } else {
-                        *(uint2*)out = *(const uint2*)src;
-                    }
+                    for (int k = 0; k < PER; k += 4)
+                        *(uint4*)(dst + k) =
+                            make_uint4(src[k * G], src[(k + 1) * G], src[(k + 2) * G], src[(k + 3) * G]);
                 } else {
-#pragma unroll
-                    for (int k = 0; k < PER; ++k)
-                        if ((uint32_t)(l * PER + k) < n) out[k] = src[k];
+                    *(uint2*)dst = make_uint2(src[0], src[G]);
                 }
             }
             // the ring slots read here are written again only by later blocks
@@ -1098,50 +1148,455 @@ __device__ __forceinline__ void density_body(const DevState& D, int b)
             // cnt (one at most when a block holds 16 positions or fewer)
             if constexpr (U * G <= 16) {
                 const uint32_t c0 = cnt & ~15u;
-                if (c0 + 16u <= ncnt) flush(c0, 16u);
+                if (c0 + 16u <= ncnt) flush(c0);
             } else {
-                for (uint32_t c0 = cnt & ~15u; c0 + 16u <= ncnt; c0 += 16u) flush(c0, 16u);
+                for (uint32_t c0 = cnt & ~15u; c0 + 16u <= ncnt; c0 += 16u) flush(c0);
             }
             cnt = ncnt;
         };
         uint32_t base = 0;
         for (; base + U * G <= total; base += U * G) block(base, std::false_type());
         if (base < total) block(base, std::true_type());
-        if (cnt & 15u) flush(cnt & ~15u, cnt & 15u);  // the last, partial chunk
+        if (cnt & 15u) flush(cnt & ~15u);  // the last, partial chunk
     }
     group_merge<G>(sum);
-    {
-        // the largest count past the list: one atomic per wave (the lanes
-        // still here; the loop over the overflowing groups is wave-uniform)
-        uint64_t over = __ballot(cnt > cap);
-        if (over) {
-            uint32_t mx = 0;
-            for (; over; over &= over - 1) {
-                const uint32_t c = (uint32_t)__shfl(cnt, __ffsll((unsigned long long)over) - 1, SPHE_WAVE);
-                mx = c > mx ? c : mx;
-            }
-            const uint64_t here = __ballot(1);
-            if ((int)(threadIdx.x & (SPHE_WAVE - 1)) == __ffsll((unsigned long long)here) - 1) atomicMax(D.ovf, mx);
-        }
-    }
-    if (l != 0) return;
-    D.nbc[slot] = cnt;
-    D.pbase[slot] = pb;
-    const T rho = sum.value() * K.mc6;
-    const T p = K.k * (rho - K.rho0);
-    ((T*)D.rho)[slot] = rho;
-    // (x, y, z, p / rho^2) and vel.w = m / rho: what the force pass gathers
-    // per neighbour, in two 16-byte loads
-    V4<T> pa = pi;
-    pa.w = p / (rho * rho);
-    ((V4<T>*)D.posa)[slot] = pa;
-    ((T*)D.s_vel)[4 * slot + 3] = K.mass / rho;
+    density_out<T>(D, K, slot, l, pi, sum.value(), cnt, cap, out.pb);
 }
 
 template <typename T, int SM, int G>
 __global__ __launch_bounds__(512) void k_density(DevState D, int nblk, int remap)
 {
     density_body<T, SM, G>(D, xcd_block(blockIdx.x, nblk, remap));
+}
+
+// The density pass for four lanes a particle and cubic or halved cells (YZ =
+// 1 or 2): the same streams, sums and lists as density_body, bit for bit, in
+// two thirds to nine tenths of its time: 18.0 -> 10.5 us on a dam break of
+// 4,096 particles, 88.5 -> 66 us on a settled column of 262,144, 162 -> 143 us
+// on 48 settled scenes of 877,000 in all (cubic cells), 1,443 -> 1,273 us on a
+// settled layer of 4,194,304.  density_body serves the other lane counts,
+// thirds of cells and the persistent launch.
+//
+// Measured rates here (cycles a wave64 instruction a SIMD): plain FP32 and
+// integer adds, multiplies, logic and right shifts on VGPRs or literals 2.4;
+// min / max, compares, selects, bit counts, DPP, conversions, anything with
+// an SGPR operand 4.4.  The pass is bound by issue, so:
+// * Rows are set up plane by plane: lane l takes the rows dy = l - YZ of each
+//   plane, whose y gap is the lane's own constant and whose z gap the plane's,
+//   with the fifth row of each plane (YZ = 2) in the lanes of two more rounds.
+//   A row or plane outside the grid has gap 2 (out of reach).  Two loads of
+//   cell records a row.
+// * The table of the rows that hold candidates has the offset from stream
+//   position to slot and the first position of each; a bit per stream position
+//   marks where a row starts.  A block's row of position p is then a bit count
+//   of the block's marks up to p, with no walk along the table and no chain
+//   of LDS reads.  The marks cover a segment of SPHE_SEG positions and are
+//   set again from the table for each further segment.
+// * A candidate's place in the list is a bit count of the block's accepted
+//   positions up to it (the quad's 16 bits or-ed together with two DPP ors).
+//   The entries are staged in a 32-word buffer that is moved down by 16 words
+//   when its first chunk is written out, so a place is one shift and add.
+// * The particle's own slot is looked for only in blocks where a group of the
+//   wave has its own.
+// * The accept masks stay in scalar registers (ballots): as booleans over the
+//   branch around the own-slot test they became a byte per lane, 16 more
+//   instructions a block.
+// * Six waves a SIMD (80 registers): with 72 or 64 the loop spills (1,449 and
+//   1,886 us on the layer).
+// UNIT: every smoothing length is at most 1, so h^2 - d2 can be clamped to
+// [0, 1] by the subtraction's own modifier instead of a max.
+#define SPHE_SEG 256  // 6.4 KB of LDS a wave with 5x5 rows: no limit to six waves a SIMD
+constexpr int QUAD_STAGE = 128;                 // bytes of a group's staging buffer
+constexpr int QUAD_MARKS = SPHE_SEG / 8 + 16;   // marks (and the prefetch past them)
+__host__ __device__ constexpr int quad_group_bytes(int yz)
+{
+    // 16 bytes more than needed: a stride of 100 or 68 words puts the same
+    // word of a wave's 16 groups in different banks
+    return QUAD_STAGE + QUAD_MARKS + ((2 * yz + 1) * (2 * yz + 1) * 8 + 15) / 16 * 16 + 16;
+}
+
+typedef __attribute__((address_space(3))) uint16_t lds_u16;
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) u32x2 lds_u32x2;
+template <typename P>
+__device__ __forceinline__ P* lds_at(uint32_t addr) { return (P*)(uintptr_t)addr; }
+
+// A uniform value in a VGPR: an operand that costs the full-rate form.
+__device__ __forceinline__ float in_vgpr(float x) { asm volatile("" : "+v"(x)); return x; }
+__device__ __forceinline__ double in_vgpr(double x) { asm volatile("" : "+v"(x)); return x; }
+
+template <int CTRL>
+__device__ __forceinline__ uint32_t quad_dpp(uint32_t x)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, CTRL, 0xF, 0xF, true);
+}
+// sum of x over the lanes of the quad up to this one (m1, m2: all ones in
+// lanes 1.. and 2..), and the quad's total
+__device__ __forceinline__ uint32_t quad_prefix(uint32_t x, uint32_t m1, uint32_t m2, uint32_t* tot)
+{
+    uint32_t y = x + (quad_dpp<0x90>(x) & m1);  // quad_perm [0,0,1,2]
+    y += quad_dpp<0x40>(y) & m2;                // quad_perm [0,0,0,1]
+    *tot = quad_dpp<0xFF>(y);                   // quad_perm [3,3,3,3]
+    return y;
+}
+
+// max(x, 0); UNIT: x <= 1, as the clamp of the instruction that makes x
+template <bool UNIT>
+__device__ __forceinline__ float pos_part(float x)
+{
+    return UNIT ? __builtin_amdgcn_fmed3f(x, 0.f, 1.f) : (x > 0.f ? x : 0.f);
+}
+template <bool UNIT>
+__device__ __forceinline__ double pos_part(double x) { return x > 0.0 ? x : 0.0; }
+
+// floor(x) clamped to [lo, hi] (exact integers below 2^24), NaN giving lo
+__device__ __forceinline__ int floor_clamp(float x, float lo, float hi)
+{
+    return (int)__builtin_amdgcn_fmed3f(__builtin_floorf(x), lo, hi);
+}
+__device__ __forceinline__ int floor_clamp(double x, double lo, double hi)
+{
+    return (int)d_fmin(d_fmax(d_floor(x), lo), hi);
+}
+
+// The half-width of a row plus its margin, times the slab count s (a power of
+// two, so every step is RowWidth's scaled exactly): s (width(x) + margin).
+__device__ __forceinline__ float row_width(float x, float s, float s15, float sm)
+{
+    float y = __int_as_float(0x5f375a86 - (__float_as_int(x) >> 1));
+    const float t = ((0.5f * x) * s) * y;
+    y = y * __builtin_fmaf(-t, y, s15);
+    return x * y + sm;
+}
+__device__ __forceinline__ double row_width(double x, double s, double, double sm) { return d_sqrt(x) * s + sm; }
+
+// Orders the wave's LDS accesses before against those after (the lanes of a
+// group are one wave's, and a wave's LDS accesses are done in order).
+__device__ __forceinline__ void wave_order()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <typename T, int SM, int YZ, bool UNIT>
+__device__ __forceinline__ void density_quad(const DevState& D, int b)
+{
+    constexpr int W = 2 * YZ + 1;
+    constexpr uint32_t VB = (uint32_t)sizeof(V4<T>);
+    const int64_t gt = (int64_t)b * blockDim.x + threadIdx.x;
+    const int l = (int)(threadIdx.x & 3);
+    const int lane = (int)(threadIdx.x & (SPHE_WAVE - 1));
+    // the wave's first slot (slots are below 2^30; P is a multiple of 64, so
+    // waves are whole)
+    const uint32_t wslot = __builtin_amdgcn_readfirstlane((uint32_t)(gt >> 6)) * 16u;
+    if (wslot >= (uint64_t)D.P) return;
+    const uint32_t slot = wslot + (uint32_t)(lane >> 2);
+    const SceneDev& S = D.scenes[wave_scene(D.chunk_scene, wslot)];
+    const uint32_t lo = (uint32_t)S.p_begin, hi = (uint32_t)(S.p_begin + S.n);
+    if (wslot >= hi) return;  // only padding
+    const SceneConsts<T>& K = SceneSel<T>::get(S);
+    const V4<T>* __restrict__ pos = (const V4<T>*)D.s_pos;
+    const uint32_t self = slot * VB;
+    const uint32_t cap = (uint32_t)D.maxn;
+    ListOut out{D.nbl + slot * (int64_t)D.maxn, cap};
+    const int gfirst = lane & ~3;
+    const uint32_t m1 = l >= 1 ? ~0u : 0u, m2 = l >= 2 ? ~0u : 0u;
+
+    // the group's LDS: staging buffer, marks, row table
+    extern __shared__ __attribute__((aligned(256))) uint2 rowtab[];
+    constexpr uint32_t GB = (uint32_t)quad_group_bytes(YZ);
+    const uint32_t stage = (uint32_t)(uintptr_t)rowtab + (threadIdx.x >> 2) * GB;
+    const uint32_t marks = stage + QUAD_STAGE;
+    const uint32_t tab = marks + QUAD_MARKS;
+
+    // positions p = 4 u + l of a block, u = 0..3: the bits up to p
+    uint32_t upto[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) upto[u] = (2u << (4 * u + l)) - 1u;
+
+    Acc<T, SM != SUM_PLAIN> sum;
+    const T h2 = in_vgpr(K.h2);
+    const T thr = K.thr;
+    uint32_t rows = 0;     // marks before the current block: rows started
+    uint32_t placed = ~0u; // entries in the staging buffer, less 1
+    uint32_t done = 0;     // entries written out
+    uint32_t total = 0;    // candidates of the stream
+    uint32_t selfpos = 0;  // this lane's stream position of the particle itself (~0: another lane's)
+
+    // Sets the mark of stream position p of the segment.
+    auto mark = [&](uint32_t p) {
+        if (p < SPHE_SEG)
+            (void)__hip_atomic_fetch_or(lds_at<lds_u32>(marks + (p >> 5) * 4u), 1u << (p & 31u), __ATOMIC_RELAXED,
+                                        __HIP_MEMORY_SCOPE_WAVEFRONT);
+    };
+    auto clear_marks = [&]() {
+        *lds_at<lds_u32x2>(marks + 8u * (uint32_t)l) = u32x2{0u, 0u};
+        static_assert(SPHE_SEG / 8 == 32, "one 8-byte store a lane");
+        wave_order();
+    };
+    // The clipped rows: a table of those that hold candidates, and the marks of
+    // the first segment.
+    // The rows' slot ranges are found with the lanes laid out by quarters of
+    // the wave: lane 16 qr + g does rows of particle g, so that 16 lanes in a
+    // row read cell records of neighbouring cells (a load of a wave touches a
+    // few lines instead of 64; the L1 does one line access a cycle, and the
+    // pass is close to that limit).  They go through the table's memory to the
+    // quads.
+    uint32_t nrows;
+    {
+        const int qr = lane >> 4;
+        const int nx = S.dims[0], ny = S.dims[1], nz = S.dims[2], nyx = ny * nx;
+        const int sl = D.sub_log2, smax = (1 << sl) - 1;
+        const T s = T(1 << sl), q = K.yz_scale;
+        const V4<T> pr = pos[wslot + (lane & 15)];
+        const T gx = (pr.x - K.org[0]) * K.inv_cell;
+        const T gy = (pr.y - K.org[1]) * K.inv_yz, gz = (pr.z - K.org[2]) * K.inv_yz;
+        const int kx = cidx<T>(d_floor(gx), nx - 1);
+        const int ky = cidx<T>(d_floor(gy), ny - 1);
+        const int kz = cidx<T>(d_floor(gz), nz - 1);
+        const uint32_t rbase = (uint32_t)S.cell_off + (uint32_t)((kz * ny + ky) * nx);
+        const T fy = gy - T(ky), fz = gz - T(kz);
+        // squared gap to the rows or planes d cells away; out of the grid: 4
+        auto gap2 = [&](T f, int k, int n, int d) {
+            if (d == 0) return T(0);
+            const T g = row_gap<T>((d == -1 ? f : d == 1 ? T(1) - f : d == -2 ? T(1) + f : T(1) + (T(1) - f)) * q);
+            return (d < 0 ? k >= -d : k + d < n) ? g * g : T(4);
+        };
+        T mz[W];
+#pragma unroll
+        for (int k = 0; k < W; ++k) mz[k] = gap2(fz, kz, nz, k - YZ);
+        // the lane's rows dy = qr - YZ (YZ = 1: quarter 3 has none)
+        T my = gap2(fy, ky, ny, -YZ);
+        if (qr == 1) my = gap2(fy, ky, ny, 1 - YZ);
+        if (qr == 2) my = gap2(fy, ky, ny, 2 - YZ);
+        if (qr == 3) my = YZ == 1 ? T(4) : gap2(fy, ky, ny, 1);
+        const uint32_t rlane = rbase + (uint32_t)((qr - YZ) * nx);
+        const T gs = gx * s, s15 = T(1.5) * s, sm = T(SPHE_ROW_MARGIN) * s;
+        // slabs of the cells kx - 1 .. kx + 1 inside the grid
+        const T flo_min = T((kx > 0 ? kx - 1 : 0) << sl), fmax = T((nx << sl) - 1);
+        const T fhi_max = T(((kx < nx - 1 ? kx + 1 : nx - 1) << sl) + smax);
+        // offset shifts by the low two bits of a slab index, from byte tables:
+        // 10 (slab - 1) for the first slab taken (30, an empty field, for slab
+        // 0), 10 slab for the last
+        const uint32_t tlo = sl == 2 ? 0x140A001Eu : (sl == 1 ? 0x001E001Eu : 0x1E1E1E1Eu);
+        const uint32_t thi = sl == 2 ? 0x1E140A00u : (sl == 1 ? 0x1E001E00u : 0x1E1E1E1Eu);
+        const uint32_t raw = (uint32_t)(uintptr_t)rowtab + ((threadIdx.x >> 2 & ~15u) + (uint32_t)(lane & 15)) * GB +
+                             QUAD_STAGE + QUAD_MARKS;  // the table of the lane's particle here
+        auto row = [&](int at, T r2, uint32_t cell) {
+            const bool on = r2 <= T(1);
+            const T w = row_width(T(1) - r2, s, s15, sm);
+            const int flo = floor_clamp(gs - w, flo_min, fmax), fhi = floor_clamp(gs + w, T(0), fhi_max);
+            const uint32_t rk = on ? cell : rbase;
+            const uint2* clo = D.cells + (rk + (uint32_t)(flo >> sl));
+            const uint2* chi = D.cells + (rk + (uint32_t)(fhi >> sl));
+            const uint2 a = clo[0], c = chi[0];
+            const uint32_t c1 = chi[1].x;
+            const uint32_t slo = tlo >> (((uint32_t)flo << 3) & 31u), shi = thi >> (((uint32_t)fhi << 3) & 31u);
+            const uint32_t first = a.x + __builtin_amdgcn_ubfe(a.y & 0x3FFFFFFFu, slo, 10);
+            const bool whole = (fhi & smax) == smax || (int32_t)c.y < 0;
+            const uint32_t last = c.x + __builtin_amdgcn_ubfe(c.y, shi, 10);
+            const uint32_t e = min(whole ? c1 : last, hi);
+            const uint32_t j = max(first, lo);
+            *lds_at<lds_u32x2>(raw + 8u * (uint32_t)at) = u32x2{j, on && e > j ? e - j : 0u};
+        };
+#pragma unroll
+        for (int k = 0; k < W; ++k) {
+            if (qr < W) row(k * W + qr, my + mz[k], rlane + (uint32_t)((k - YZ) * nyx));
+            if (k == 3) __builtin_amdgcn_sched_barrier(0);  // four rows' loads in flight: fewer registers
+        }
+        if constexpr (YZ == 2) {
+            const T m5 = gap2(fy, ky, ny, 2);
+            row(qr * W + 4, m5 + (qr == 0 ? mz[0] : qr == 1 ? mz[1] : qr == 2 ? mz[2] : mz[3]),
+                rbase + (uint32_t)((qr - 2) * nyx + 2 * nx));
+            if (qr == 0) row(4 * W + 4, m5 + mz[4], rbase + (uint32_t)(2 * nyx + 2 * nx));
+        }
+    }
+    if (slot >= hi) return;  // padding: whole groups leave together
+    const V4<T> pi = pos[slot];
+    {
+        clear_marks();
+        constexpr int NR = YZ == 1 ? 3 : 7;  // the planes' rows l, then the fifth rows
+        uint32_t j0[NR], len[NR];
+        auto take = [&](int k, bool have, int at) {
+            const u32x2 e = *lds_at<lds_u32x2>(tab + 8u * (uint32_t)at);
+            j0[k] = e.x;
+            len[k] = have ? e.y : 0u;
+        };
+#pragma unroll
+        for (int k = 0; k < W; ++k) take(k, l < W, k * W + (l < W ? l : 0));
+        if constexpr (YZ == 2) {
+            take(5, true, l * W + 4);
+            take(6, l == 0, 4 * W + 4);
+        }
+        wave_order();
+        // place of each row that holds candidates among them: 6-bit fields, one
+        // a plane, of the lane's own rows; prefixes over the quad, then planes
+        uint32_t has = 0, fifth = 0;
+#pragma unroll
+        for (int k = 0; k < W; ++k) has |= (len[k] != 0u ? 1u : 0u) << (6 * k);
+        uint32_t htot;
+        uint32_t place = quad_prefix(has, m1, m2, &htot) - has;
+        if constexpr (YZ == 2) {
+            const uint32_t f5 = len[5] != 0u ? 1u : 0u, f6 = len[6] != 0u ? 1u : 0u;
+            fifth = quad_dpp<0x00>(f5) | quad_dpp<0x55>(f5) << 6 | quad_dpp<0xAA>(f5) << 12 |
+                    quad_dpp<0xFF>(f5) << 18 | quad_dpp<0x00>(f6) << 24;
+        }
+        // rows of the planes before: running sums of the planes' totals
+        const uint32_t before = ((htot + fifth) * 0x01041041u) << 6;
+        place += before;
+        nrows = ((before + htot + fifth) >> (6 * (W - 1))) & 63u;
+        // stream starts, the table and the marks
+        uint32_t ends = 0, s5 = 0, p5 = 0;
+        auto put = [&](uint32_t at, uint32_t start, int k) {
+            if (len[k] == 0u) return;
+            *lds_at<lds_u32x2>(tab + 8u * at) = u32x2{start, (j0[k] - start) * VB};
+            mark(start);
+        };
+#pragma unroll
+        for (int k = 0; k < W; ++k) {
+            uint32_t tot;
+            const uint32_t st = ends + quad_prefix(len[k], m1, m2, &tot) - len[k];
+            if (k == YZ)  // the particle's own row: dy = 0 is lane YZ's
+                selfpos = quad_dpp<YZ * 0x55>(slot - j0[k] + st);
+            put((place >> (6 * k)) & 63u, st, k);
+            ends += tot;
+            if constexpr (YZ == 2) {
+                const uint32_t at5 = ((before + htot) >> (6 * k)) & 63u;
+                const uint32_t l5 = k == 0   ? quad_dpp<0x00>(len[5])
+                                    : k == 1 ? quad_dpp<0x55>(len[5])
+                                    : k == 2 ? quad_dpp<0xAA>(len[5])
+                                    : k == 3 ? quad_dpp<0xFF>(len[5])
+                                             : quad_dpp<0x00>(len[6]);
+                if (k < 4) {
+                    if (l == k) {
+                        s5 = ends;
+                        p5 = at5;
+                    }
+                } else if (l == 0) {
+                    put(at5, ends, 6);
+                }
+                ends += l5;
+            }
+        }
+        if constexpr (YZ == 2) put(p5, s5, 5);
+        selfpos = (selfpos & 3u) == (uint32_t)l ? selfpos : ~0u;
+        total = ends;
+        wave_order();
+    }
+
+    // Writes the first 16 staged entries out, lane l its entries l, l + 4, ...
+    // with one 16-byte store, and moves the rest down.
+    auto flush = [&]() {
+        wave_order();
+        const uint32_t at = stage + 4u * (uint32_t)l;
+        const u32x4 e = {*lds_at<lds_u32>(at), *lds_at<lds_u32>(at + 16u), *lds_at<lds_u32>(at + 32u),
+                         *lds_at<lds_u32>(at + 48u)};
+        const u32x4 rest = *lds_at<lds_u32x4>(stage + 64u + 16u * (uint32_t)l);
+        wave_order();
+        *lds_at<lds_u32x4>(stage + 16u * (uint32_t)l) = rest;
+        uint32_t* dst = out.chunk(D, done, l, gfirst);
+        if (dst) *(u32x4*)(dst + 4 * l) = e;
+        done += 16u;
+        placed -= 16u;
+        wave_order();
+    };
+
+    // The slots of the block at t (positions t + 4 u + l), looked up while the
+    // block before is computed; a new segment's marks are set from the table
+    // first.  Past the stream's end they are slots of its last row or beyond.
+    uint32_t t = 0, jn[4];
+    uint32_t mk = *lds_at<lds_u16>(marks), mnext = marks + 2u;
+    auto lookup = [&](uint32_t at) {
+        if (at != 0u && at % SPHE_SEG == 0u && at < total) {
+            wave_order();
+            clear_marks();
+            for (uint32_t r = (uint32_t)l; r < nrows; r += 4u) mark(*lds_at<lds_u32>(tab + 8u * r) - at);
+            wave_order();
+            mk = *lds_at<lds_u16>(marks);
+            mnext = marks + 2u;
+        }
+        const uint32_t m = mk;
+        mk = *lds_at<lds_u16>(mnext);
+        mnext += 2u;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const uint32_t r = (uint32_t)__popc(m & upto[u]) + rows;      // rows started up to the position
+            const uint32_t off = *lds_at<lds_u32>((r << 3) + (tab - 4u));  // row r - 1's
+            jn[u] = off + (at * VB + (uint32_t)l * VB) + (uint32_t)(4 * u) * VB;
+        }
+        rows += (uint32_t)__popc(m);
+    };
+    auto block = [&](auto tail) {
+        constexpr bool TAIL = decltype(tail)::value;
+        uint32_t jj[4];
+        V4<T> p[4];
+        uint64_t ok[4];  // lanes with a candidate
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            jj[u] = jn[u];
+            if constexpr (TAIL) {
+                ok[u] = __builtin_amdgcn_ballot_w64(t + (uint32_t)(4 * u + l) < total);
+                jj[u] = __builtin_amdgcn_inverse_ballot_w64(ok[u]) ? jj[u] : self;
+            }
+            p[u] = at_byte(pos, jj[u]);
+        }
+        if constexpr (!TAIL) lookup(t + 16u);
+        T part = T(0);
+        uint64_t in[4];  // lanes whose candidate is inside the radius
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const T dx = pi.x - p[u].x, dy = pi.y - p[u].y, dz = pi.z - p[u].z;
+            const T d2 = (dx * dx + dy * dy) + dz * dz;
+            in[u] = __builtin_amdgcn_ballot_w64(d2 <= thr);
+            const T q = pos_part<UNIT>(h2 - d2);
+            T w = (q * q) * q;
+            if constexpr (TAIL) {
+                in[u] &= ok[u];
+                w = __builtin_amdgcn_inverse_ballot_w64(ok[u]) ? w : T(0);
+            }
+            part = u ? part + w : w;
+        }
+        sum.add(part);
+        // the particle itself is not listed
+        const uint32_t ds = selfpos - t;  // 4 u + l where it is this lane's
+        if (__builtin_amdgcn_ballot_w64(ds < 16u)) {
+#pragma unroll
+            for (int u = 0; u < 4; ++u) in[u] &= __builtin_amdgcn_ballot_w64(ds != (uint32_t)(4 * u + l));
+        }
+        uint32_t acc = 0;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) acc |= __builtin_amdgcn_inverse_ballot_w64(in[u]) ? 1u << (4 * u) : 0u;
+        acc <<= l;
+        acc |= quad_dpp<0xB1>(acc);  // quad_perm [1,0,3,2]
+        acc |= quad_dpp<0x4E>(acc);  // quad_perm [2,3,0,1]
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const uint32_t at = (uint32_t)__popc(acc & upto[u]) + placed;
+            if (__builtin_amdgcn_inverse_ballot_w64(in[u])) *lds_at<lds_u32>(stage + (at << 2)) = jj[u];
+        }
+        placed += (uint32_t)__popc(acc);
+        if ((int32_t)placed >= 15) flush();
+    };
+    if (total != 0u) lookup(0u);
+    for (; t + 16u <= total; t += 16u) block(std::false_type());
+    if (t < total) block(std::true_type());
+    if ((int32_t)placed >= 0) {
+        const uint32_t left = placed + 1u;
+        flush();
+        done = done - 16u + left;
+    }
+    group_merge<4>(sum);
+    density_out<T>(D, K, slot, l, pi, sum.value(), done, cap, out.pb);
+}
+
+template <typename T, int SM, int YZ, bool UNIT>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? 6 : 4, 8))) void k_density_quad(
+    DevState D, int nblk, int remap)
+{
+    density_quad<T, SM, YZ, UNIT>(D, xcd_block(blockIdx.x, nblk, remap));
 }
 
 // ----------------------------------------------------------------- force
@@ -1459,28 +1914,44 @@ __device__ __forceinline__ int64_t erode_exchange(const SceneDev& S, const Scene
 }
 
 // Lane l's share of the force sums from list entries l, l+G, l+2G, ... of
-// a particle's neighbour sequence (fetch(k) = the byte offset of its k-th
-// neighbour's slot in the V4<T> vectors): the lanes
-// of a particle differ by one neighbour at most.  Four neighbours per
-// iteration (eight gathers in flight), summed (a + b) + (c + d) before they
-// enter the lane's sums; then one pair, then a single.
+// a particle's neighbour sequence: the lanes of a particle differ by one
+// neighbour at most.  An entry is the byte offset of the neighbour's slot in
+// the V4<T> vectors; chunk(c) gives the 16 entries c .. c+15 (c a multiple of
+// 16), laid out for the lanes (density_body).  Four neighbours per iteration
+// (eight gathers in flight), summed (a + b) + (c + d) before they enter the
+// lane's sums; then one pair, then a single.
+//
+// The pass is bound by VALU issue (92% on a 4.2M-particle layer) and close
+// behind by the L1's line accesses (2,170 per wave of 16 particles): a
+// wave's list read touches 16 lines, one per group, however few bytes each
+// lane takes, so the four entries of an iteration come with one 16-byte load
+// instead of four 4-byte ones.
 template <typename T, int SM, int G, typename F>
 __device__ __forceinline__ void force_list(const DevState& D, const SceneConsts<T>& K, int l, uint32_t cnt,
                                           const V4<T>& pi, const V4<T>& vi, T a_i, ForceAcc<T, SM>& acc,
-                                          F&& fetch)
+                                          F&& chunk)
 {
     const V4<T>* __restrict__ posa = (const V4<T>*)D.posa;
     const V4<T>* __restrict__ vel = (const V4<T>*)D.s_vel;
-    uint32_t k = (uint32_t)l;
-    // the list entries of the next four-neighbour iteration load while the
-    // current one computes
-    uint32_t na = 0, nb = 0, nc = 0, nd = 0;
-    if (k + 3 * G < cnt) { na = fetch(k); nb = fetch(k + G); nc = fetch(k + 2 * G); nd = fetch(k + 3 * G); }
-    for (; k + 3 * G < cnt; k += 4 * G) {
-        const uint32_t ja = na, jb = nb, jc = nc, jd = nd;
-        if (k + 7 * G < cnt) {
-            na = fetch(k + 4 * G); nb = fetch(k + 5 * G); nc = fetch(k + 6 * G); nd = fetch(k + 7 * G);
+    // the lane's four entries of the iteration of entries base .. base+4G-1
+    auto fetch = [&](uint32_t base) {
+        constexpr uint32_t PER = 16 / G;
+        if constexpr (G <= 4) {
+            return *(const uint4*)(chunk(base & ~15u) + (uint32_t)l * PER + (base & 15u) / G);
+        } else {
+            const uint2 a = *(const uint2*)(chunk(base) + (uint32_t)l * PER);
+            uint2 b = make_uint2(0u, 0u);
+            if (base + 16u < cnt) b = *(const uint2*)(chunk(base + 16u) + (uint32_t)l * PER);
+            return make_uint4(a.x, a.y, b.x, b.y);
         }
+    };
+    uint32_t k = (uint32_t)l;
+    // the list entries of the next iteration load while the current one computes
+    uint4 n = make_uint4(0u, 0u, 0u, 0u);
+    if (k < cnt) n = fetch(0u);
+    for (; k + 3 * G < cnt; k += 4 * G) {
+        const uint32_t ja = n.x, jb = n.y, jc = n.z, jd = n.w;
+        if (k + 4 * G < cnt) n = fetch(k - (uint32_t)l + 4 * G);
         const V4<T> pa = at_byte(posa, ja), va = at_byte(vel, ja), pb = at_byte(posa, jb), vb = at_byte(vel, jb);
         const V4<T> pc = at_byte(posa, jc), vc = at_byte(vel, jc), pd = at_byte(posa, jd), vd = at_byte(vel, jd);
         Terms<T> ab, cd;
@@ -1502,24 +1973,23 @@ __device__ __forceinline__ void force_list(const DevState& D, const SceneConsts<
         }
         acc.add4(ab, cd);
     }
-    for (; k + G < cnt; k += 2 * G) {
-        const uint32_t ja = fetch(k);
-        const uint32_t jb = fetch(k + G);
-        const V4<T> pa = at_byte(posa, ja);
-        const V4<T> va = at_byte(vel, ja);
-        const V4<T> pb = at_byte(posa, jb);
-        const V4<T> vb = at_byte(vel, jb);
+    // the lane's last one to three neighbours
+    uint32_t last = n.x;
+    if (k + G < cnt) {
+        const uint32_t ja = n.x, jb = n.y;
+        const V4<T> pa = at_byte(posa, ja), va = at_byte(vel, ja), pb = at_byte(posa, jb), vb = at_byte(vel, jb);
         const T ax = pi.x - pa.x, ay = pi.y - pa.y, az = pi.z - pa.z;
         const T a2 = (ax * ax + ay * ay) + az * az;
         const T bx = pi.x - pb.x, by = pi.y - pb.y, bz = pi.z - pb.z;
         const T b2 = (bx * bx + by * by) + bz * bz;
         acc.add2(pair_terms<T>(K, ax, ay, az, a2, a_i, pa.w, va.w, vi, va),
                  pair_terms<T>(K, bx, by, bz, b2, a_i, pb.w, vb.w, vi, vb));
+        k += 2 * G;
+        last = n.z;
     }
     if (k < cnt) {
-        const uint32_t j = fetch(k);
-        const V4<T> pj = at_byte(posa, j);
-        const V4<T> vj = at_byte(vel, j);
+        const V4<T> pj = at_byte(posa, last);
+        const V4<T> vj = at_byte(vel, last);
         const T dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
         const T d2 = (dx * dx + dy * dy) + dz * dz;
         acc.add(pair_terms<T>(K, dx, dy, dz, d2, a_i, pj.w, vj.w, vi, vj));
@@ -1538,14 +2008,14 @@ __device__ __forceinline__ void force_share(const DevState& D, const SceneDev& S
     const uint32_t cap = (uint32_t)D.maxn;
     const uint32_t* __restrict__ nbl = D.nbl + slot * (int64_t)D.maxn;
     if (cnt <= cap) {
-        force_list<T, SM, G>(D, K, l, cnt, pi, vi, a_i, acc, [&](uint32_t k) { return nbl[k]; });
+        force_list<T, SM, G>(D, K, l, cnt, pi, vi, a_i, acc, [&](uint32_t c) { return nbl + c; });
         return;
     }
     const uint32_t pb = D.pbase[slot];
     if (pb != ~0u && cnt - cap <= (uint32_t)D.ocap) {
-        const uint32_t* __restrict__ chunk = D.pool + (size_t)pb * SPHE_POOL_UNIT;
+        const uint32_t* __restrict__ more = D.pool + (size_t)pb * SPHE_POOL_UNIT;
         force_list<T, SM, G>(D, K, l, cnt, pi, vi, a_i, acc,
-                               [&](uint32_t k) { return k < cap ? nbl[k] : chunk[k - cap]; });
+                               [&](uint32_t c) { return c < cap ? nbl + c : more + (c - cap); });
         return;
     }
     // no room in list and pool: the stencil again (same order, same result)
@@ -2255,8 +2725,8 @@ void sphe_launch_hash(const DevState& D, hipStream_t st, hipEvent_t e0, hipEvent
     else klaunch(k_hash_count<float>, grid_of(D.P, 256), 256, st, e0, e1, D);
 }
 
-template <int ITEMS>
-static void launch_scan_t(uint32_t* cnt, uint32_t* start, int64_t n, uint32_t* partial, bool zero_counts,
+template <int ITEMS, typename S>
+static void launch_scan_t(uint32_t* cnt, S* start, int64_t n, uint32_t* partial, bool zero_counts,
                           unsigned long long* zero, unsigned long long zero_to, uint32_t* occ, uint32_t* fill,
                           hipStream_t st, hipEvent_t e0, hipEvent_t e1)
 {
@@ -2264,18 +2734,26 @@ static void launch_scan_t(uint32_t* cnt, uint32_t* start, int64_t n, uint32_t* p
     klaunch(k_scan_reduce<ITEMS>, (unsigned)nb, 256, st, e0, nullptr, (const uint32_t*)cnt, n, partial,
             (const uint32_t*)occ);
     klaunch(k_scan_tiles, 1, 1024, st, nullptr, nullptr, partial, nb);
-    klaunch(k_scan_down<ITEMS>, (unsigned)nb, 256, st, nullptr, e1, cnt, start, n, (const uint32_t*)partial,
+    klaunch(k_scan_down<ITEMS, S>, (unsigned)nb, 256, st, nullptr, e1, cnt, start, n, (const uint32_t*)partial,
             zero_counts ? 1 : 0, zero, zero_to, occ, occ ? fill : nullptr);
 }
 
 void sphe_launch_scan(uint32_t* cnt, uint32_t* start, int64_t n, uint32_t* partial, bool zero_counts,
-                      unsigned long long* zero, unsigned long long zero_to, uint32_t* occ, uint32_t* fill,
-                      int scan_log2, hipStream_t st, hipEvent_t e0, hipEvent_t e1)
+                      hipStream_t st, hipEvent_t e0, hipEvent_t e1)
 {
-    if (scan_log2 == 11) launch_scan_t<8>(cnt, start, n, partial, zero_counts, zero, zero_to, occ, fill, st, e0, e1);
-    else if (scan_log2 == 13)
-        launch_scan_t<32>(cnt, start, n, partial, zero_counts, zero, zero_to, occ, fill, st, e0, e1);
-    else launch_scan_t<16>(cnt, start, n, partial, zero_counts, zero, zero_to, occ, fill, st, e0, e1);
+    launch_scan_t<(1 << SPHE_SCAN_LOG2_DEFAULT) / 256>(cnt, start, n, partial, zero_counts, nullptr, 0ull, nullptr,
+                                                       nullptr, st, e0, e1);
+}
+
+void sphe_launch_scan_cells(const DevState& D, hipStream_t st, hipEvent_t e0, hipEvent_t e1)
+{
+    const unsigned long long to = (unsigned long long)D.pool_origin;
+    const int64_t n = D.C + 1;
+    if (D.scan_log2 == 11)
+        launch_scan_t<8>(D.cnt, D.cells, n, D.partial, false, D.ptop, to, D.tocc, D.tfill, st, e0, e1);
+    else if (D.scan_log2 == 13)
+        launch_scan_t<32>(D.cnt, D.cells, n, D.partial, false, D.ptop, to, D.tocc, D.tfill, st, e0, e1);
+    else launch_scan_t<16>(D.cnt, D.cells, n, D.partial, false, D.ptop, to, D.tocc, D.tfill, st, e0, e1);
 }
 
 int64_t sphe_scan_partials(int64_t n) { return (n + (1 << SPHE_SCAN_LOG2_MIN) - 1) >> SPHE_SCAN_LOG2_MIN; }
@@ -2296,6 +2774,22 @@ void sphe_launch_reorder(const DevState& D, hipStream_t st, hipEvent_t e0, hipEv
 template <int G>
 static void launch_density_g(const DevState& D, int block, int remap, hipStream_t st, hipEvent_t e0, hipEvent_t e1)
 {
+    if constexpr (G == 4) {
+        if (!D.persistent && D.yz <= 2) {
+            const size_t lds = (size_t)quad_group_bytes(D.yz) * (size_t)(block / 4);
+            const int nblk = (int)grid_of(D.P * G, block);
+#define CALL(T, SM)                                                                                       \
+    do {                                                                                                  \
+        void (*k)(DevState, int, int) =                                                                   \
+            D.yz == 1 ? (D.h_unit ? k_density_quad<T, SM, 1, true> : k_density_quad<T, SM, 1, false>)     \
+                      : (D.h_unit ? k_density_quad<T, SM, 2, true> : k_density_quad<T, SM, 2, false>);    \
+        klaunch_lds(k, nblk, block, lds, st, e0, e1, D, nblk, remap);                                     \
+    } while (0)
+            SPHE_PREC_SWITCH(D.precision, CALL);
+#undef CALL
+            return;
+        }
+    }
     // one row table and one list staging ring per group, at most 64 KiB per
     // block with the persistent form's static word (halve the block until
     // it fits)
@@ -2370,7 +2864,7 @@ static void launch_scan_heights_t(const DevState& D, hipStream_t st, hipEvent_t 
     const int64_t nh = (int64_t)grid_of(D.TC / 4, 256);  // TC: a multiple of 64
     klaunch(k_scan_reduce_heights<ITEMS>, (unsigned)(nb + nh), 256, st, e0, nullptr, D, (int)nb);
     klaunch(k_scan_tiles, 1, 1024, st, nullptr, nullptr, D.partial, nb);
-    klaunch(k_scan_down<ITEMS>, (unsigned)nb, 256, st, nullptr, e1, D.cnt, D.start, n, (const uint32_t*)D.partial,
+    klaunch(k_scan_down<ITEMS, uint2>, (unsigned)nb, 256, st, nullptr, e1, D.cnt, D.cells, n, (const uint32_t*)D.partial,
             0, D.ptop, (unsigned long long)D.pool_origin, D.tocc, D.tfill);
 }
 
@@ -2391,8 +2885,7 @@ void sphe_launch_two_phase(const DevState& D, hipStream_t st, hipEvent_t e0, hip
 {
     if (D.TC == 0 || D.P == 0) return;
     klaunch(k_tcount, grid_of(D.P, 256), 256, st, e0, nullptr, D);
-    sphe_launch_scan(D.tcnt, D.tstart, D.TC + 1, D.tpartial, true, nullptr, 0ull, nullptr, nullptr,
-                     SPHE_SCAN_LOG2_DEFAULT, st);
+    sphe_launch_scan(D.tcnt, D.tstart, D.TC + 1, D.tpartial, true, st);
     k_tscatter<<<grid_of(D.P, 256), 256, 0, st>>>(D);
     klaunch(k_tapply, grid_of(D.TC, 256), 256, st, nullptr, e1, D);
 }

@@ -528,8 +528,7 @@ int build_layout(sphe_ctx* c)
     DALLOC(D.tmp_kid, Pn * 8);
     DALLOC(D.tmp_src, Pn * 4);
     DALLOC(D.cnt, (size_t)(C + 1) * 4);
-    DALLOC(D.start, (size_t)(C + 1) * 4);
-    DALLOC(D.subw, (size_t)(C + 1) * 4);
+    DALLOC(D.cells, (size_t)(C + 2) * 8);  // two records are loaded at once
     D.yz = c->yz;
     D.sub_log2 = c->sub_log2;
     D.scan_log2 = c->scan_log2;
@@ -590,7 +589,7 @@ int build_layout(sphe_ctx* c)
     HIPCHK(c, hipMemsetAsync(D.cnt, 0, (size_t)(C + 1) * 4, c->stream));
     HIPCHK(c, hipMemsetAsync(D.tocc, 0, (size_t)D.npartial * 4, c->stream));
     HIPCHK(c, hipMemsetAsync(D.tfill, 0xFF, (size_t)D.npartial * 4, c->stream));  // no tile known filled
-    HIPCHK(c, hipMemsetAsync(D.subw, 0, (size_t)(C + 1) * 4, c->stream));
+    HIPCHK(c, hipMemsetAsync(D.cells, 0, (size_t)(C + 2) * 8, c->stream));
     HIPCHK(c, hipMemsetAsync(D.tcnt, 0, (size_t)(TC + 1) * 4, c->stream));
     HIPCHK(c, hipMemsetAsync(D.status, 0, 64, c->stream));
     HIPCHK(c, hipMemsetAsync(D.ovf, 0, 64, c->stream));
@@ -760,6 +759,9 @@ int upload_table(sphe_ctx* c, bool force)
         std::memset(&t[i], 0, sizeof(SceneDev));
         derive(c->scenes[i], t[i], c->yz);
     }
+    c->D.h_unit = 1;
+    for (const SceneDev& d : t)
+        if (!(d.f.h2 <= 1.0f)) c->D.h_unit = 0;
     if (!force && c->table_uploaded && t.size() == c->table.size() &&
         std::memcmp(t.data(), c->table.data(), t.size() * sizeof(SceneDev)) == 0)
         return SPHE_OK;
@@ -849,8 +851,7 @@ void launch_sort(sphe_ctx* c)
         // with erosion the terrain heights of the last force pass are computed
         // in the scan's first launch (this step's force pass samples them)
         if (any_erosion(c, -1) && D.TC > 0) sphe_launch_scan_heights(D, c->stream, t.a, t.b);
-        else sphe_launch_scan(D.cnt, D.start, D.C + 1, D.partial, false, D.ptop,
-                              (unsigned long long)D.pool_origin, D.tocc, D.tfill, D.scan_log2, c->stream, t.a, t.b);
+        else sphe_launch_scan_cells(D, c->stream, t.a, t.b);
     }
     {
         Timed t(c, "scatter");
@@ -884,12 +885,13 @@ std::string plan_signature(const sphe_ctx* c)
 {
     // everything the captured kernels take by value (DevState) or as launch shape
     char b[384];
-    snprintf(b, sizeof(b), "%d/%d/%d/%d/%d/%lld/%lld/%lld/%d/%d/%p/%p/%p/%d/%d/%d/%d/%lld/%d/%d", c->precision, c->block,
+    snprintf(b, sizeof(b), "%d/%d/%d/%d/%d/%lld/%lld/%lld/%d/%d/%p/%p/%p/%d/%d/%d/%d/%lld/%d/%d/%d",
+             c->precision, c->block,
              force_block(c), c->remap,
              c->lanes, (long long)c->D.P, (long long)c->D.C, (long long)c->D.TC, (int)any_erosion(c, -1),
              (int)any_erosion(c, SPHE_EROSION_TWO_PHASE), (const void*)c->D.u_pos, (const void*)c->D.nbl,
              (const void*)c->D.pool, c->D.maxn, c->D.sub_log2, c->D.yz, c->D.ocap, (long long)c->D.pool_cap,
-             c->D.scan_log2, c->D.persistent);
+             c->D.scan_log2, c->D.persistent, c->D.h_unit);
     return b;
 }
 

@@ -1,0 +1,74 @@
+"""GPU tests of the neighbour passes' branches against the FP32 twin (bit for
+bit): streams of candidates shorter and longer than one segment of row marks
+(256 positions) and ones ending on its edges, cells of more than 1,023
+particles, smoothing lengths above and at 1 (the clamped kernel serves lengths
+up to 1), coincident and almost coincident neighbours, scenes that leave part
+of a wave empty."""
+import numpy as np
+import pytest
+
+import oracle as O
+import sphe
+from gpu_common import orc_scene_from
+
+pytestmark = pytest.mark.gpu
+
+
+def _params(h, half, dt=1e-5, centre=0.0):
+    return sphe.default_params(h=h, mass=0.02 * (h / 0.0457) ** 3, dt=dt, box_half=half, box_center=(centre,) * 3)
+
+
+def _compare(p, pos, yz, precision=sphe.FP32, comp=1, steps=2):
+    n = len(pos)
+    pos = np.ascontiguousarray(pos, dtype=np.float32)
+    ctx = sphe.Context(precision)
+    ctx.set_yz_split(yz)
+    sid = ctx.add_scene(p)
+    ctx.set_particles(sid, pos)
+    ctx.step(steps)
+    gp, gv = ctx.state_f64(sid)
+    rho = ctx.density(sid)
+    osc = orc_scene_from(p)
+    osc.yz = yz
+    st = dict(pos=pos.astype(np.float64), vel=np.zeros((n, 3)), sed=np.zeros(n, np.int64))
+    for _ in range(steps):
+        st = O.orc_step(osc, st["pos"], st["vel"], st["sed"], np.arange(n, dtype=np.int32), real=4, comp=comp)
+    assert np.array_equal(gp, st["pos"]) and np.array_equal(gv, st["vel"])
+    assert np.array_equal(rho.astype(np.float64), st["rho"])
+
+
+@pytest.mark.parametrize("yz", [1, 2])
+@pytest.mark.parametrize("n,edge", [(1, 0.5), (15, 0.3), (66, 0.5), (255, 0.4), (256, 0.4), (257, 0.4), (273, 0.4),
+                                    (512, 0.45), (700, 1.5), (2500, 1.2)])
+def test_stream_lengths_bit_exact_twin(n, edge, yz):
+    """n particles in a cube of `edge` smoothing lengths: in the small cubes
+    every particle is a candidate of every other, so streams have n positions
+    (256 and 512 end on a segment's edge); 2,500 fill cells past 1,023."""
+    h = 0.0457
+    rng = np.random.default_rng(n)
+    pos = rng.uniform(0.0, edge * h, (n, 3)) + 0.013
+    _compare(_params(h, 0.2), pos, yz)
+
+
+@pytest.mark.parametrize("h", [1.0, 1.7, 0.02])
+@pytest.mark.parametrize("precision,comp", [(sphe.FP32, 1), (sphe.FP32_NAIVE, 0)])
+def test_smoothing_lengths_bit_exact_twin(h, precision, comp):
+    """Lengths above 1 take the kernels without the clamp; 1 is its limit."""
+    rng = np.random.default_rng(7)
+    pos = rng.uniform(-1.6 * h, 1.6 * h, (900, 3))
+    _compare(_params(h, 4.0 * h), pos, 2, precision, comp)
+
+
+@pytest.mark.parametrize("yz", [1, 2])
+def test_coincident_neighbours_bit_exact_twin(yz):
+    """Neighbours at distance 0, just inside and just outside 1e-4 among
+    ordinary ones, at every place of the list's groups of four."""
+    h = 0.0457
+    rng = np.random.default_rng(3)
+    base = rng.uniform(-0.06, 0.06, (300, 3))
+    near = np.repeat(base[:40], 3, axis=0)
+    near[0::3] += 0.0
+    near[1::3, 0] += 9.9e-5
+    near[2::3, 1] += 1.02e-4
+    pos = np.concatenate([base, near])[rng.permutation(420)]
+    _compare(_params(h, 0.2, dt=1e-6), pos, yz)
