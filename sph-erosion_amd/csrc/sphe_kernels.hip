@@ -72,6 +72,12 @@ __device__ __forceinline__ int xcd_block(int bid, int nblk, int chunk)
     return ((i / chunk) * 8 + x) * chunk + i % chunk;
 }
 
+// Index of this wave in block b of a one-dimensional grid of whole waves.
+__device__ __forceinline__ uint32_t wave_index(int b)
+{
+    return (uint32_t)b * (blockDim.x / SPHE_WAVE) + __builtin_amdgcn_readfirstlane(threadIdx.x / SPHE_WAVE);
+}
+
 __device__ __forceinline__ int wave_scene(const int32_t* chunk_scene, int64_t slot)
 {
     return __builtin_amdgcn_readfirstlane(chunk_scene[slot >> 6]);
@@ -1173,7 +1179,7 @@ __global__ __launch_bounds__(512) void k_density(DevState D, int nblk, int remap
 // 1 or 2): the same streams, sums and lists as density_body, bit for bit, in
 // two thirds to nine tenths of its time: 18.0 -> 10.5 us on a dam break of
 // 4,096 particles, 88.5 -> 66 us on a settled column of 262,144, 162 -> 143 us
-// on 48 settled scenes of 877,000 in all (cubic cells), 1,443 -> 1,273 us on a
+// on 48 settled scenes of 879,000 in all (cubic cells), 1,443 -> 1,273 us on a
 // settled layer of 4,194,304.  density_body serves the other lane counts,
 // thirds of cells and the persistent launch.
 //
@@ -1286,12 +1292,11 @@ __device__ __forceinline__ void density_quad(const DevState& D, int b)
 {
     constexpr int W = 2 * YZ + 1;
     constexpr uint32_t VB = (uint32_t)sizeof(V4<T>);
-    const int64_t gt = (int64_t)b * blockDim.x + threadIdx.x;
     const int l = (int)(threadIdx.x & 3);
     const int lane = (int)(threadIdx.x & (SPHE_WAVE - 1));
     // the wave's first slot (slots are below 2^30; P is a multiple of 64, so
     // waves are whole)
-    const uint32_t wslot = __builtin_amdgcn_readfirstlane((uint32_t)(gt >> 6)) * 16u;
+    const uint32_t wslot = wave_index(b) * 16u;
     if (wslot >= (uint64_t)D.P) return;
     const uint32_t slot = wslot + (uint32_t)(lane >> 2);
     const SceneDev& S = D.scenes[wave_scene(D.chunk_scene, wslot)];
@@ -1658,23 +1663,34 @@ __device__ __forceinline__ Terms<T> terms_sum(const Terms<T>& a, const Terms<T>&
     return t;
 }
 
+// The constants of the pair terms.
 template <typename T>
-__device__ __forceinline__ Terms<T> pair_terms(const SceneConsts<T>& K, T dx, T dy, T dz, T d2, T a_i, T a_j,
+struct PairConsts {
+    T h, h2, t3h2, eps_r, inv_sqrt3;
+};
+
+template <bool UNIT, typename T>
+__device__ __forceinline__ Terms<T> pair_terms(const PairConsts<T>& K, T dx, T dy, T dz, T d2, T a_i, T a_j,
                                                T b_j, const V4<T>& vi, const V4<T>& vj)
 {
     Terms<T> t;
-    T q = K.h2 - d2;
-    q = q > T(0) ? q : T(0);
+    const T q = pos_part<UNIT>(K.h2 - d2);
     t.lap = b_j * (q * (K.t3h2 - T(7) * d2));
     T r, inv;
     Root<T>::of(d2, r, inv);
     const T hr = K.h - r;
+    T ux = dx * inv, uy = dy * inv, uz = dz * inv;
     // coincident pair: the reference points along normalize(1,1,1)
-    // (fluid_system.h:438-440); the reciprocal is discarded then
+    // (fluid_system.h:438-440); the reciprocal is discarded then.  Rare: the
+    // selects run only where a lane of the wave has one (the empty asm keeps
+    // the compiler from making them unconditional).
     const bool near = r < K.eps_r;
-    const T ux = near ? K.inv_sqrt3 : dx * inv;
-    const T uy = near ? K.inv_sqrt3 : dy * inv;
-    const T uz = near ? K.inv_sqrt3 : dz * inv;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(near) != 0ull, 0)) {
+        asm volatile("");
+        ux = near ? K.inv_sqrt3 : ux;
+        uy = near ? K.inv_sqrt3 : uy;
+        uz = near ? K.inv_sqrt3 : uz;
+    }
     const T sp = (a_i + a_j) * (hr * hr);
     t.fp0 = sp * ux;
     t.fp1 = sp * uy;
@@ -1718,14 +1734,6 @@ struct ForceAcc {
         fp0.add(t.fp0); fp1.add(t.fp1); fp2.add(t.fp2);
         fv0.add(t.fv0); fv1.add(t.fv1); fv2.add(t.fv2);
         nn0.add(t.nn0); nn1.add(t.nn1); nn2.add(t.nn2);
-    }
-
-    __device__ __forceinline__ void add2(const Terms<T>& a, const Terms<T>& b)
-    {
-        lap.add(a.lap + b.lap);
-        fp0.add(a.fp0 + b.fp0); fp1.add(a.fp1 + b.fp1); fp2.add(a.fp2 + b.fp2);
-        fv0.add(a.fv0 + b.fv0); fv1.add(a.fv1 + b.fv1); fv2.add(a.fv2 + b.fv2);
-        nn0.add(a.nn0 + b.nn0); nn1.add(a.nn1 + b.nn1); nn2.add(a.nn2 + b.nn2);
     }
 
     // four consecutive terms as two plain pair sums ab = a + b, cd = c + d:
@@ -1782,6 +1790,7 @@ __device__ __forceinline__ void force_share_walk(const DevState& D, const SceneD
     Terms<T> ab, c;
     int np = 0;  // terms of the group so far
     uint32_t m = 0;    // canonical index of the next accepted neighbour
+    const PairConsts<T> C{K.h, K.h2, K.t3h2, K.eps_r, K.inv_sqrt3};
     if (l == 0) ++count;  // the particle itself
     visit_neighbours<T>(D, S, K, pos, pi.x, pi.y, pi.z, [&](uint32_t j, T dx, T dy, T dz, T d2) {
         if ((int64_t)j == slot) return;  // own term: ForceAcc::self_term
@@ -1792,7 +1801,7 @@ __device__ __forceinline__ void force_share_walk(const DevState& D, const SceneD
         const int32_t idj = D.s_id[j];
         nbmax = idj > nbmax ? idj : nbmax;
         const V4<T> vj = at(vel, j);
-        const Terms<T> t = pair_terms<T>(K, dx, dy, dz, d2, a_i, at(posa, j).w, vj.w, vi, vj);
+        const Terms<T> t = pair_terms<false, T>(C, dx, dy, dz, d2, a_i, at(posa, j).w, vj.w, vi, vj);
         if (np == 0) ab = t;
         else if (np == 1) ab = terms_sum(ab, t);
         else if (np == 2) c = t;
@@ -1916,150 +1925,174 @@ __device__ __forceinline__ int64_t erode_exchange(const SceneDev& S, const Scene
 // Lane l's share of the force sums from list entries l, l+G, l+2G, ... of
 // a particle's neighbour sequence: the lanes of a particle differ by one
 // neighbour at most.  An entry is the byte offset of the neighbour's slot in
-// the V4<T> vectors; chunk(c) gives the 16 entries c .. c+15 (c a multiple of
-// 16), laid out for the lanes (density_body).  Four neighbours per iteration
-// (eight gathers in flight), summed (a + b) + (c + d) before they enter the
-// lane's sums; then one pair, then a single.
+// the V4<T> vectors; fetch(more) gives the lane's next four (mine in all).
+// Four neighbours per iteration (eight gathers in flight), summed
+// (a + b) + (c + d) before they enter the lane's sums; then one pair, then a
+// single.
 //
-// The pass is bound by VALU issue (92% on a 4.2M-particle layer) and close
-// behind by the L1's line accesses (2,170 per wave of 16 particles): a
-// wave's list read touches 16 lines, one per group, however few bytes each
-// lane takes, so the four entries of an iteration come with one 16-byte load
-// instead of four 4-byte ones.
-template <typename T, int SM, int G, typename F>
-__device__ __forceinline__ void force_list(const DevState& D, const SceneConsts<T>& K, int l, uint32_t cnt,
-                                          const V4<T>& pi, const V4<T>& vi, T a_i, ForceAcc<T, SM>& acc,
-                                          F&& chunk)
+// No unit is saturated: on a settled 4.2M-particle layer (1,437 us before, 1,320
+// now) the gathers' line accesses take 55% of the L1's cycles, the VALU is
+// busy for half the time, the lists come from HBM, and 20 waves a CU wait for
+// each other.  So waves in flight count most: five a SIMD, 96 registers, with
+// nothing spilled on the way through the loop.  What lies behind that:
+// * a wave's list read touches 16 lines, one per group, however few bytes a lane
+//   takes: the four entries of an iteration come with one 16-byte load;
+// * one loop for lists with and without an overflow chunk (a wave with one
+//   overflowing particle ran both loops: 90 -> 70 us on a column of 262,144
+//   with lists of 256 entries);
+// * values that the epilogue or the rare paths make from the thread index are
+//   made again there (opaque_tid): kept over the loop they were spilled by
+//   every wave, 0.6 GB a launch;
+// * coincident pairs' selects behind a branch that is hardly ever taken.
+// Eight gathers in flight with five waves beat four gathers with six or
+// seven, a pair ahead with four waves, and lists two iterations ahead.
+template <bool UNIT, typename T, int SM, int G, typename F>
+__device__ __forceinline__ void force_list(const DevState& D, const SceneConsts<T>& K, uint32_t mine, const V4<T>& pi,
+                                           const V4<T>& vi, T a_i, ForceAcc<T, SM>& acc, F&& fetch)
 {
+    if (mine == 0u) return;
     const V4<T>* __restrict__ posa = (const V4<T>*)D.posa;
     const V4<T>* __restrict__ vel = (const V4<T>*)D.s_vel;
-    // the lane's four entries of the iteration of entries base .. base+4G-1
-    auto fetch = [&](uint32_t base) {
-        constexpr uint32_t PER = 16 / G;
-        if constexpr (G <= 4) {
-            return *(const uint4*)(chunk(base & ~15u) + (uint32_t)l * PER + (base & 15u) / G);
-        } else {
-            const uint2 a = *(const uint2*)(chunk(base) + (uint32_t)l * PER);
-            uint2 b = make_uint2(0u, 0u);
-            if (base + 16u < cnt) b = *(const uint2*)(chunk(base + 16u) + (uint32_t)l * PER);
-            return make_uint4(a.x, a.y, b.x, b.y);
-        }
-    };
-    uint32_t k = (uint32_t)l;
-    // the list entries of the next iteration load while the current one computes
-    uint4 n = make_uint4(0u, 0u, 0u, 0u);
-    if (k < cnt) n = fetch(0u);
-    for (; k + 3 * G < cnt; k += 4 * G) {
-        const uint32_t ja = n.x, jb = n.y, jc = n.z, jd = n.w;
-        if (k + 4 * G < cnt) n = fetch(k - (uint32_t)l + 4 * G);
-        const V4<T> pa = at_byte(posa, ja), va = at_byte(vel, ja), pb = at_byte(posa, jb), vb = at_byte(vel, jb);
-        const V4<T> pc = at_byte(posa, jc), vc = at_byte(vel, jc), pd = at_byte(posa, jd), vd = at_byte(vel, jd);
-        Terms<T> ab, cd;
-        {
-            const T ax = pi.x - pa.x, ay = pi.y - pa.y, az = pi.z - pa.z;
-            const T a2 = (ax * ax + ay * ay) + az * az;
-            const T bx = pi.x - pb.x, by = pi.y - pb.y, bz = pi.z - pb.z;
-            const T b2 = (bx * bx + by * by) + bz * bz;
-            ab = terms_sum(pair_terms<T>(K, ax, ay, az, a2, a_i, pa.w, va.w, vi, va),
-                           pair_terms<T>(K, bx, by, bz, b2, a_i, pb.w, vb.w, vi, vb));
-        }
-        {
-            const T ax = pi.x - pc.x, ay = pi.y - pc.y, az = pi.z - pc.z;
-            const T a2 = (ax * ax + ay * ay) + az * az;
-            const T bx = pi.x - pd.x, by = pi.y - pd.y, bz = pi.z - pd.z;
-            const T b2 = (bx * bx + by * by) + bz * bz;
-            cd = terms_sum(pair_terms<T>(K, ax, ay, az, a2, a_i, pc.w, vc.w, vi, vc),
-                           pair_terms<T>(K, bx, by, bz, b2, a_i, pd.w, vd.w, vi, vd));
-        }
-        acc.add4(ab, cd);
-    }
-    // the lane's last one to three neighbours
-    uint32_t last = n.x;
-    if (k + G < cnt) {
-        const uint32_t ja = n.x, jb = n.y;
-        const V4<T> pa = at_byte(posa, ja), va = at_byte(vel, ja), pb = at_byte(posa, jb), vb = at_byte(vel, jb);
-        const T ax = pi.x - pa.x, ay = pi.y - pa.y, az = pi.z - pa.z;
-        const T a2 = (ax * ax + ay * ay) + az * az;
-        const T bx = pi.x - pb.x, by = pi.y - pb.y, bz = pi.z - pb.z;
-        const T b2 = (bx * bx + by * by) + bz * bz;
-        acc.add2(pair_terms<T>(K, ax, ay, az, a2, a_i, pa.w, va.w, vi, va),
-                 pair_terms<T>(K, bx, by, bz, b2, a_i, pb.w, vb.w, vi, vb));
-        k += 2 * G;
-        last = n.z;
-    }
-    if (k < cnt) {
-        const V4<T> pj = at_byte(posa, last);
-        const V4<T> vj = at_byte(vel, last);
-        const T dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
+    const PairConsts<T> C{K.h, K.h2, K.t3h2, K.eps_r, K.inv_sqrt3};
+    struct Nb { V4<T> p, v; };
+    auto load = [&](uint32_t j) { return Nb{at_byte(posa, j), at_byte(vel, j)}; };
+    auto terms = [&](const Nb& b) {
+        const T dx = pi.x - b.p.x, dy = pi.y - b.p.y, dz = pi.z - b.p.z;
         const T d2 = (dx * dx + dy * dy) + dz * dz;
-        acc.add(pair_terms<T>(K, dx, dy, dz, d2, a_i, pj.w, vj.w, vi, vj));
+        return pair_terms<UNIT, T>(C, dx, dy, dz, d2, a_i, b.p.w, b.v.w, vi, b.v);
+    };
+    // The list entries of the next iteration load while the current one
+    // computes: always, and after the gathers, whose waits then leave that load
+    // in flight (memory operations complete in order; a load that may or may
+    // not have been issued would have to be waited for).
+    uint4 n = fetch(mine > 4u);
+    for (; mine >= 4u; mine -= 4u) {
+        const Nb a = load(n.x), b = load(n.y), c = load(n.z), d = load(n.w);
+        __builtin_amdgcn_sched_barrier(0);
+        n = fetch(mine > 8u);
+        __builtin_amdgcn_sched_barrier(0);
+        const Terms<T> ab = terms_sum(terms(a), terms(b));
+        acc.add4(ab, terms_sum(terms(c), terms(d)));
     }
+    // the lane's last one to three neighbours: a pair, then a single
+    if (mine >= 2u) {
+        const Nb a = load(n.x), b = load(n.y);
+        acc.add(terms_sum(terms(a), terms(b)));
+        n.x = n.z;
+    }
+    if (mine & 1u) acc.add(terms(load(n.x)));
+}
+
+// The thread index as a value the compiler knows nothing of: what is made of
+// it is not kept in registers from an earlier use of the index (over the list
+// loop, a register more is a spill).
+__device__ __forceinline__ uint32_t opaque_tid()
+{
+    uint32_t t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t;
 }
 
 // Lane l's share of the force sums of one particle: from its list, the
 // list continued in its overflow chunk, or (no room for all neighbours)
-// by walking the stencil.
-template <typename T, int SM, int G>
+// by walking the stencil.  wslot: the wave's first slot.
+template <bool UNIT, typename T, int SM, int G>
 __device__ __forceinline__ void force_share(const DevState& D, const SceneDev& S, const SceneConsts<T>& K,
-                                           int64_t slot, int l, const V4<T>& pi, const V4<T>& vi, T a_i,
-                                           ForceAcc<T, SM>& acc, bool report_walk)
+                                           uint32_t slot, uint32_t wslot, int l, const V4<T>& pi, const V4<T>& vi,
+                                           T a_i, ForceAcc<T, SM>& acc, bool report_walk)
 {
+    constexpr uint32_t PER = 16 / G;
     const uint32_t cnt = D.nbc[slot];
     const uint32_t cap = (uint32_t)D.maxn;
-    const uint32_t* __restrict__ nbl = D.nbl + slot * (int64_t)D.maxn;
-    if (cnt <= cap) {
-        force_list<T, SM, G>(D, K, l, cnt, pi, vi, a_i, acc, [&](uint32_t c) { return nbl + c; });
-        return;
-    }
-    const uint32_t pb = D.pbase[slot];
-    if (pb != ~0u && cnt - cap <= (uint32_t)D.ocap) {
-        const uint32_t* __restrict__ more = D.pool + (size_t)pb * SPHE_POOL_UNIT;
-        force_list<T, SM, G>(D, K, l, cnt, pi, vi, a_i, acc,
-                               [&](uint32_t c) { return c < cap ? nbl + c : more + (c - cap); });
+    if (cnt <= cap || (cnt - cap <= (uint32_t)D.ocap && D.pbase[slot] != ~0u)) {
+        // the lane's entries l, l + G, ... are words l PER .. of each chunk of
+        // 16; e: the first entry of the next iteration's 4G (uniform, since the
+        // lanes go through their lists in step).  fetch(more) gives the entries
+        // of this iteration, again if it was told there are no more.
+        const uint32_t mine = (cnt + (uint32_t)(G - 1 - l)) / G;
+        const uint32_t* list = D.nbl + (size_t)slot * cap + (uint32_t)l * PER;
+        auto pool = [&]() {
+            const uint32_t t = opaque_tid();
+            return D.pool + (size_t)D.pbase[wslot + (t & (SPHE_WAVE - 1)) / G] * SPHE_POOL_UNIT + (t & (G - 1)) * PER;
+        };
+        uint32_t e = 0;
+        if constexpr (G == 4) {
+            force_list<UNIT, T, SM, G>(D, K, mine, pi, vi, a_i, acc, [&](bool more) {
+                const uint4 n = *(const uint4*)list;
+                e += 16u;
+                if (__builtin_expect(e == cap, 0)) {
+                    if (more) list = pool();
+                } else {
+                    list += more ? 16 : 0;
+                }
+                return n;
+            });
+        } else {
+            auto chunk = [&](uint32_t c) { return c < cap ? list + c : pool() + (c - cap); };
+            force_list<UNIT, T, SM, G>(D, K, mine, pi, vi, a_i, acc, [&](bool more) {
+                uint4 n;
+                if constexpr (G < 4) {
+                    n = *(const uint4*)(chunk(e & ~15u) + (e & 15u) / G);
+                } else {
+                    const uint2 a = *(const uint2*)chunk(e);
+                    uint2 b = a;
+                    if (e + 16u < cnt) b = *(const uint2*)chunk(e + 16u);
+                    n = make_uint4(a.x, a.y, b.x, b.y);
+                }
+                if (more) e += 4 * G;
+                return n;
+            });
+        }
         return;
     }
     // no room in list and pool: the stencil again (same order, same result)
+    const uint32_t t = opaque_tid();
+    l = (int)(t & (G - 1));
     if (report_walk && l == 0) atomicOr(D.status, 4u);
     int32_t nbmax = -1, count = 0;
-    force_share_walk<T, SM, G>(D, S, K, slot, l, pi, vi, a_i, acc, nbmax, count);
+    force_share_walk<T, SM, G>(D, S, K, wslot + (t & (SPHE_WAVE - 1)) / G, l, pi, vi, a_i, acc, nbmax, count);
 }
 
 // One G-lane group per particle: the lanes sum their shares, merge them
 // (xor shuffles), and lane 0 integrates, collides, erodes, stores the new
 // state and counts the particle's next cell.
-template <typename T, int SM, int G>
+template <bool UNIT, typename T, int SM, int G>
 __device__ __forceinline__ void force_body(const DevState& D, int b)
 {
-    const int64_t gt = (int64_t)b * blockDim.x + threadIdx.x;
-    const int64_t slot = gt / G;
-    const int l = (int)(gt & (G - 1));
-    if (slot >= D.P) return;
-    const SceneDev& S = D.scenes[wave_scene(D.chunk_scene, slot)];
+    const int l = (int)(threadIdx.x & (G - 1));
+    // the wave's first slot (slots are below 2^30; P is a multiple of 64, so
+    // waves are whole)
+    const uint32_t wslot = wave_index(b) * (uint32_t)(SPHE_WAVE / G);
+    if (wslot >= (uint64_t)D.P) return;
+    const uint32_t slot0 = wslot + (uint32_t)(threadIdx.x & (SPHE_WAVE - 1)) / G;
+    const SceneDev& S = D.scenes[wave_scene(D.chunk_scene, wslot)];
     V4<T>* __restrict__ upos = (V4<T>*)D.u_pos;
     V4<T>* __restrict__ uvel = (V4<T>*)D.u_vel;
     const V4<T>* __restrict__ spos = (const V4<T>*)D.s_pos;
     const V4<T>* __restrict__ svel = (const V4<T>*)D.s_vel;
-    if (slot >= S.p_begin + S.n) {
+    if (slot0 >= (uint32_t)(S.p_begin + S.n)) {
         if (l != 0) return;
         // padding: carried through, counted into the scene's pad cell
-        upos[slot] = spos[slot];
-        uvel[slot] = svel[slot];
-        D.u_sed[slot] = D.s_sed[slot];
-        D.u_id[slot] = D.s_id[slot];
-        count_pad(D, S, slot);
-        if (S.erosion == 2) D.tcell[slot] = -1;
+        upos[slot0] = spos[slot0];
+        uvel[slot0] = svel[slot0];
+        D.u_sed[slot0] = D.s_sed[slot0];
+        D.u_id[slot0] = D.s_id[slot0];
+        count_pad(D, S, slot0);
+        if (S.erosion == 2) D.tcell[slot0] = -1;
         return;
     }
     const SceneConsts<T>& K = SceneSel<T>::get(S);
-    const V4<T> pi = spos[slot];
-    const V4<T> vi = svel[slot];
-    const T rho_i = ((const T*)D.rho)[slot];
-    const T a_i = ((const V4<T>*)D.posa)[slot].w;
+    const V4<T> pi = spos[slot0];
+    const V4<T> vi = svel[slot0];
+    const T a_i = ((const V4<T>*)D.posa)[slot0].w;
     ForceAcc<T, SM> acc;
     if (l == 0) acc.self_term(K, vi.w);
-    force_share<T, SM, G>(D, S, K, slot, l, pi, vi, a_i, acc, true);
+    force_share<UNIT, T, SM, G>(D, S, K, slot0, wslot, l, pi, vi, a_i, acc, true);
     acc.template merge<G>();
-    if (l != 0) return;
+    const uint32_t tid = opaque_tid();
+    if ((tid & (G - 1)) != 0) return;
+    const uint32_t slot = wslot + (tid & (SPHE_WAVE - 1)) / G;
+    const T rho_i = ((const T*)D.rho)[slot];
     ForceOut<T> o;
     acc.finish(K, rho_i, o);
 
@@ -2110,11 +2143,11 @@ __device__ __forceinline__ void force_body(const DevState& D, int b)
 // only the rarely taken stencil walk of overflowing particles spills.
 // Unbounded, the walk raises the count and the occupancy of the whole
 // kernel drops to 4.
-template <int SM, int G>
+template <int SM, int G, bool UNIT>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_force_f32(DevState D, int nblk,
                                                                                               int remap)
 {
-    force_body<float, SM, G>(D, xcd_block(blockIdx.x, nblk, remap));
+    force_body<UNIT, float, SM, G>(D, xcd_block(blockIdx.x, nblk, remap));
 }
 
 // FP64: at most 168 registers (3 waves per SIMD instead of 2 unbounded).
@@ -2122,7 +2155,7 @@ template <int G>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_force_f64(DevState D, int nblk,
                                                                                               int remap)
 {
-    force_body<double, SUM_PLAIN, G>(D, xcd_block(blockIdx.x, nblk, remap));
+    force_body<false, double, SUM_PLAIN, G>(D, xcd_block(blockIdx.x, nblk, remap));
 }
 
 // ------------------------------------------------------ persistent passes
@@ -2188,13 +2221,13 @@ template <int SM, int G>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_force_f32_pers(
     DevState D, int nblk, int chunk, uint32_t* work)
 {
-    SPHE_PERSISTENT_LOOP((force_body<float, SM, G>(D, b)))
+    SPHE_PERSISTENT_LOOP((force_body<false, float, SM, G>(D, b)))
 }
 
 template <int G>
 __global__ __launch_bounds__(512) void k_force_f64_pers(DevState D, int nblk, int chunk, uint32_t* work)
 {
-    SPHE_PERSISTENT_LOOP((force_body<double, SUM_PLAIN, G>(D, b)))
+    SPHE_PERSISTENT_LOOP((force_body<false, double, SUM_PLAIN, G>(D, b)))
 }
 
 // --------------------------------------------------------------- terrain
@@ -2410,7 +2443,8 @@ __global__ __launch_bounds__(256) void k_accel(DevState D, int scene, double* __
     const T a_i = ((const V4<T>*)D.posa)[slot].w;
     ForceAcc<T, SM> acc;
     if (l == 0) acc.self_term(K, vi.w);
-    force_share<T, SM, G>(D, S, K, slot, l, pi, vi, a_i, acc, false);
+    force_share<false, T, SM, G>(D, S, K, (uint32_t)slot, wave_index((int)blockIdx.x) * (uint32_t)(SPHE_WAVE / G), l, pi,
+                                  vi, a_i, acc, false);
     acc.template merge<G>();
     if (l != 0) return;
     ForceOut<T> o;
@@ -2827,7 +2861,9 @@ static void launch_force_g(const DevState& D, int block, int remap, hipStream_t 
         klaunch(k_force_f64<G>, nblk, block, st, e0, e1, D, nblk, remap);
         return;
     }
-#define CALL(T, SM) klaunch(k_force_f32<SM, G>, nblk, block, st, e0, e1, D, nblk, remap)
+    const bool unit = D.h_unit != 0;
+#define CALL(T, SM) \
+    klaunch(unit ? k_force_f32<SM, G, G == 4> : k_force_f32<SM, G, false>, nblk, block, st, e0, e1, D, nblk, remap)
     SPHE_PREC_SWITCH(D.precision, CALL);
 #undef CALL
 }
