@@ -2,7 +2,7 @@
 //
 // One step (all scenes of a context at once), reference Erosion/fluid_system.h
 // FluidSystemSPH::Run (:104-183) + advance (:306-353):
-//   scan      counts -> cell starts (2 kernels; tiles no particle counted
+//   scan      counts -> cell starts (1 to 3 kernels; tiles no particle counted
 //             into are not read)
 //   scatter   each particle to its cell segment (arrival order); resets
 //             its cell's count for the next step
@@ -477,86 +477,66 @@ __global__ __launch_bounds__(256) void k_hash_count(DevState D)
     }
 }
 
-// A scan tile is 256 threads x ITEMS consecutive counts (ITEMS = 8, 16 or
-// 32: tiles of 2^11, 2^12 or 2^13 cells, DevState::scan_log2).
+// A scan tile is 256 threads x ITEMS counts (ITEMS = 8, 16 or 32: tiles of
+// 2^11, 2^12 or 2^13 cells, DevState::scan_log2).  A wave takes a run of
+// 64 ITEMS consecutive cells, four cells a lane at a time (chunks of 256
+// cells), so that its loads and stores are runs of consecutive lines.
 
-// Exclusive scan of v over a 256-thread block, with its total, and the
-// block total of a second value w: one LDS exchange (lds: 8 words).
-__device__ __forceinline__ uint32_t block_scan_sum(uint32_t v, uint32_t w, uint32_t* total, uint32_t* wtotal,
-                                                   uint32_t* lds)
+// Inclusive sums of x over the wave's lanes, in six DPP adds.
+__device__ __forceinline__ uint32_t wave_sums(uint32_t x)
 {
-    // wave-inclusive scan and wave sum with shuffles, then the 4 wave totals
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    uint32_t x = v;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        uint32_t y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
-    }
-    uint32_t r = w;
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) r += __shfl_xor(r, o, 64);
-    if (lane == 63) lds[wave] = x;
-    if (lane == 0) lds[4 + wave] = r;
-    __syncthreads();
-    uint32_t base = 0, tot = 0, wt = 0;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        const uint32_t t = lds[k];
-        if (k < wave) base += t;
-        tot += t;
-        wt += lds[4 + k];
-    }
-    *total = tot;
-    *wtotal = wt;
-    return base + x - v;
+#define SPHE_DPP_ADD(ctrl, rows) x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, ctrl, rows, 0xF, false)
+    SPHE_DPP_ADD(0x111, 0xF);  // row_shr 1, 2, 4, 8: within rows of 16 lanes
+    SPHE_DPP_ADD(0x112, 0xF);
+    SPHE_DPP_ADD(0x114, 0xF);
+    SPHE_DPP_ADD(0x118, 0xF);
+    SPHE_DPP_ADD(0x142, 0xA);  // row_bcast 15 into rows 1 and 3
+    SPHE_DPP_ADD(0x143, 0xC);  // row_bcast 31 into rows 2 and 3
+#undef SPHE_DPP_ADD
+    return x;
+}
+__device__ __forceinline__ uint32_t wave_total(uint32_t x)
+{
+    return (uint32_t)__builtin_amdgcn_readlane((int)wave_sums(x), 63);
 }
 
-// ITEMS consecutive words per thread, as 16-byte accesses where the whole
-// run is inside [0, n) (tiles start at multiples of 64 bytes).
+// First cell of chunk c of this lane's wave in the tile.
 template <int ITEMS>
-__device__ __forceinline__ void load_run(const uint32_t* __restrict__ p, int64_t base, int64_t n,
-                                         uint32_t* v)
+__device__ __forceinline__ int64_t tile_cell(int64_t tile, int c)
 {
-    if (base + ITEMS <= n) {
-        const uint4* q = (const uint4*)(p + base);
-#pragma unroll
-        for (int k = 0; k < ITEMS / 4; ++k) {
-            const uint4 a = q[k];
-            v[4 * k] = a.x; v[4 * k + 1] = a.y; v[4 * k + 2] = a.z; v[4 * k + 3] = a.w;
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i) v[i] = base + i < n ? p[base + i] : 0u;
-    }
-}
-
-// The same as cell records (start, 0).
-template <int ITEMS>
-__device__ __forceinline__ void store_run(uint2* __restrict__ p, int64_t base, int64_t n, const uint32_t* v)
-{
-    if (base + ITEMS <= n) {
-        uint4* q = (uint4*)(p + base);
-#pragma unroll
-        for (int k = 0; k < ITEMS / 2; ++k) q[k] = make_uint4(v[2 * k], 0u, v[2 * k + 1], 0u);
-    } else {
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i)
-            if (base + i < n) p[base + i] = make_uint2(v[i], 0u);
-    }
+    return tile * (256 * ITEMS) + (int64_t)(threadIdx.x >> 6) * (64 * ITEMS) + c * 256 + (threadIdx.x & 63) * 4;
 }
 
 template <int ITEMS>
-__device__ __forceinline__ void store_run(uint32_t* __restrict__ p, int64_t base, int64_t n, const uint32_t* v)
+__device__ __forceinline__ void load_tile(const uint32_t* __restrict__ p, int64_t tile, int64_t n, uint4* v)
 {
-    if (base + ITEMS <= n) {
-        uint4* q = (uint4*)(p + base);
 #pragma unroll
-        for (int k = 0; k < ITEMS / 4; ++k) q[k] = make_uint4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
+    for (int c = 0; c < ITEMS / 4; ++c) {
+        const int64_t i = tile_cell<ITEMS>(tile, c);
+        if (i + 4 <= n) v[c] = *(const uint4*)(p + i);
+        else v[c] = make_uint4(i < n ? p[i] : 0u, i + 1 < n ? p[i + 1] : 0u, i + 2 < n ? p[i + 2] : 0u, 0u);
+    }
+}
+
+// Four consecutive values, as plain words or as cell records (value, 0).
+__device__ __forceinline__ void store4(uint32_t* __restrict__ p, int64_t i, int64_t n, uint4 v)
+{
+    if (i + 4 <= n) *(uint4*)(p + i) = v;
+    else {
+        if (i < n) p[i] = v.x;
+        if (i + 1 < n) p[i + 1] = v.y;
+        if (i + 2 < n) p[i + 2] = v.z;
+    }
+}
+__device__ __forceinline__ void store4(uint2* __restrict__ p, int64_t i, int64_t n, uint4 v)
+{
+    if (i + 4 <= n) {
+        ((uint4*)(p + i))[0] = make_uint4(v.x, 0u, v.y, 0u);
+        ((uint4*)(p + i))[1] = make_uint4(v.z, 0u, v.w, 0u);
     } else {
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i)
-            if (base + i < n) p[base + i] = v[i];
+        if (i < n) p[i] = make_uint2(v.x, 0u);
+        if (i + 1 < n) p[i + 1] = make_uint2(v.y, 0u);
+        if (i + 2 < n) p[i + 2] = make_uint2(v.z, 0u);
     }
 }
 
@@ -571,24 +551,23 @@ __device__ __forceinline__ void scan_reduce_tile(const uint32_t* __restrict__ in
         if (threadIdx.x == 0) partial[tile] = 0u;
         return;
     }
-    const int64_t base = (int64_t)tile * (256 * ITEMS) + (int64_t)threadIdx.x * ITEMS;
-    uint32_t v[ITEMS];
-    load_run<ITEMS>(in, base, n, v);
+    uint4 v[ITEMS / 4];
+    load_tile<ITEMS>(in, tile, n, v);
     uint32_t s = 0;
 #pragma unroll
-    for (int i = 0; i < ITEMS; ++i) s += v[i];
-    uint32_t tot, none;
-    (void)block_scan_sum(0u, s, &none, &tot, lds);
-    if (threadIdx.x == 0) partial[tile] = tot;
+    for (int c = 0; c < ITEMS / 4; ++c) s += (v[c].x + v[c].y) + (v[c].z + v[c].w);
+    s = wave_total(s);
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) partial[tile] = (lds[0] + lds[1]) + (lds[2] + lds[3]);
 }
 
 template <int ITEMS>
 __global__ __launch_bounds__(256) void k_scan_reduce(const uint32_t* __restrict__ in, int64_t n,
-                                                     uint32_t* __restrict__ partial,
-                                                     const uint32_t* __restrict__ occ)
+                                                     uint32_t* __restrict__ partial)
 {
-    __shared__ uint32_t lds[8];
-    scan_reduce_tile<ITEMS>(in, n, partial, occ, (int)blockIdx.x, lds);
+    __shared__ uint32_t lds[4];
+    scan_reduce_tile<ITEMS>(in, n, partial, nullptr, (int)blockIdx.x, lds);
 }
 
 // Exclusive prefix of the n tile totals, in place, by one block of 1,024
@@ -605,16 +584,12 @@ __global__ __launch_bounds__(1024) void k_scan_tiles(uint32_t* __restrict__ part
     for (int64_t c0 = 0; c0 < n; c0 += 1024 * ITEMS) {
         const int64_t base = c0 + (int64_t)threadIdx.x * ITEMS;
         uint32_t v[ITEMS];
-        load_run<ITEMS>(partial, base, n, v);
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) v[i] = base + i < n ? partial[base + i] : 0u;
         uint32_t s = 0;
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i) s += v[i];
-        uint32_t x = s;  // inclusive scan over the wave, then the 16 wave totals
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t y = __shfl_up(x, o, 64);
-            if (lane >= o) x += y;
-        }
+        const uint32_t x = wave_sums(s);  // over the wave, then the 16 wave totals
         if (lane == 63) lds[wave] = x;
         __syncthreads();
         uint32_t before = 0, tot = 0;
@@ -631,70 +606,119 @@ __global__ __launch_bounds__(1024) void k_scan_tiles(uint32_t* __restrict__ part
             v[i] = run;
             run += c;
         }
-        store_run<ITEMS>(partial, base, n, v);
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i)
+            if (base + i < n) partial[base + i] = v[i];
         carry += tot;
         __syncthreads();  // the wave totals of the next chunk reuse lds
     }
 }
 
-// start[i] = exclusive prefix of counts, from partial[b]: the total of the
-// tiles before tile b (k_scan_tiles).  With zero_counts the counts are
-// reset to zero for the next arrivals (the particle sort instead has each
-// particle's scatter reset its own cell); the optional single word *zero is
-// set to zero_to.  occ (optional): the tile flags; an unflagged tile's counts are
-// not read (all zero), and each block clears its tile's flag once read.
-// fill (optional, with occ): per tile, the value all of an empty tile's
-// starts hold since the tile was last written empty (~0: not known); an
-// empty tile whose prefix equals it is not written again.
-// S: what a start is written as, a plain word or a cell record (start, 0).
-template <int ITEMS, typename S>
-__global__ __launch_bounds__(256) void k_scan_down(uint32_t* __restrict__ cnt, S* __restrict__ start,
-                                                   int64_t n, const uint32_t* __restrict__ partial,
-                                                   int zero_counts, unsigned long long* __restrict__ zero,
-                                                   unsigned long long zero_to,
-                                                   uint32_t* __restrict__ occ, uint32_t* __restrict__ fill)
+// Where a tile's prefix (the total of the tiles before it) comes from: a word
+// that k_scan_tiles left; the tiles' totals, added here; the counts before the
+// tile, added here, with no pass over the tiles before this one.  A launch
+// costs 4.5 us, so for few tiles the last two are faster although every block
+// repeats the sum: up to SCAN_SUM_TILES tiles a block adds 4 words a thread on
+// average at the limit, which its loads hide; up to SCAN_COUNT_TILES it reads
+// at most 256 KB of counts from L2.  Three launches against these: 12.8 -> 4.8
+// us on a grid of 2,900 cells and 13.2 -> 7.3 us on one of 39,000 (one launch),
+// 19.8 -> 13.4 us on 6.7M cells (two).  Runs of consecutive lines instead of
+// each thread's own 64 or 128 bytes: 57 -> 40 us on 16.7M cells (three).
+enum { SCAN_PREFIX, SCAN_SUMS, SCAN_COUNTS };
+#define SPHE_SCAN_SUM_TILES 4096
+#define SPHE_SCAN_COUNT_TILES 16
+
+// start = exclusive prefix of the counts of one tile.  With zero_counts the
+// counts are reset to zero for the next arrivals (not with SCAN_COUNTS; the
+// particle sort instead has each cell's first scatter reset its count).  occ
+// (optional): the tile flags; an unflagged tile's counts are not read (all
+// zero), and the block clears its tile's flag once read.  fill (optional, with
+// occ): per tile, the value all of an empty tile's starts hold since the tile
+// was last written empty (~0: not known); an empty tile whose prefix equals it
+// is not written again.
+template <int ITEMS, int FROM, typename S>
+__device__ __forceinline__ void scan_down_tile(uint32_t* __restrict__ cnt, S* __restrict__ start, int64_t n,
+                                               const uint32_t* __restrict__ partial, bool zero_counts,
+                                               uint32_t* __restrict__ occ, uint32_t* __restrict__ fill, int tile,
+                                               uint32_t* lds)
 {
-    if (zero && blockIdx.x == 0 && threadIdx.x == 0) *zero = zero_to;
-    __shared__ uint32_t lds[8];
-    const int64_t base = (int64_t)blockIdx.x * (256 * ITEMS) + (int64_t)threadIdx.x * ITEMS;
-    const bool empty = occ && occ[blockIdx.x] == 0u;  // block-uniform
-    const uint32_t filled = fill ? fill[blockIdx.x] : ~0u;
-    uint32_t v[ITEMS];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const bool empty = occ && occ[tile] == 0u;  // block-uniform
+    const uint32_t filled = fill ? fill[tile] : ~0u;
+    uint4 v[ITEMS / 4];
     if (empty) {
 #pragma unroll
-        for (int i = 0; i < ITEMS; ++i) v[i] = 0u;
+        for (int c = 0; c < ITEMS / 4; ++c) v[c] = make_uint4(0u, 0u, 0u, 0u);
     } else {
-        load_run<ITEMS>(cnt, base, n, v);
+        load_tile<ITEMS>(cnt, tile, n, v);
     }
-    // the total of the tiles before this one (k_scan_tiles' prefix)
-    const uint32_t ptot = partial[blockIdx.x];
-    uint32_t s = 0;
+    uint32_t pre = 0;  // this thread's share of the prefix
+    if constexpr (FROM == SCAN_PREFIX) {
+        pre = threadIdx.x == 0 ? partial[tile] : 0u;
+    } else if constexpr (FROM == SCAN_SUMS) {
+#pragma unroll 4
+        for (int i = (int)threadIdx.x; i < tile; i += 256) pre += partial[i];
+    } else {
+        // whole tiles, all of a tile's loads in flight
+        for (int k = 0; k < tile; ++k) {
+            uint4 q[ITEMS / 4];
 #pragma unroll
-    for (int i = 0; i < ITEMS; ++i) s += v[i];
-    uint32_t tot, none;
-    uint32_t run = block_scan_sum(s, 0u, &tot, &none, lds);
-    run += ptot;
-    uint32_t z[ITEMS];
+            for (int c = 0; c < ITEMS / 4; ++c) q[c] = *(const uint4*)(cnt + tile_cell<ITEMS>(k, c));
 #pragma unroll
-    for (int i = 0; i < ITEMS; ++i) {
-        const uint32_t c = v[i];
-        v[i] = run;
-        run += c;
-        z[i] = 0u;
-    }
-    // an empty tile's starts all equal ptot (its prefix): unwritten when they
-    // already hold it
-    if (!(empty && filled == ptot)) store_run<ITEMS>(start, base, n, v);
-    if (zero_counts && !empty) store_run<ITEMS>(cnt, base, n, z);
-    // every thread read the flag and the fill word before the barrier of the
-    // scan above
-    if (threadIdx.x == 0) {
-        if (occ && !empty) occ[blockIdx.x] = 0u;
-        if (fill) {
-            const uint32_t nf = empty ? ptot : ~0u;
-            if (nf != filled) fill[blockIdx.x] = nf;
+            for (int c = 0; c < ITEMS / 4; ++c) pre += (q[c].x + q[c].y) + (q[c].z + q[c].w);
         }
     }
+    // sums over the wave of each chunk, then of the waves before
+    uint32_t run[ITEMS / 4], sum = 0;
+#pragma unroll
+    for (int c = 0; c < ITEMS / 4; ++c) {
+        const uint32_t q = (v[c].x + v[c].y) + (v[c].z + v[c].w);
+        const uint32_t x = wave_sums(q);
+        run[c] = sum + x - q;
+        sum += (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+    }
+    const uint32_t wpre = wave_total(pre);
+    if (lane == 0) {
+        lds[wave] = sum;
+        lds[4 + wave] = wpre;
+    }
+    __syncthreads();
+    const uint32_t ptot = (lds[4] + lds[5]) + (lds[6] + lds[7]);
+    uint32_t base = ptot;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) base += k < wave ? lds[k] : 0u;
+    // an empty tile's starts all equal ptot: unwritten when they already do
+    if (!(empty && filled == ptot)) {
+#pragma unroll
+        for (int c = 0; c < ITEMS / 4; ++c) {
+            uint4 o;
+            o.x = base + run[c];
+            o.y = o.x + v[c].x;
+            o.z = o.y + v[c].y;
+            o.w = o.z + v[c].z;
+            store4(start, tile_cell<ITEMS>(tile, c), n, o);
+        }
+    }
+    if (zero_counts && !empty)
+#pragma unroll
+        for (int c = 0; c < ITEMS / 4; ++c)
+            store4(cnt, tile_cell<ITEMS>(tile, c), n, make_uint4(0u, 0u, 0u, 0u));
+    // every thread read the flag and the fill word before the barrier
+    if (threadIdx.x == 0) {
+        if (occ && !empty) occ[tile] = 0u;
+        if (fill) {
+            const uint32_t nf = empty ? ptot : ~0u;
+            if (nf != filled) fill[tile] = nf;
+        }
+    }
+}
+
+template <int ITEMS, int FROM>
+__global__ __launch_bounds__(256) void k_scan_down(uint32_t* __restrict__ cnt, uint32_t* __restrict__ start, int64_t n,
+                                                   const uint32_t* __restrict__ partial, int zero_counts)
+{
+    __shared__ uint32_t lds[8];
+    scan_down_tile<ITEMS, FROM>(cnt, start, n, partial, zero_counts != 0, nullptr, nullptr, (int)blockIdx.x, lds);
 }
 
 __global__ __launch_bounds__(256) void k_scatter(DevState D)
@@ -2257,20 +2281,32 @@ __global__ __launch_bounds__(256) void k_heights(DevState D)
     if (t0 < D.TC) heights_quad(D, t0);
 }
 
-// The particle scan's first kernel and the terrain heights in one launch
-// (both need only the force pass done): blocks [0, nscan) total the count
-// tiles, the others compute heights from the volumes the last force pass
-// eroded, before this step's force pass samples them.
+// The particle scan's kernels.  Blocks past the nscan tiles of the first one
+// launched compute terrain heights (both need only the force pass done): from
+// the volumes the last force pass eroded, before this step's samples them.
+__device__ __forceinline__ bool heights_block(const DevState& D, int nscan)
+{
+    if ((int)blockIdx.x < nscan) return false;
+    const int64_t t0 = ((int64_t)((int)blockIdx.x - nscan) * blockDim.x + threadIdx.x) * 4;
+    if (t0 < D.TC) heights_quad(D, t0);
+    return true;
+}
+
 template <int ITEMS>
-__global__ __launch_bounds__(256) void k_scan_reduce_heights(DevState D, int nscan)
+__global__ __launch_bounds__(256) void k_scan_reduce_cells(DevState D, int nscan)
+{
+    __shared__ uint32_t lds[4];
+    if (heights_block(D, nscan)) return;  // block-uniform: no barrier is skipped by part of a block
+    scan_reduce_tile<ITEMS>(D.cnt, D.C + 1, D.partial, D.tocc, (int)blockIdx.x, lds);
+}
+
+template <int ITEMS, int FROM>
+__global__ __launch_bounds__(256) void k_scan_cells(DevState D, int nscan)
 {
     __shared__ uint32_t lds[8];
-    if ((int)blockIdx.x >= nscan) {  // block-uniform: no barrier is skipped by part of a block
-        const int64_t t0 = ((int64_t)(blockIdx.x - nscan) * blockDim.x + threadIdx.x) * 4;
-        if (t0 < D.TC) heights_quad(D, t0);
-        return;
-    }
-    scan_reduce_tile<ITEMS>(D.cnt, D.C + 1, D.partial, D.tocc, (int)blockIdx.x, lds);
+    if (FROM == SCAN_COUNTS && heights_block(D, nscan)) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) *D.ptop = (unsigned long long)D.pool_origin;  // the pool's claims
+    scan_down_tile<ITEMS, FROM>(D.cnt, D.cells, D.C + 1, D.partial, false, D.tocc, D.tfill, (int)blockIdx.x, lds);
 }
 
 // Two-phase erosion, phase 2a: count exchanges per terrain cell.
@@ -2759,35 +2795,37 @@ void sphe_launch_hash(const DevState& D, hipStream_t st, hipEvent_t e0, hipEvent
     else klaunch(k_hash_count<float>, grid_of(D.P, 256), 256, st, e0, e1, D);
 }
 
-template <int ITEMS, typename S>
-static void launch_scan_t(uint32_t* cnt, S* start, int64_t n, uint32_t* partial, bool zero_counts,
-                          unsigned long long* zero, unsigned long long zero_to, uint32_t* occ, uint32_t* fill,
-                          hipStream_t st, hipEvent_t e0, hipEvent_t e1)
+void sphe_launch_scan(uint32_t* cnt, uint32_t* start, int64_t n, uint32_t* partial, bool zero_counts, hipStream_t st)
 {
+    constexpr int ITEMS = (1 << SPHE_SCAN_LOG2_DEFAULT) / 256;
     const int64_t nb = (n + 256 * ITEMS - 1) / (256 * ITEMS);
-    klaunch(k_scan_reduce<ITEMS>, (unsigned)nb, 256, st, e0, nullptr, (const uint32_t*)cnt, n, partial,
-            (const uint32_t*)occ);
-    klaunch(k_scan_tiles, 1, 1024, st, nullptr, nullptr, partial, nb);
-    klaunch(k_scan_down<ITEMS, S>, (unsigned)nb, 256, st, nullptr, e1, cnt, start, n, (const uint32_t*)partial,
-            zero_counts ? 1 : 0, zero, zero_to, occ, occ ? fill : nullptr);
+    const bool sums = nb <= SPHE_SCAN_SUM_TILES;
+    klaunch(k_scan_reduce<ITEMS>, (unsigned)nb, 256, st, nullptr, nullptr, (const uint32_t*)cnt, n, partial);
+    if (!sums) klaunch(k_scan_tiles, 1, 1024, st, nullptr, nullptr, partial, nb);
+    klaunch(sums ? k_scan_down<ITEMS, SCAN_SUMS> : k_scan_down<ITEMS, SCAN_PREFIX>, (unsigned)nb, 256, st, nullptr,
+            nullptr, cnt, start, n, (const uint32_t*)partial, zero_counts ? 1 : 0);
 }
 
-void sphe_launch_scan(uint32_t* cnt, uint32_t* start, int64_t n, uint32_t* partial, bool zero_counts,
-                      hipStream_t st, hipEvent_t e0, hipEvent_t e1)
+template <int ITEMS>
+static void launch_scan_cells_t(const DevState& D, bool heights, hipStream_t st, hipEvent_t e0, hipEvent_t e1)
 {
-    launch_scan_t<(1 << SPHE_SCAN_LOG2_DEFAULT) / 256>(cnt, start, n, partial, zero_counts, nullptr, 0ull, nullptr,
-                                                       nullptr, st, e0, e1);
+    const int nb = (int)((D.C + 1 + 256 * ITEMS - 1) / (256 * ITEMS));
+    const int nh = heights ? (int)grid_of(D.TC / 4, 256) : 0;  // TC: a multiple of 64
+    if (nb <= SPHE_SCAN_COUNT_TILES) {
+        klaunch(k_scan_cells<ITEMS, SCAN_COUNTS>, nb + nh, 256, st, e0, e1, D, nb);
+        return;
+    }
+    const bool sums = nb <= SPHE_SCAN_SUM_TILES;
+    klaunch(k_scan_reduce_cells<ITEMS>, nb + nh, 256, st, e0, nullptr, D, nb);
+    if (!sums) klaunch(k_scan_tiles, 1, 1024, st, nullptr, nullptr, D.partial, (int64_t)nb);
+    klaunch(sums ? k_scan_cells<ITEMS, SCAN_SUMS> : k_scan_cells<ITEMS, SCAN_PREFIX>, nb, 256, st, nullptr, e1, D, nb);
 }
 
-void sphe_launch_scan_cells(const DevState& D, hipStream_t st, hipEvent_t e0, hipEvent_t e1)
+void sphe_launch_scan_cells(const DevState& D, bool heights, hipStream_t st, hipEvent_t e0, hipEvent_t e1)
 {
-    const unsigned long long to = (unsigned long long)D.pool_origin;
-    const int64_t n = D.C + 1;
-    if (D.scan_log2 == 11)
-        launch_scan_t<8>(D.cnt, D.cells, n, D.partial, false, D.ptop, to, D.tocc, D.tfill, st, e0, e1);
-    else if (D.scan_log2 == 13)
-        launch_scan_t<32>(D.cnt, D.cells, n, D.partial, false, D.ptop, to, D.tocc, D.tfill, st, e0, e1);
-    else launch_scan_t<16>(D.cnt, D.cells, n, D.partial, false, D.ptop, to, D.tocc, D.tfill, st, e0, e1);
+    if (D.scan_log2 == 11) launch_scan_cells_t<8>(D, heights, st, e0, e1);
+    else if (D.scan_log2 == 13) launch_scan_cells_t<32>(D, heights, st, e0, e1);
+    else launch_scan_cells_t<16>(D, heights, st, e0, e1);
 }
 
 int64_t sphe_scan_partials(int64_t n) { return (n + (1 << SPHE_SCAN_LOG2_MIN) - 1) >> SPHE_SCAN_LOG2_MIN; }
@@ -2890,25 +2928,6 @@ void sphe_launch_force(const DevState& D, int block, int remap, int lanes, hipSt
     case 8: launch_force_g<8>(D, block, remap, st, e0, e1); break;
     default: launch_force_g<4>(D, block, remap, st, e0, e1); break;
     }
-}
-
-template <int ITEMS>
-static void launch_scan_heights_t(const DevState& D, hipStream_t st, hipEvent_t e0, hipEvent_t e1)
-{
-    const int64_t n = D.C + 1;
-    const int64_t nb = (n + 256 * ITEMS - 1) / (256 * ITEMS);
-    const int64_t nh = (int64_t)grid_of(D.TC / 4, 256);  // TC: a multiple of 64
-    klaunch(k_scan_reduce_heights<ITEMS>, (unsigned)(nb + nh), 256, st, e0, nullptr, D, (int)nb);
-    klaunch(k_scan_tiles, 1, 1024, st, nullptr, nullptr, D.partial, nb);
-    klaunch(k_scan_down<ITEMS, uint2>, (unsigned)nb, 256, st, nullptr, e1, D.cnt, D.cells, n, (const uint32_t*)D.partial,
-            0, D.ptop, (unsigned long long)D.pool_origin, D.tocc, D.tfill);
-}
-
-void sphe_launch_scan_heights(const DevState& D, hipStream_t st, hipEvent_t e0, hipEvent_t e1)
-{
-    if (D.scan_log2 == 11) launch_scan_heights_t<8>(D, st, e0, e1);
-    else if (D.scan_log2 == 13) launch_scan_heights_t<32>(D, st, e0, e1);
-    else launch_scan_heights_t<16>(D, st, e0, e1);
 }
 
 void sphe_launch_heights(const DevState& D, hipStream_t st, hipEvent_t e0, hipEvent_t e1)

@@ -10,13 +10,13 @@
 void sphe_launch_hash(const DevState& D, hipStream_t st, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 // Exclusive prefix of n counts; with zero_counts the counts are reset.
 void sphe_launch_scan(uint32_t* cnt, uint32_t* start, int64_t n, uint32_t* partial, bool zero_counts,
-                      hipStream_t st, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
-// The particle scan: counts -> cell records, the pool's claim counter reset.
-void sphe_launch_scan_cells(const DevState& D, hipStream_t st, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
+                      hipStream_t st);
+// The particle scan: counts -> cell records, the pool's claim counter reset;
+// with heights also the terrain heights, in its first launch.
+void sphe_launch_scan_cells(const DevState& D, bool heights, hipStream_t st, hipEvent_t e0 = nullptr,
+                            hipEvent_t e1 = nullptr);
 // tiles of n counts at the smallest tile size (the size of the per-tile arrays)
 int64_t sphe_scan_partials(int64_t n);
-// The particle scan with the terrain heights computed in its first launch.
-void sphe_launch_scan_heights(const DevState& D, hipStream_t st, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 void sphe_launch_scatter(const DevState& D, hipStream_t st, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 void sphe_launch_reorder(const DevState& D, hipStream_t st, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 void sphe_launch_density(const DevState& D, int block, int remap, int lanes, hipStream_t st,

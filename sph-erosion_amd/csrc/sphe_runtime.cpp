@@ -850,8 +850,7 @@ void launch_sort(sphe_ctx* c)
         Timed t(c, "scan");
         // with erosion the terrain heights of the last force pass are computed
         // in the scan's first launch (this step's force pass samples them)
-        if (any_erosion(c, -1) && D.TC > 0) sphe_launch_scan_heights(D, c->stream, t.a, t.b);
-        else sphe_launch_scan_cells(D, c->stream, t.a, t.b);
+        sphe_launch_scan_cells(D, any_erosion(c, -1) && D.TC > 0, c->stream, t.a, t.b);
     }
     {
         Timed t(c, "scatter");

@@ -72,3 +72,48 @@ def test_coincident_neighbours_bit_exact_twin(yz):
     near[2::3, 1] += 1.02e-4
     pos = np.concatenate([base, near])[rng.permutation(420)]
     _compare(_params(h, 0.2, dt=1e-6), pos, yz)
+
+
+def _cells(p, yz=2):
+    """Cells of a scene's grid (one pad cell not counted)."""
+    ctx = sphe.Context()
+    ctx.set_yz_split(yz)
+    sid = ctx.add_scene(p)
+    c = ctx.debug_consts(sid)
+    return int(c["dim_x"] * c["dim_y"] * c["dim_z"])
+
+
+@pytest.mark.parametrize("tiles", [2, 16, 17, 4096, 4097])
+def test_scan_forms_give_the_same_steps(tiles):
+    """The cell scan takes one launch up to 16 tiles, two up to 4,096, three
+    beyond: a scene steps to the same bits beside scenes that bring the
+    context to exactly that many tiles (of 2,048 cells)."""
+    h = 0.0457
+    p = _params(h, 0.2, dt=1e-4)
+    rng = np.random.default_rng(11)
+    pos = rng.uniform(-0.12, 0.12, (2000, 3)).astype(np.float32)
+    alone = sphe.Context()
+    s0 = alone.add_scene(p)
+    alone.set_particles(s0, pos)
+    alone.step(6)
+    want = alone.state_f64(s0)
+
+    ctx = sphe.Context()
+    ctx.set_scan_tile(11)
+    sid = ctx.add_scene(p)
+    ctx.set_particles(sid, pos)
+    # other scenes, the largest first, while more than a tile is left; a
+    # scene's cells are followed by one pad cell, the context's by one more
+    left = 2048 * tiles - (_cells(p) + 1) - 1
+    for half in (2.9, 0.4, 0.2, 0.1, 0.05, 0.01):
+        n = _cells(_params(h, half)) + 1
+        while left >= 2048 and n <= left:
+            left -= n
+            o = ctx.add_scene(_params(h, half, dt=1e-4))
+            # three falling particles, so that far tiles fill and empty
+            ctx.set_particles(o, np.float32(0.4 * half) * np.array([[1, 1, 1], [-1, 1, 1], [1, -1, 1]], np.float32))
+    assert 0 <= left < 2048  # the last tile is partly filled
+    ctx.step(6)
+    got = ctx.state_f64(sid)
+    assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+    assert ctx.status() == 0
