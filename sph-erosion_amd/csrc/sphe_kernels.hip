@@ -2077,6 +2077,20 @@ __device__ __forceinline__ void force_share(const DevState& D, const SceneDev& S
     force_share_walk<T, SM, G>(D, S, K, wslot + (t & (SPHE_WAVE - 1)) / G, l, pi, vi, a_i, acc, nbmax, count);
 }
 
+// Copies the list-overflow words (largest overflowing count, failed pool
+// claims) and the pool entries the density pass claimed, all final once it is
+// done, into host memory mapped for the device (vector stores), where the host
+// reads them between step sequences without waiting for the stream.
+__device__ __forceinline__ void publish(const DevState& D)
+{
+    const unsigned long long t = *D.ptop;
+    volatile uint32_t* d = D.pub;
+    d[0] = D.ovf[0];
+    d[1] = D.ovf[1];
+    d[2] = (uint32_t)t;
+    d[3] = (uint32_t)(t >> 32);
+}
+
 // One G-lane group per particle: the lanes sum their shares, merge them
 // (xor shuffles), and lane 0 integrates, collides, erodes, stores the new
 // state and counts the particle's next cell.
@@ -2088,6 +2102,7 @@ __device__ __forceinline__ void force_body(const DevState& D, int b)
     // waves are whole)
     const uint32_t wslot = wave_index(b) * (uint32_t)(SPHE_WAVE / G);
     if (wslot >= (uint64_t)D.P) return;
+    if (b == 0 && threadIdx.x == 0) publish(D);  // no launch of its own (4 us)
     const uint32_t slot0 = wslot + (uint32_t)(threadIdx.x & (SPHE_WAVE - 1)) / G;
     const SceneDev& S = D.scenes[wave_scene(D.chunk_scene, wslot)];
     V4<T>* __restrict__ upos = (V4<T>*)D.u_pos;
@@ -2284,6 +2299,8 @@ __global__ __launch_bounds__(256) void k_heights(DevState D)
 // The particle scan's kernels.  Blocks past the nscan tiles of the first one
 // launched compute terrain heights (both need only the force pass done): from
 // the volumes the last force pass eroded, before this step's samples them.
+// first: the first step of a call, whose status word starts from 0 (later
+// kernels of the step set its bits).
 __device__ __forceinline__ bool heights_block(const DevState& D, int nscan)
 {
     if ((int)blockIdx.x < nscan) return false;
@@ -2293,17 +2310,19 @@ __device__ __forceinline__ bool heights_block(const DevState& D, int nscan)
 }
 
 template <int ITEMS>
-__global__ __launch_bounds__(256) void k_scan_reduce_cells(DevState D, int nscan)
+__global__ __launch_bounds__(256) void k_scan_reduce_cells(DevState D, int nscan, int first)
 {
     __shared__ uint32_t lds[4];
+    if (first && blockIdx.x == 0 && threadIdx.x == 0) *D.status = 0u;
     if (heights_block(D, nscan)) return;  // block-uniform: no barrier is skipped by part of a block
     scan_reduce_tile<ITEMS>(D.cnt, D.C + 1, D.partial, D.tocc, (int)blockIdx.x, lds);
 }
 
 template <int ITEMS, int FROM>
-__global__ __launch_bounds__(256) void k_scan_cells(DevState D, int nscan)
+__global__ __launch_bounds__(256) void k_scan_cells(DevState D, int nscan, int first)
 {
     __shared__ uint32_t lds[8];
+    if (first && blockIdx.x == 0 && threadIdx.x == 0) *D.status = 0u;
     if (FROM == SCAN_COUNTS && heights_block(D, nscan)) return;
     if (blockIdx.x == 0 && threadIdx.x == 0) *D.ptop = (unsigned long long)D.pool_origin;  // the pool's claims
     scan_down_tile<ITEMS, FROM>(D.cnt, D.cells, D.C + 1, D.partial, false, D.tocc, D.tfill, (int)blockIdx.x, lds);
@@ -2575,22 +2594,6 @@ __global__ void k_clear_status(uint32_t* status)
     if (threadIdx.x == 0 && blockIdx.x == 0) *status = 0u;
 }
 
-// Copies the list-overflow words (largest overflowing count, failed pool
-// claims) and the pool entries the last density pass claimed into host memory
-// mapped for the device (vector stores), where the host reads them between
-// step sequences without waiting for the stream.
-__global__ void k_publish(const uint32_t* __restrict__ ovf, const unsigned long long* __restrict__ ptop,
-                          uint32_t* __restrict__ dst)
-{
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    const unsigned long long t = *ptop;
-    volatile uint32_t* d = dst;
-    d[0] = ovf[0];
-    d[1] = ovf[1];
-    d[2] = (uint32_t)t;
-    d[3] = (uint32_t)(t >> 32);
-}
-
 // Mass bookkeeping of one scene: FP64 sums of terrain volume and carried
 // sediment, and the exact mod-2^64 sum of their fixed-point units.  Each
 // block writes its partial; k_mass_final adds them in block order.
@@ -2807,25 +2810,26 @@ void sphe_launch_scan(uint32_t* cnt, uint32_t* start, int64_t n, uint32_t* parti
 }
 
 template <int ITEMS>
-static void launch_scan_cells_t(const DevState& D, bool heights, hipStream_t st, hipEvent_t e0, hipEvent_t e1)
+static void launch_scan_cells_t(const DevState& D, bool heights, int first, hipStream_t st, hipEvent_t e0, hipEvent_t e1)
 {
     const int nb = (int)((D.C + 1 + 256 * ITEMS - 1) / (256 * ITEMS));
     const int nh = heights ? (int)grid_of(D.TC / 4, 256) : 0;  // TC: a multiple of 64
     if (nb <= SPHE_SCAN_COUNT_TILES) {
-        klaunch(k_scan_cells<ITEMS, SCAN_COUNTS>, nb + nh, 256, st, e0, e1, D, nb);
+        klaunch(k_scan_cells<ITEMS, SCAN_COUNTS>, nb + nh, 256, st, e0, e1, D, nb, first);
         return;
     }
     const bool sums = nb <= SPHE_SCAN_SUM_TILES;
-    klaunch(k_scan_reduce_cells<ITEMS>, nb + nh, 256, st, e0, nullptr, D, nb);
+    klaunch(k_scan_reduce_cells<ITEMS>, nb + nh, 256, st, e0, nullptr, D, nb, first);
     if (!sums) klaunch(k_scan_tiles, 1, 1024, st, nullptr, nullptr, D.partial, (int64_t)nb);
-    klaunch(sums ? k_scan_cells<ITEMS, SCAN_SUMS> : k_scan_cells<ITEMS, SCAN_PREFIX>, nb, 256, st, nullptr, e1, D, nb);
+    klaunch(sums ? k_scan_cells<ITEMS, SCAN_SUMS> : k_scan_cells<ITEMS, SCAN_PREFIX>, nb, 256, st, nullptr, e1, D, nb,
+            0);
 }
 
-void sphe_launch_scan_cells(const DevState& D, bool heights, hipStream_t st, hipEvent_t e0, hipEvent_t e1)
+void sphe_launch_scan_cells(const DevState& D, bool heights, bool first, hipStream_t st, hipEvent_t e0, hipEvent_t e1)
 {
-    if (D.scan_log2 == 11) launch_scan_cells_t<8>(D, heights, st, e0, e1);
-    else if (D.scan_log2 == 13) launch_scan_cells_t<32>(D, heights, st, e0, e1);
-    else launch_scan_cells_t<16>(D, heights, st, e0, e1);
+    if (D.scan_log2 == 11) launch_scan_cells_t<8>(D, heights, first, st, e0, e1);
+    else if (D.scan_log2 == 13) launch_scan_cells_t<32>(D, heights, first, st, e0, e1);
+    else launch_scan_cells_t<16>(D, heights, first, st, e0, e1);
 }
 
 int64_t sphe_scan_partials(int64_t n) { return (n + (1 << SPHE_SCAN_LOG2_MIN) - 1) >> SPHE_SCAN_LOG2_MIN; }
@@ -2946,11 +2950,6 @@ void sphe_launch_two_phase(const DevState& D, hipStream_t st, hipEvent_t e0, hip
 }
 
 void sphe_launch_clear_status(const DevState& D, hipStream_t st) { k_clear_status<<<1, 64, 0, st>>>(D.status); }
-
-void sphe_launch_publish(const DevState& D, uint32_t* host_word, hipStream_t st)
-{
-    k_publish<<<1, 64, 0, st>>>(D.ovf, D.ptop, host_word);
-}
 
 void sphe_launch_terrain_mesh(const float* H, int nx, int nz, float cell, float ox, float oz, float* out,
                               hipStream_t st)

@@ -12,8 +12,9 @@ void sphe_launch_hash(const DevState& D, hipStream_t st, hipEvent_t e0 = nullptr
 void sphe_launch_scan(uint32_t* cnt, uint32_t* start, int64_t n, uint32_t* partial, bool zero_counts,
                       hipStream_t st);
 // The particle scan: counts -> cell records, the pool's claim counter reset;
-// with heights also the terrain heights, in its first launch.
-void sphe_launch_scan_cells(const DevState& D, bool heights, hipStream_t st, hipEvent_t e0 = nullptr,
+// with heights also the terrain heights, in its first launch; with first the
+// status word is cleared.
+void sphe_launch_scan_cells(const DevState& D, bool heights, bool first, hipStream_t st, hipEvent_t e0 = nullptr,
                             hipEvent_t e1 = nullptr);
 // tiles of n counts at the smallest tile size (the size of the per-tile arrays)
 int64_t sphe_scan_partials(int64_t n);
@@ -26,9 +27,6 @@ void sphe_launch_force(const DevState& D, int block, int remap, int lanes, hipSt
 void sphe_launch_heights(const DevState& D, hipStream_t st, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 void sphe_launch_two_phase(const DevState& D, hipStream_t st, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 void sphe_launch_clear_status(const DevState& D, hipStream_t st);
-// Copies D.ovf[0], D.ovf[1] and the 64-bit *D.ptop (low, high) to four host
-// words mapped for the device.
-void sphe_launch_publish(const DevState& D, uint32_t* host_word, hipStream_t st);
 void sphe_launch_terrain_mesh(const float* H, int nx, int nz, float cell, float ox, float oz, float* out,
                               hipStream_t st);
 // The 112-byte record's values of the particle at sorted slot *slotp (device

@@ -88,9 +88,13 @@ struct sphe_ctx {
     bool table_uploaded = false;
 
     bool use_graph = true;
-    // captured step sequences by length (steps per graph launch)
-    std::map<int, std::pair<hipGraph_t, hipGraphExec_t>> graphs;
+    // captured step sequences by length (steps per graph launch) and whether
+    // the sequence starts a call (clears the status word)
+    std::map<std::pair<int, bool>, std::pair<hipGraph_t, hipGraphExec_t>> graphs;
     std::string graph_sig;
+    // calls by the length of what their whole sequences left over, under the
+    // current plan: a length that comes again gets a sequence of its own
+    std::map<int, int> rest_seen;
     // the list-overflow word as the last step sequence published it: host
     // memory mapped for the device (h_ovf_dev), written by a kernel at the
     // end of every sequence and read by the host without a stream wait
@@ -417,6 +421,7 @@ void drop_graphs(sphe_ctx* c)
     }
     c->graphs.clear();
     c->graph_sig.clear();
+    c->rest_seen.clear();
 }
 
 void free_device(sphe_ctx* c)
@@ -558,6 +563,7 @@ int build_layout(sphe_ctx* c)
     DALLOC(D.pbase, Pn * 4);
     DALLOC(D.ptop, 64);
     DALLOC(D.ovf, 64);
+    D.pub = c->h_ovf_dev;
     DALLOC(D.status, 64);
     DALLOC(D.work, 64);
     D.persistent = c->persistent ? 1 : 0;
@@ -843,14 +849,14 @@ bool any_erosion(const sphe_ctx* c, int mode)
     return false;
 }
 
-void launch_sort(sphe_ctx* c)
+void launch_sort(sphe_ctx* c, bool first)
 {
     const DevState& D = c->D;
     {
         Timed t(c, "scan");
         // with erosion the terrain heights of the last force pass are computed
         // in the scan's first launch (this step's force pass samples them)
-        sphe_launch_scan_cells(D, any_erosion(c, -1) && D.TC > 0, c->stream, t.a, t.b);
+        sphe_launch_scan_cells(D, any_erosion(c, -1) && D.TC > 0, first, c->stream, t.a, t.b);
     }
     {
         Timed t(c, "scatter");
@@ -862,10 +868,11 @@ void launch_sort(sphe_ctx* c)
     }
 }
 
-void launch_step(sphe_ctx* c)
+// first: the first step of a call (its scan clears the status word)
+void launch_step(sphe_ctx* c, bool first)
 {
     const DevState& D = c->D;
-    launch_sort(c);
+    launch_sort(c, first);
     {
         Timed t(c, "density");
         sphe_launch_density(D, c->block, c->remap, c->lanes, c->stream, t.a, t.b);
@@ -894,24 +901,28 @@ std::string plan_signature(const sphe_ctx* c)
     return b;
 }
 
-// The executable graph of a sequence of k steps (captured on first use; all
-// sequences are dropped when the launch plan changes).  The sequence ends by
-// publishing the list-overflow word to the host.
-int ensure_graph(sphe_ctx* c, int k, hipGraphExec_t* exec)
+// Drops the captured sequences when the launch plan has changed.
+void check_plan(sphe_ctx* c)
 {
     const std::string sig = plan_signature(c);
     if (sig != c->graph_sig) {
         drop_graphs(c);
         c->graph_sig = sig;
     }
-    auto it = c->graphs.find(k);
+}
+
+// The executable graph of a sequence of k steps, captured on first use.  Every
+// force pass in it publishes the list-overflow words to the host.
+int ensure_graph(sphe_ctx* c, int k, bool first, hipGraphExec_t* exec)
+{
+    const auto key = std::make_pair(k, first);
+    auto it = c->graphs.find(key);
     if (it != c->graphs.end()) {
         *exec = it->second.second;
         return SPHE_OK;
     }
     HIPCHK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    for (int i = 0; i < k; ++i) launch_step(c);
-    sphe_launch_publish(c->D, c->h_ovf_dev, c->stream);
+    for (int i = 0; i < k; ++i) launch_step(c, first && i == 0);
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(c->stream, &g);
     if (e != hipSuccess) return fail(c, SPHE_EHIP, "graph capture: %s", hipGetErrorString(e));
@@ -921,7 +932,7 @@ int ensure_graph(sphe_ctx* c, int k, hipGraphExec_t* exec)
         (void)hipGraphDestroy(g);
         return fail(c, SPHE_EHIP, "graph instantiate: %s", hipGetErrorString(e));
     }
-    c->graphs[k] = std::make_pair(g, x);
+    c->graphs[key] = std::make_pair(g, x);
     *exec = x;
     return SPHE_OK;
 }
@@ -1052,12 +1063,26 @@ int grow_lists(sphe_ctx* c)
 // too short for the state grow at most this many launches late.
 const int kInFlight = 2;
 
+// Whether the `rest` steps that a call's whole sequences leave over run as one
+// captured sequence: a single step always, more from the second call with that
+// rest on, for up to kMaxSequences sequences in all (else one step at a time,
+// launched directly).  Between two one-step graphs the device idles for 13 us
+// (a tenth of a step of 100,000 particles) and between two direct steps for
+// 10; a capture costs the host about as much per step, once, which a call that
+// never comes again would not win back.
+const size_t kMaxSequences = 10;
+bool rest_as_sequence(sphe_ctx* c, int rest, bool first)
+{
+    if (rest == 0) return false;
+    if (c->graphs.count(std::make_pair(rest, first))) return true;
+    return (rest == 1 && first) || (++c->rest_seen[rest] > 1 && c->graphs.size() < kMaxSequences);
+}
+
 int do_steps(sphe_ctx* c, int nsteps)
 {
     int r = prepare(c);
     if (r) return r;
     if (c->D.P == 0) return SPHE_OK;
-    sphe_launch_clear_status(c->D, c->stream);
     if (!c->counted) {
         r = recount(c);
         if (r) return r;
@@ -1065,28 +1090,38 @@ int do_steps(sphe_ctx* c, int nsteps)
     HIPCHK(c, hipGetLastError());
     const bool graph = c->use_graph && !c->profiling;
     // Graph mode: sequences of c->seq_steps steps in one graph launch, the rest
-    // one step per launch; direct launches (profiling, or graphs off) one
-    // step at a time.  Before each launch the host looks at the overflow word
-    // the last finished sequence published.
+    // in one sequence or one step at a time; direct launches (profiling, or
+    // graphs off) one step at a time.  Before each launch the host looks at the
+    // overflow words the last finished sequence published.  The call's first
+    // step clears the status word, by a kernel of its own before the first of
+    // several sequences (which are the same graph), else in its scan.
+    const int rest = nsteps % c->seq_steps;
+    const bool several = nsteps > c->seq_steps;
+    if (graph) check_plan(c);
+    const bool rest_seq = graph && rest_as_sequence(c, rest, !several);
+    if (graph && several) sphe_launch_clear_status(c->D, c->stream);
+    bool first = !(graph && several);
     for (int done = 0; done < nsteps;) {
         hipEvent_t& ev = c->seq_ev[c->seq_count % kInFlight];
         if (c->seq_count >= (uint64_t)kInFlight) HIPCHK(c, hipEventSynchronize(ev));
         r = grow_lists(c);
         if (r) return r;
-        const int k = graph && nsteps - done >= c->seq_steps ? c->seq_steps : 1;
-        if (graph) {
+        const int left = nsteps - done;
+        const int k = graph && left >= c->seq_steps ? c->seq_steps : (rest_seq && left == rest ? rest : 0);
+        if (k > 0) {
+            check_plan(c);
             hipGraphExec_t x = nullptr;
-            r = ensure_graph(c, k, &x);
+            r = ensure_graph(c, k, first, &x);
             if (r) return r;
             HIPCHK(c, hipGraphLaunch(x, c->stream));
         } else {
-            launch_step(c);
-            sphe_launch_publish(c->D, c->h_ovf_dev, c->stream);
+            launch_step(c, first);
         }
+        first = false;
         HIPCHK(c, hipGetLastError());
         HIPCHK(c, hipEventRecord(ev, c->stream));
         ++c->seq_count;
-        done += k;
+        done += k > 0 ? k : 1;
         if (any_erosion(c, -1)) c->heights_stale = true;
         c->stepped = true;
     }
@@ -1128,7 +1163,7 @@ int sort_current(sphe_ctx* c)
         r = recount(c);
         if (r) return r;
     }
-    launch_sort(c);
+    launch_sort(c, false);
     sphe_launch_density(c->D, c->block, c->remap, c->lanes, c->stream);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipStreamSynchronize(c->stream));
