@@ -2371,11 +2371,14 @@ __global__ __launch_bounds__(256) void k_tapply(DevState D)
 // sums of that step (same lane split and merge as k_force) from the retained
 // sorted state, and reads the state the step left in the same slot.  The
 // slot comes from device memory (the id map or the id search; INT32_MAX or
-// out of range: no such particle, out[22] = -1).
+// out of range: no such particle, out[22] = -1).  lists: the neighbour lists
+// still hold the step's (else the stencil is walked: 22 us against 5.5 for 30
+// neighbours, a chain of dependent loads either way).  One wave; out may be
+// mapped host memory.
 template <typename T, int SM, int G>
-__global__ void k_inspect(DevState D, const int32_t* __restrict__ slotp, double* out)
+__global__ __launch_bounds__(64) void k_inspect(DevState D, const int32_t* __restrict__ slotp, int lists, double* out)
 {
-    if (blockIdx.x != 0 || threadIdx.x >= G) return;
+    if (blockIdx.x != 0) return;
     const int32_t s32 = *slotp;
     if (s32 < 0 || (int64_t)s32 >= D.P) {  // the same in every lane
         if (threadIdx.x == 0) out[22] = -1.0;
@@ -2390,15 +2393,35 @@ __global__ void k_inspect(DevState D, const int32_t* __restrict__ slotp, double*
     const T rho_i = ((const T*)D.rho)[slot];
     const T a_i = ((const V4<T>*)D.posa)[slot].w;
     ForceAcc<T, SM> acc;
-    if (l == 0) acc.self_term(K, vi.w);
     int32_t nbmax = -1, count = 0;
-    force_share_walk<T, SM, G>(D, S, K, slot, l, pi, vi, a_i, acc, nbmax, count);
-    acc.template merge<G>();
+    const uint32_t cnt = D.nbc[slot], cap = (uint32_t)D.maxn;
+    const bool listed =
+        lists && (cnt <= cap || (cnt - cap <= (uint32_t)D.ocap && D.pbase[slot] != ~0u));  // the same in every lane
+    if (listed) {
+        // the largest neighbour id by the whole wave
+        const uint32_t* more = cnt > cap ? D.pool + (size_t)D.pbase[slot] * SPHE_POOL_UNIT : nullptr;
+        for (uint32_t e = (uint32_t)l; e < cnt; e += SPHE_WAVE) {
+            const uint32_t c = e & ~15u, word = (e % G) * (16 / G) + (e & 15u) / G;
+            const uint32_t* q = c < cap ? D.nbl + (size_t)slot * cap + c : more + (c - cap);
+            nbmax = max(nbmax, D.s_id[q[word] / (uint32_t)sizeof(V4<T>)]);
+        }
 #pragma unroll
-    for (int m = 1; m < G; m <<= 1) {
-        nbmax = max(nbmax, __shfl_xor(nbmax, m, SPHE_WAVE));
-        count += __shfl_xor(count, m, SPHE_WAVE);
+        for (int m = 1; m < SPHE_WAVE; m <<= 1) nbmax = max(nbmax, __shfl_xor(nbmax, m, SPHE_WAVE));
+        count = (int32_t)cnt + 1;
     }
+    if (l >= G) return;
+    if (l == 0) acc.self_term(K, vi.w);
+    if (listed) {
+        force_share<false, T, SM, G>(D, S, K, (uint32_t)slot, (uint32_t)slot, l, pi, vi, a_i, acc, false);
+    } else {
+        force_share_walk<T, SM, G>(D, S, K, slot, l, pi, vi, a_i, acc, nbmax, count);
+#pragma unroll
+        for (int m = 1; m < G; m <<= 1) {
+            nbmax = max(nbmax, __shfl_xor(nbmax, m, SPHE_WAVE));
+            count += __shfl_xor(count, m, SPHE_WAVE);
+        }
+    }
+    acc.template merge<G>();
     if (l != 0) return;
     ForceOut<T> o;
     acc.finish(K, rho_i, o);
@@ -2429,16 +2452,20 @@ __global__ __launch_bounds__(256) void k_fill_i32(int32_t* __restrict__ p, int64
     if (i < n) p[i] = v;
 }
 
-// id -> sorted slot of the last step, for the scenes with a map (cleared to
-// INT32_MAX first; duplicate ids keep their lowest slot).
+// id -> slot of the current state, for the scenes with a map.  UNIQUE: every
+// entry of the map belongs to one particle; otherwise the map was cleared to
+// INT32_MAX first, and duplicate ids keep their lowest slot.
+template <bool UNIQUE>
 __global__ __launch_bounds__(256) void k_idmap(DevState D, int32_t* __restrict__ map)
 {
     const int64_t slot = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (slot >= D.P) return;
     const SceneDev& S = D.scenes[wave_scene(D.chunk_scene, slot)];
     if (slot >= S.p_begin + S.n || S.idmap_off < 0) return;
-    const int32_t id = D.s_id[slot];
-    if (id >= 0 && id < S.idmap_len) atomicMin(&map[S.idmap_off + id], (int32_t)slot);
+    const int32_t id = D.u_id[slot];
+    if (id < 0 || id >= S.idmap_len) return;
+    if constexpr (UNIQUE) map[S.idmap_off + id] = (int32_t)slot;
+    else atomicMin(&map[S.idmap_off + id], (int32_t)slot);
 }
 
 // Positions (what 0), velocities (1) or the last step's densities (2) of the
@@ -2462,6 +2489,24 @@ __global__ __launch_bounds__(256) void k_feed(DevState D, int64_t p0, int64_t n,
     o[0] = (float)v.x;
     o[1] = (float)v.y;
     o[2] = (float)v.z;
+}
+
+// The same values by the id map, for out in mapped host memory: one thread per
+// value, so that every wave writes 256 consecutive bytes over the link (k_feed
+// would send each value by itself).  1,000 positions 3.7 us, 13,824 5.1; with
+// the map built by the first reader after a step (2.4 and 3.1), k_feed and the
+// runtime's copy to pageable memory took some 17 us more for each read.
+template <typename T>
+__global__ __launch_bounds__(256) void k_gather(DevState D, const int32_t* __restrict__ map, int64_t n, int what,
+                                                float* __restrict__ out)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const uint32_t p = what == 2 ? (uint32_t)i : (uint32_t)i / 3u;
+    const int32_t slot = map[p];
+    if (slot < 0 || (int64_t)slot >= D.P) return;
+    out[i] = (float)(what == 2 ? ((const T*)D.rho)[slot]
+                               : ((const T*)(what ? D.u_vel : D.u_pos))[4 * (int64_t)slot + ((uint32_t)i - 3u * p)]);
 }
 
 // The sorted slot of particle `id` of one scene without a map (lowest slot
@@ -2960,27 +3005,32 @@ void sphe_launch_terrain_mesh(const float* H, int nx, int nz, float cell, float 
 }
 
 template <int G>
-static void launch_inspect_g(const DevState& D, const int32_t* slotp, double* out, hipStream_t st)
+static void launch_inspect_g(const DevState& D, const int32_t* slotp, bool lists, double* out, hipStream_t st)
 {
-#define CALL(T, SM) k_inspect<T, SM, G><<<1, 64, 0, st>>>(D, slotp, out)
+#define CALL(T, SM) k_inspect<T, SM, G><<<1, 64, 0, st>>>(D, slotp, lists, out)
     SPHE_PREC_SWITCH(D.precision, CALL);
 #undef CALL
 }
 
-void sphe_launch_inspect(const DevState& D, const int32_t* slotp, int lanes, double* out, hipStream_t st)
+void sphe_launch_inspect(const DevState& D, const int32_t* slotp, int lanes, bool lists, double* out, hipStream_t st)
 {
     switch (lanes) {
-    case 1: launch_inspect_g<1>(D, slotp, out, st); break;
-    case 2: launch_inspect_g<2>(D, slotp, out, st); break;
-    case 8: launch_inspect_g<8>(D, slotp, out, st); break;
-    default: launch_inspect_g<4>(D, slotp, out, st); break;
+    case 1: launch_inspect_g<1>(D, slotp, lists, out, st); break;
+    case 2: launch_inspect_g<2>(D, slotp, lists, out, st); break;
+    case 8: launch_inspect_g<8>(D, slotp, lists, out, st); break;
+    default: launch_inspect_g<4>(D, slotp, lists, out, st); break;
     }
 }
 
-void sphe_launch_idmap(const DevState& D, int32_t* map, int64_t len, hipStream_t st)
+void sphe_launch_idmap(const DevState& D, int32_t* map, int64_t len, bool unique, hipStream_t st)
 {
-    if (len > 0) k_fill_i32<<<grid_of(len, 256), 256, 0, st>>>(map, len, INT32_MAX);
-    if (D.P > 0 && len > 0) k_idmap<<<grid_of(D.P, 256), 256, 0, st>>>(D, map);
+    if (D.P == 0 || len == 0) return;
+    if (unique) {
+        k_idmap<true><<<grid_of(D.P, 256), 256, 0, st>>>(D, map);
+    } else {
+        k_fill_i32<<<grid_of(len, 256), 256, 0, st>>>(map, len, INT32_MAX);
+        k_idmap<false><<<grid_of(D.P, 256), 256, 0, st>>>(D, map);
+    }
 }
 
 void sphe_launch_feed(const DevState& D, int64_t p0, int64_t n, int what, float* out, hipStream_t st)
@@ -2988,6 +3038,13 @@ void sphe_launch_feed(const DevState& D, int64_t p0, int64_t n, int what, float*
     if (n <= 0) return;
     if (D.precision == 2) k_feed<double><<<grid_of(n, 256), 256, 0, st>>>(D, p0, n, what, out);
     else k_feed<float><<<grid_of(n, 256), 256, 0, st>>>(D, p0, n, what, out);
+}
+
+void sphe_launch_gather(const DevState& D, const int32_t* map, int64_t n, int what, float* out, hipStream_t st)
+{
+    if (n <= 0) return;
+    if (D.precision == 2) k_gather<double><<<grid_of(n, 256), 256, 0, st>>>(D, map, n, what, out);
+    else k_gather<float><<<grid_of(n, 256), 256, 0, st>>>(D, map, n, what, out);
 }
 
 void sphe_launch_find_id(const DevState& D, int scene, int32_t id, int32_t* slot_out, hipStream_t st)

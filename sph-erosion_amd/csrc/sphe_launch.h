@@ -30,14 +30,19 @@ void sphe_launch_clear_status(const DevState& D, hipStream_t st);
 void sphe_launch_terrain_mesh(const float* H, int nx, int nz, float cell, float ox, float oz, float* out,
                               hipStream_t st);
 // The 112-byte record's values of the particle at sorted slot *slotp (device
-// memory) into out[0 .. 28]; out[22] = -1 when *slotp names no slot.
-void sphe_launch_inspect(const DevState& D, const int32_t* slotp, int lanes, double* out, hipStream_t st);
-// id -> sorted slot map of the last step for the scenes that have one.
-void sphe_launch_idmap(const DevState& D, int32_t* map, int64_t len, hipStream_t st);
+// memory) into out[0 .. 28]; out[22] = -1 when *slotp names no slot.  lists:
+// the neighbour lists are still the last step's.
+void sphe_launch_inspect(const DevState& D, const int32_t* slotp, int lanes, bool lists, double* out, hipStream_t st);
+// id -> slot map of the current state for the scenes that have one; unique:
+// every entry belongs to exactly one particle.
+void sphe_launch_idmap(const DevState& D, int32_t* map, int64_t len, bool unique, hipStream_t st);
 // Positions (what 0) or velocities (1) of the n particles at slots p0 ..
 // p0+n-1, whose ids are 0 .. n-1, as 3 floats at out[3 id]; their last
 // densities (2) as one float at out[id].
 void sphe_launch_feed(const DevState& D, int64_t p0, int64_t n, int what, float* out, hipStream_t st);
+// The same n floats (what 0, 1: 3 per particle) by a scene's part of the id
+// map, written in order: out may be mapped host memory.
+void sphe_launch_gather(const DevState& D, const int32_t* map, int64_t n, int what, float* out, hipStream_t st);
 // Sorted slot of one particle id of a scene by a search over its slots.
 void sphe_launch_find_id(const DevState& D, int scene, int32_t id, int32_t* slot_out, hipStream_t st);
 void sphe_launch_accel(const DevState& D, int scene, int lanes, double* out, hipStream_t st);

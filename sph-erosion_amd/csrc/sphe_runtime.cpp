@@ -54,6 +54,8 @@ struct Scene {
     bool ids_dense = false;                 // the ids are 0 .. n-1 (the device gathers in id order)
 };
 
+const size_t kStageBytes = 256 * 1024;
+
 struct ProfRec {
     std::string name;
     hipEvent_t a, b;
@@ -100,6 +102,10 @@ struct sphe_ctx {
     // end of every sequence and read by the host without a stream wait
     uint32_t* h_ovf = nullptr;
     uint32_t* h_ovf_dev = nullptr;
+    // what small reads come back through (kStageBytes after the words above):
+    // kernels write it, the host copies from it once the stream is done
+    char* h_stage = nullptr;
+    char* h_stage_dev = nullptr;
     // completion of the last launches (one event per launch slot): before a
     // launch the host waits for the one kInFlight launches back, so the
     // overflow word it reads is at most that many launches old
@@ -136,12 +142,13 @@ struct sphe_ctx {
     // address of its copy), for sphe_mass_all_noalloc; null if the lookup failed
     double* noalloc_scratch = nullptr;
     size_t noalloc_doubles = 0;
-    double* d_inspect = nullptr;
-    // id -> sorted slot map of the last step (sphe_get_particle), rebuilt on
-    // the first inspection after a step; d_slot: the slot of a searched id
+    // id -> slot map of the current state (sphe_get_particle, small reads),
+    // rebuilt by the first of them after a step; d_slot: the slot of a searched id
     int32_t* d_idmap = nullptr;
     int64_t idmap_len = 0;
     bool idmap_valid = false;
+    bool idmap_unique = false;  // every entry belongs to one particle (ids 0 .. n-1 in every mapped scene)
+    bool lists_valid = false;   // the neighbour lists are the last step's
     int32_t* d_slot = nullptr;
     // lane count and slab count the last step ran with: its inspection
     // repeats its sums in the same order whatever was set since
@@ -492,6 +499,7 @@ int build_layout(sphe_ctx* c)
     // are dense enough (max id below 2 n + 4096; ids are sorted ascending in
     // the staging arrays); the others are searched on inspection
     int64_t M = 0;
+    c->idmap_unique = true;
     for (Scene& s : c->scenes) {
         s.idmap_off = -1;
         s.idmap_len = 0;
@@ -502,6 +510,7 @@ int build_layout(sphe_ctx* c)
         if (len > 2 * (int64_t)s.ids.size() + 4096 || M + len > INT32_MAX / 2) continue;
         s.idmap_off = M;
         s.idmap_len = len;
+        c->idmap_unique = c->idmap_unique && s.ids_dense;
         M += len;
     }
     // per-slot vectors are addressed with 32-bit byte offsets: each stays under
@@ -569,7 +578,6 @@ int build_layout(sphe_ctx* c)
     D.persistent = c->persistent ? 1 : 0;
     DALLOC(c->d_mass_part, (size_t)sphe_mass_blocks() * 3 * 8);
     DALLOC(c->d_mass_out, 64);
-    DALLOC(c->d_inspect, 64 * 8);
     DALLOC(c->d_slot, 64);
     if (M > 0) DALLOC(c->d_idmap, (size_t)M * 4);
     c->idmap_len = M;
@@ -675,6 +683,7 @@ int upload(sphe_ctx* c)
     c->device_valid = true;
     c->counted = false;
     c->stepped = false;
+    c->idmap_valid = false;
     ++c->epoch;
     return SPHE_OK;
 }
@@ -1003,7 +1012,8 @@ int resize_lists(sphe_ctx* c, int maxn, int ocap, int64_t chunks)
     c->maxn = c->D.maxn;
     c->ocap = c->D.ocap;
     c->pool_chunks = (c->D.pool_cap - c->D.pool_origin) / c->D.ocap;
-    ++c->epoch;  // the new lists hold nothing yet
+    c->lists_valid = false;  // the new lists hold nothing yet
+    ++c->epoch;
     return SPHE_OK;
 }
 
@@ -1124,10 +1134,11 @@ int do_steps(sphe_ctx* c, int nsteps)
         done += k > 0 ? k : 1;
         if (any_erosion(c, -1)) c->heights_stale = true;
         c->stepped = true;
+        c->lists_valid = true;
+        c->step_lanes = c->lanes;
+        c->step_sub_log2 = c->D.sub_log2;
+        c->idmap_valid = false;
     }
-    c->step_lanes = c->lanes;
-    c->step_sub_log2 = c->D.sub_log2;
-    c->idmap_valid = false;
     c->host_valid = false;
     ++c->epoch;
     return SPHE_OK;
@@ -1169,7 +1180,6 @@ int sort_current(sphe_ctx* c)
     HIPCHK(c, hipStreamSynchronize(c->stream));
     c->counted = false;
     c->stepped = false;
-    c->idmap_valid = false;
     c->sorted_epoch = c->epoch;
     // the sorted buffers now hold the current state; keep the unsorted
     // state authoritative for the next step (its counts were consumed)
@@ -1269,7 +1279,7 @@ int sphe_create(int precision, sphe_ctx** out)
         return SPHE_EHIP;
     }
     void* h = nullptr;
-    if (hipHostMalloc(&h, 64, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
+    if (hipHostMalloc(&h, 256 + kStageBytes, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
         hipHostGetDevicePointer((void**)&c->h_ovf_dev, h, 0) != hipSuccess) {
         (void)hipGetLastError();
         if (h) (void)hipHostFree(h);
@@ -1278,6 +1288,8 @@ int sphe_create(int precision, sphe_ctx** out)
         return SPHE_EHIP;
     }
     c->h_ovf = (uint32_t*)h;
+    c->h_stage = (char*)h + 256;
+    c->h_stage_dev = (char*)c->h_ovf_dev + 256;
     clear_published(c);  // pinned memory may come back holding an earlier owner's words
     for (hipEvent_t& e : c->seq_ev) {
         if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
@@ -1556,6 +1568,16 @@ static int feed_on_device(sphe_ctx* c, const Scene* s, int what, float** out)
     return SPHE_OK;
 }
 
+// The id map of the current state, for the first reader since it changed.
+static int ensure_idmap(sphe_ctx* c)
+{
+    if (c->idmap_valid) return SPHE_OK;
+    sphe_launch_idmap(c->D, c->d_idmap, c->idmap_len, c->idmap_unique, c->stream);
+    HIPCHK(c, hipGetLastError());
+    c->idmap_valid = true;
+    return SPHE_OK;
+}
+
 int sphe_read_buffer(sphe_ctx* c, int scene, int which, void* out, size_t bytes)
 {
     SCENE_OR_FAIL(s, c, scene);
@@ -1569,11 +1591,24 @@ int sphe_read_buffer(sphe_ctx* c, int scene, int which, void* out, size_t bytes)
     if (n > 0 && s->ids_dense && c->device_valid && ((state && !c->host_valid) || (rho && c->stepped))) {
         // the device holds the values: gather this scene alone in id order
         // and copy 4 bytes per value, with no host sync of the rest
-        float* d = nullptr;
-        int r = feed_on_device(c, s, which == SPHE_BUF_POS ? FEED_POS : (state ? FEED_VEL : FEED_RHO), &d);
-        if (r) return r;
-        HIPCHK(c, hipMemcpyAsync(out, d, n * comps * 4, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
+        const int what = which == SPHE_BUF_POS ? FEED_POS : (state ? FEED_VEL : FEED_RHO);
+        const size_t nbytes = n * comps * 4;
+        if (nbytes <= kStageBytes && s->idmap_off >= 0) {
+            int r = ensure_device(c);
+            if (!r) r = ensure_idmap(c);
+            if (r) return r;
+            sphe_launch_gather(c->D, c->d_idmap + s->idmap_off, (int64_t)(n * comps), what, (float*)c->h_stage_dev,
+                               c->stream);
+            HIPCHK(c, hipGetLastError());
+            HIPCHK(c, hipStreamSynchronize(c->stream));
+            std::memcpy(out, c->h_stage, nbytes);
+        } else {
+            float* d = nullptr;
+            int r = feed_on_device(c, s, what, &d);
+            if (r) return r;
+            HIPCHK(c, hipMemcpyAsync(out, d, nbytes, hipMemcpyDeviceToHost, c->stream));
+            HIPCHK(c, hipStreamSynchronize(c->stream));
+        }
         if (which == SPHE_BUF_PRESS)
             for (size_t i = 0; i < n; ++i) f[i] = s->prm.stiffness * (f[i] - s->prm.rest_density);
         return SPHE_OK;
@@ -1674,15 +1709,12 @@ int sphe_get_particle(sphe_ctx* c, int scene, int id, sphe_particle* out)
     }
     if (id < 0) return fail(c, SPHE_ERANGE, "no particle with id %d", id);
     // the slot of the id in the last step's sorted buffers: from the id map
-    // (rebuilt once per step, on the first inspection) or by a search
+    // (rebuilt once per step, by its first reader) or by a search
     const int32_t* slotp = nullptr;
     if (s->idmap_off >= 0) {
         if (id >= s->idmap_len) return fail(c, SPHE_ERANGE, "no particle with id %d", id);
-        if (!c->idmap_valid) {
-            sphe_launch_idmap(c->D, c->d_idmap, c->idmap_len, c->stream);
-            HIPCHK(c, hipGetLastError());
-            c->idmap_valid = true;
-        }
+        int r = ensure_idmap(c);
+        if (r) return r;
         slotp = c->d_idmap + s->idmap_off + id;
     } else {
         sphe_launch_find_id(c->D, scene, id, c->d_slot, c->stream);
@@ -1692,11 +1724,11 @@ int sphe_get_particle(sphe_ctx* c, int scene, int id, sphe_particle* out)
     // the sums in the order the step took them
     DevState D = c->D;
     D.sub_log2 = c->step_sub_log2;
-    sphe_launch_inspect(D, slotp, c->step_lanes, c->d_inspect, c->stream);
+    sphe_launch_inspect(D, slotp, c->step_lanes, c->lists_valid, (double*)c->h_stage_dev, c->stream);
     HIPCHK(c, hipGetLastError());
-    double v[29];
-    HIPCHK(c, hipMemcpyAsync(v, c->d_inspect, sizeof(v), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
+    double v[29];
+    std::memcpy(v, c->h_stage, sizeof(v));
     if (v[22] < 0.0) return fail(c, SPHE_ERANGE, "no particle with id %d", id);
     for (int a = 0; a < 3; ++a) {
         out->Position[a] = (float)v[23 + a];

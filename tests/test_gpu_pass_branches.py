@@ -117,3 +117,65 @@ def test_scan_forms_give_the_same_steps(tiles):
     got = ctx.state_f64(sid)
     assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
     assert ctx.status() == 0
+
+
+@pytest.mark.parametrize("lanes", [1, 2, 4, 8])
+@pytest.mark.parametrize("precision", [sphe.FP32, sphe.FP32_NAIVE, sphe.FP64])
+def test_inspection_by_list_equals_by_walk(lanes, precision):
+    """A record from the neighbour list (in its 32 entries, in the overflow
+    chunk, past both) is the stencil walk's bit for bit; new lists, which hold
+    nothing until the next step, are not read."""
+    rng = np.random.default_rng(3)
+    pos = rng.normal(0.0, 0.035, (1500, 3)).astype(np.float32)
+    recs = []
+    for renewed in (False, True):
+        ctx = sphe.Context(precision)
+        ctx.set_lanes(lanes)
+        sid = ctx.add_scene(_params(0.0457, 0.5))
+        ctx.set_particles(sid, pos)
+        ctx.set_list_capacity(32)
+        counts = ctx.debug_neighbours(sid, csr=False)[0] - 1
+        assert (counts <= 32).any() and ((counts > 32) & (counts <= 64)).any() and (counts > 64).any()
+        ctx.step(1)
+        if renewed:
+            ctx.set_list_capacity(1024)
+        ids = np.concatenate([np.argsort(counts)[[0, 1, -2, -1]], np.flatnonzero(counts == 32)[:3],
+                              np.flatnonzero((counts > 32) & (counts <= 64))[::40], np.arange(0, 1500, 250)])
+        recs.append([bytes(ctx.particle(sid, int(i))) for i in ids])
+    assert recs[0] == recs[1]
+
+
+@pytest.mark.parametrize("precision", [sphe.FP32, sphe.FP64])
+def test_small_and_large_reads(precision):
+    """Positions, velocities and densities of scenes whose values fit the
+    staging buffer (read by the id map) and do not (gathered in device memory),
+    beside a scene of sparse ids, after steps, edits and the hooks that sort
+    again: the state's own values in id order."""
+    rng = np.random.default_rng(8)
+    ctx = sphe.Context(precision)
+    ids = [None, None, np.arange(700, dtype=np.int32) * 3 + 5, None, None]
+    sids = []
+    for n, i in zip((1, 1000, 700, 21845, 21846), ids):  # 21,845 positions: 4 bytes below the buffer's size
+        pos = rng.uniform(-0.3, 0.3, (n, 3)).astype(np.float32)
+        sids.append(ctx.add_scene(_params(0.0457, 0.4)))
+        ctx.set_particles(sids[-1], pos, ids=i)
+
+    def check():
+        got = [(ctx.positions(s), ctx.velocities(s), ctx.density(s)) for s in sids]
+        for s, (pos, vel, rho) in zip(sids, got):
+            gp, gv = ctx.state_f64(s)
+            assert np.array_equal(pos, gp.astype(np.float32)) and np.array_equal(vel, gv.astype(np.float32))
+            if len(rho) in (1, 1000):
+                assert rho[-1] == ctx.particle(s, len(rho) - 1).Density and rho[0] == ctx.particle(s, 0).Density
+    for steps in (1, 2):
+        ctx.step(steps)
+        check()
+        ctx.step(1)
+        ctx.debug_density(sids[1])  # sorts the state again, in other slots than its own
+        for s in sids:
+            pos, vel = ctx.positions(s), ctx.velocities(s)
+            gp, gv = ctx.state_f64(s)
+            assert np.array_equal(pos, gp.astype(np.float32)) and np.array_equal(vel, gv.astype(np.float32))
+    ctx.set_particles(sids[1], ctx.positions(sids[1])[::-1].copy())
+    ctx.step(1)
+    check()
