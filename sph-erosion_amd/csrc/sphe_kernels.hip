@@ -78,9 +78,27 @@ __device__ __forceinline__ uint32_t wave_index(int b)
     return (uint32_t)b * (blockDim.x / SPHE_WAVE) + __builtin_amdgcn_readfirstlane(threadIdx.x / SPHE_WAVE);
 }
 
+// A table that no kernel writes, in the constant address space: what a wave
+// reads there at a uniform address it reads with scalar loads.  From a plain
+// pointer the compiler takes vector loads instead wherever a store or an atomic
+// may have come before, one latency after the other, each wait including the
+// stores (20 in a row at the end of the force pass: 104 -> 84 us for 96 small
+// scenes, 62 -> 56 for 262,144 particles, 1,280 -> 1,232 for 4.2M).
+template <typename V>
+__device__ __forceinline__ const V* constant_table(const V* p)
+{
+    return (const V*)(const __attribute__((address_space(4))) V*)(uint64_t)p;
+}
+
+// The scene of the wave's slots (each of them lies in the same 64).
 __device__ __forceinline__ int wave_scene(const int32_t* chunk_scene, int64_t slot)
 {
-    return __builtin_amdgcn_readfirstlane(chunk_scene[slot >> 6]);
+    return constant_table(chunk_scene)[__builtin_amdgcn_readfirstlane((int32_t)(slot >> 6))];
+}
+
+__device__ __forceinline__ const SceneDev& scene_ref(const DevState& D, int scene)
+{
+    return constant_table(D.scenes)[scene];
 }
 
 // Element j of a per-slot array, addressed by a 32-bit byte offset from the
@@ -436,10 +454,10 @@ __device__ __forceinline__ void visit_neighbours(const DevState& D, const SceneD
 }
 
 // Counting-sort key of a position: the cell key shifted left by sub_log2,
-// or-ed with the x slab; the cell's count is taken with an atomic.
+// or-ed with the x slab.
 template <typename T>
-__device__ __forceinline__ void count_position(const DevState& D, const SceneDev& S, const SceneConsts<T>& K,
-                                               int64_t slot, T x, T y, T z)
+__device__ __forceinline__ int32_t position_key(const DevState& D, const SceneDev& S, const SceneConsts<T>& K, T x, T y,
+                                                T z)
 {
     const T gx = (x - K.org[0]) * K.inv_cell;
     const int kx = cidx<T>(d_floor(gx), S.dims[0] - 1);
@@ -447,9 +465,24 @@ __device__ __forceinline__ void count_position(const DevState& D, const SceneDev
     const int kz = cidx<T>(d_floor((z - K.org[2]) * K.inv_yz), S.dims[2] - 1);
     const int64_t key = S.cell_off + ((int64_t)kz * S.dims[1] + ky) * S.dims[0] + kx;
     const int sub = sub_cell<T>(gx, kx, S.dims[0], D.sub_log2);
-    D.key[slot] = (int32_t)((key << D.sub_log2) | sub);
-    D.arank[slot] = atomicAdd(&D.cnt[key], 1u);
-    D.tocc[key >> D.scan_log2] = 1u;
+    return (int32_t)((key << D.sub_log2) | sub);
+}
+
+// Counts a particle of that key into its cell: its rank of arrival.
+__device__ __forceinline__ uint32_t count_key(const DevState& D, int32_t key)
+{
+    const int32_t cell = key >> D.sub_log2;
+    D.tocc[cell >> D.scan_log2] = 1u;
+    return atomicAdd(&D.cnt[cell], 1u);
+}
+
+template <typename T>
+__device__ __forceinline__ void count_position(const DevState& D, const SceneDev& S, const SceneConsts<T>& K,
+                                               int64_t slot, T x, T y, T z)
+{
+    const int32_t key = position_key<T>(D, S, K, x, y, z);
+    D.key[slot] = key;
+    D.arank[slot] = count_key(D, key);
 }
 
 __device__ __forceinline__ void count_pad(const DevState& D, const SceneDev& S, int64_t slot)
@@ -467,7 +500,7 @@ __global__ __launch_bounds__(256) void k_hash_count(DevState D)
 {
     const int64_t slot = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (slot >= D.P) return;
-    const SceneDev& S = D.scenes[wave_scene(D.chunk_scene, slot)];
+    const SceneDev& S = scene_ref(D, wave_scene(D.chunk_scene, slot));
     if (slot < S.p_begin + S.n) {
         const SceneConsts<T>& K = SceneSel<T>::get(S);
         const V4<T> p = ((const V4<T>*)D.u_pos)[slot];
@@ -1004,7 +1037,7 @@ __device__ __forceinline__ void density_body(const DevState& D, int b)
     const int64_t slot = gt / G;
     const int l = (int)(gt & (G - 1));
     if (slot >= D.P) return;
-    const SceneDev& S = D.scenes[wave_scene(D.chunk_scene, slot)];
+    const SceneDev& S = scene_ref(D, wave_scene(D.chunk_scene, slot));
     if (slot >= S.p_begin + S.n) return;  // whole groups leave together
     const SceneConsts<T>& K = SceneSel<T>::get(S);
     const V4<T>* __restrict__ pos = (const V4<T>*)D.s_pos;
@@ -1323,7 +1356,7 @@ __device__ __forceinline__ void density_quad(const DevState& D, int b)
     const uint32_t wslot = wave_index(b) * 16u;
     if (wslot >= (uint64_t)D.P) return;
     const uint32_t slot = wslot + (uint32_t)(lane >> 2);
-    const SceneDev& S = D.scenes[wave_scene(D.chunk_scene, wslot)];
+    const SceneDev& S = scene_ref(D, wave_scene(D.chunk_scene, wslot));
     const uint32_t lo = (uint32_t)S.p_begin, hi = (uint32_t)(S.p_begin + S.n);
     if (wslot >= hi) return;  // only padding
     const SceneConsts<T>& K = SceneSel<T>::get(S);
@@ -1954,8 +1987,8 @@ __device__ __forceinline__ int64_t erode_exchange(const SceneDev& S, const Scene
 // (a + b) + (c + d) before they enter the lane's sums; then one pair, then a
 // single.
 //
-// No unit is saturated: on a settled 4.2M-particle layer (1,437 us before, 1,320
-// now) the gathers' line accesses take 55% of the L1's cycles, the VALU is
+// No unit is saturated: on a settled 4.2M-particle layer (1,437 us with the list
+// laid out entry by entry, 1,230 now) the gathers' line accesses take 55% of the L1's cycles, the VALU is
 // busy for half the time, the lists come from HBM, and 20 waves a CU wait for
 // each other.  So waves in flight count most: five a SIMD, 96 registers, with
 // nothing spilled on the way through the loop.  What lies behind that:
@@ -1972,7 +2005,7 @@ __device__ __forceinline__ int64_t erode_exchange(const SceneDev& S, const Scene
 // seven, a pair ahead with four waves, and lists two iterations ahead.
 template <bool UNIT, typename T, int SM, int G, typename F>
 __device__ __forceinline__ void force_list(const DevState& D, const SceneConsts<T>& K, uint32_t mine, const V4<T>& pi,
-                                           const V4<T>& vi, T a_i, ForceAcc<T, SM>& acc, F&& fetch)
+                                           const V4<T>& vi, T a_i, ForceAcc<T, SM>& acc, uint4 n, F&& fetch)
 {
     if (mine == 0u) return;
     const V4<T>* __restrict__ posa = (const V4<T>*)D.posa;
@@ -1989,7 +2022,6 @@ __device__ __forceinline__ void force_list(const DevState& D, const SceneConsts<
     // computes: always, and after the gathers, whose waits then leave that load
     // in flight (memory operations complete in order; a load that may or may
     // not have been issued would have to be waited for).
-    uint4 n = fetch(mine > 4u);
     for (; mine >= 4u; mine -= 4u) {
         const Nb a = load(n.x), b = load(n.y), c = load(n.z), d = load(n.w);
         __builtin_amdgcn_sched_barrier(0);
@@ -2017,16 +2049,34 @@ __device__ __forceinline__ uint32_t opaque_tid()
     return t;
 }
 
+// The start of a particle's list, loaded ahead of what it depends on: the
+// number of entries and (four lanes a particle) the lane's first four, which
+// may be anything where there are fewer.
+struct ListHead {
+    uint32_t cnt;
+    uint4 first;
+};
+template <int G>
+__device__ __forceinline__ ListHead list_head(const DevState& D, uint32_t slot, uint32_t l)
+{
+    ListHead h;
+    h.cnt = D.nbc[slot];
+    h.first = make_uint4(0u, 0u, 0u, 0u);
+    if constexpr (G == 4) h.first = *(const uint4*)(D.nbl + (size_t)slot * (uint32_t)D.maxn + l * (16 / G));
+    return h;
+}
+
 // Lane l's share of the force sums of one particle: from its list, the
 // list continued in its overflow chunk, or (no room for all neighbours)
 // by walking the stencil.  wslot: the wave's first slot.
 template <bool UNIT, typename T, int SM, int G>
 __device__ __forceinline__ void force_share(const DevState& D, const SceneDev& S, const SceneConsts<T>& K,
-                                           uint32_t slot, uint32_t wslot, int l, const V4<T>& pi, const V4<T>& vi,
-                                           T a_i, ForceAcc<T, SM>& acc, bool report_walk)
+                                           const ListHead& head, uint32_t slot, uint32_t wslot, int l,
+                                           const V4<T>& pi, const V4<T>& vi, T a_i, ForceAcc<T, SM>& acc,
+                                           bool report_walk)
 {
     constexpr uint32_t PER = 16 / G;
-    const uint32_t cnt = D.nbc[slot];
+    const uint32_t cnt = head.cnt;
     const uint32_t cap = (uint32_t)D.maxn;
     if (cnt <= cap || (cnt - cap <= (uint32_t)D.ocap && D.pbase[slot] != ~0u)) {
         // the lane's entries l, l + G, ... are words l PER .. of each chunk of
@@ -2041,19 +2091,23 @@ __device__ __forceinline__ void force_share(const DevState& D, const SceneDev& S
         };
         uint32_t e = 0;
         if constexpr (G == 4) {
-            force_list<UNIT, T, SM, G>(D, K, mine, pi, vi, a_i, acc, [&](bool more) {
-                const uint4 n = *(const uint4*)list;
+            auto advance = [&](bool more) {
                 e += 16u;
                 if (__builtin_expect(e == cap, 0)) {
                     if (more) list = pool();
                 } else {
                     list += more ? 16 : 0;
                 }
+            };
+            advance(mine > 4u);
+            force_list<UNIT, T, SM, G>(D, K, mine, pi, vi, a_i, acc, head.first, [&](bool more) {
+                const uint4 n = *(const uint4*)list;
+                advance(more);
                 return n;
             });
         } else {
             auto chunk = [&](uint32_t c) { return c < cap ? list + c : pool() + (c - cap); };
-            force_list<UNIT, T, SM, G>(D, K, mine, pi, vi, a_i, acc, [&](bool more) {
+            auto fetch = [&](bool more) {
                 uint4 n;
                 if constexpr (G < 4) {
                     n = *(const uint4*)(chunk(e & ~15u) + (e & 15u) / G);
@@ -2065,7 +2119,8 @@ __device__ __forceinline__ void force_share(const DevState& D, const SceneDev& S
                 }
                 if (more) e += 4 * G;
                 return n;
-            });
+            };
+            if (mine != 0u) force_list<UNIT, T, SM, G>(D, K, mine, pi, vi, a_i, acc, fetch(mine > 4u), fetch);
         }
         return;
     }
@@ -2083,6 +2138,7 @@ __device__ __forceinline__ void force_share(const DevState& D, const SceneDev& S
 // reads them between step sequences without waiting for the stream.
 __device__ __forceinline__ void publish(const DevState& D)
 {
+    if (blockIdx.x != 0 || threadIdx.x != 0) return;
     const unsigned long long t = *D.ptop;
     volatile uint32_t* d = D.pub;
     d[0] = D.ovf[0];
@@ -2094,6 +2150,14 @@ __device__ __forceinline__ void publish(const DevState& D)
 // One G-lane group per particle: the lanes sum their shares, merge them
 // (xor shuffles), and lane 0 integrates, collides, erodes, stores the new
 // state and counts the particle's next cell.
+// Outside the list loop a wave does little but wait, so what can be loaded
+// together is: all that the slot alone addresses before the scene is looked up
+// (the scene's padding goes through as particles without neighbours: a branch
+// there would hold the loads back), the epilogue's inputs before the merge, and
+// the cell count, whose answer the wave's last store waits for, before the
+// other stores (batches of 48 uneven scenes: 203 -> 150 us in all, 262,144
+// particles 65.5 -> 56.5, 4.2M 1,337 -> 1,230, with constant_table and one-wave
+// blocks).
 template <bool UNIT, typename T, int SM, int G>
 __device__ __forceinline__ void force_body(const DevState& D, int b)
 {
@@ -2102,36 +2166,44 @@ __device__ __forceinline__ void force_body(const DevState& D, int b)
     // waves are whole)
     const uint32_t wslot = wave_index(b) * (uint32_t)(SPHE_WAVE / G);
     if (wslot >= (uint64_t)D.P) return;
-    if (b == 0 && threadIdx.x == 0) publish(D);  // no launch of its own (4 us)
     const uint32_t slot0 = wslot + (uint32_t)(threadIdx.x & (SPHE_WAVE - 1)) / G;
-    const SceneDev& S = D.scenes[wave_scene(D.chunk_scene, wslot)];
     V4<T>* __restrict__ upos = (V4<T>*)D.u_pos;
     V4<T>* __restrict__ uvel = (V4<T>*)D.u_vel;
     const V4<T>* __restrict__ spos = (const V4<T>*)D.s_pos;
     const V4<T>* __restrict__ svel = (const V4<T>*)D.s_vel;
-    if (slot0 >= (uint32_t)(S.p_begin + S.n)) {
-        if (l != 0) return;
-        // padding: carried through, counted into the scene's pad cell
-        upos[slot0] = spos[slot0];
-        uvel[slot0] = svel[slot0];
-        D.u_sed[slot0] = D.s_sed[slot0];
-        D.u_id[slot0] = D.s_id[slot0];
-        count_pad(D, S, slot0);
-        if (S.erosion == 2) D.tcell[slot0] = -1;
-        return;
-    }
-    const SceneConsts<T>& K = SceneSel<T>::get(S);
+    // all that is loaded by the slot, before the scene is known
+    ListHead head = list_head<G>(D, slot0, (uint32_t)l);
     const V4<T> pi = spos[slot0];
     const V4<T> vi = svel[slot0];
     const T a_i = ((const V4<T>*)D.posa)[slot0].w;
+    const SceneDev& S = scene_ref(D, wave_scene(D.chunk_scene, wslot));
+    const uint32_t end = (uint32_t)(S.p_begin + S.n);
+    if (slot0 >= end) head.cnt = 0u;  // padding: no neighbours
+    const SceneConsts<T>& K = SceneSel<T>::get(S);
     ForceAcc<T, SM> acc;
     if (l == 0) acc.self_term(K, vi.w);
-    force_share<UNIT, T, SM, G>(D, S, K, slot0, wslot, l, pi, vi, a_i, acc, true);
-    acc.template merge<G>();
+    force_share<UNIT, T, SM, G>(D, S, K, head, slot0, wslot, l, pi, vi, a_i, acc, true);
+    // what the epilogue needs, while the lanes' sums are merged
     const uint32_t tid = opaque_tid();
-    if ((tid & (G - 1)) != 0) return;
     const uint32_t slot = wslot + (tid & (SPHE_WAVE - 1)) / G;
     const T rho_i = ((const T*)D.rho)[slot];
+    int64_t sed = D.s_sed[slot];
+    const int32_t id = D.s_id[slot];
+    acc.template merge<G>();
+    if ((tid & (G - 1)) != 0) return;
+    if (slot >= end) {
+        // padding: carried through, counted into the scene's pad cell
+        upos[slot] = spos[slot];
+        uvel[slot] = svel[slot];
+        D.u_sed[slot] = sed;
+        D.u_id[slot] = id;
+        count_pad(D, S, slot);
+        if (S.erosion == 2) D.tcell[slot] = -1;
+        // kept apart from the end of the function, where the rank's wait would
+        // otherwise become one for every store
+        asm volatile("");
+        return;
+    }
     ForceOut<T> o;
     acc.finish(K, rho_i, o);
 
@@ -2143,7 +2215,6 @@ __device__ __forceinline__ void force_body(const DevState& D, int b)
         v[a] = vin[a] + o.acc[a] * K.dt;
         p[a] = xin[a] + v[a] * K.dt;
     }
-    int64_t sed = D.s_sed[slot];
     const bool moving = K.dt != T(0);
     if (moving) box_response<T>(K, p, v);
     int32_t tc = -1;
@@ -2156,6 +2227,10 @@ __device__ __forceinline__ void force_body(const DevState& D, int b)
             if (S.erosion) dq = erode_exchange<T>(S, K, p, hs, v, sed, &tc);
         }
     }
+    // the cell count of the new position for the next step's sort: its answer
+    // comes while the state is stored
+    const int32_t key = position_key<T>(D, S, K, p[0], p[1], p[2]);
+    const uint32_t rank = count_key(D, key);
     if (S.erosion == 1 && dq != 0) {
         sed += dq;
         atomicAdd((unsigned long long*)&D.vol[S.t_off + tc], (unsigned long long)(-dq));
@@ -2170,12 +2245,12 @@ __device__ __forceinline__ void force_body(const DevState& D, int b)
     upos[slot] = np;
     uvel[slot] = nv;
     D.u_sed[slot] = sed;
-    D.u_id[slot] = D.s_id[slot];
+    D.u_id[slot] = id;
     if (!(d_finite(p[0]) && d_finite(p[1]) && d_finite(p[2]) && d_finite(v[0]) && d_finite(v[1]) &&
           d_finite(v[2])))
         atomicOr(D.status, 1u);
-    // cell count of the new position for the next step's sort
-    count_position<T>(D, S, K, slot, p[0], p[1], p[2]);
+    D.key[slot] = key;
+    D.arank[slot] = rank;
 }
 
 // FP32: at most 96 registers (5 waves per SIMD): the list loop fits, and
@@ -2183,18 +2258,18 @@ __device__ __forceinline__ void force_body(const DevState& D, int b)
 // Unbounded, the walk raises the count and the occupancy of the whole
 // kernel drops to 4.
 template <int SM, int G, bool UNIT>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_force_f32(DevState D, int nblk,
-                                                                                              int remap)
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(5, 8))) void k_force_f32(DevState D)
 {
-    force_body<UNIT, float, SM, G>(D, xcd_block(blockIdx.x, nblk, remap));
+    force_body<UNIT, float, SM, G>(D, (int)blockIdx.x);
+    publish(D);
 }
 
 // FP64: at most 168 registers (3 waves per SIMD instead of 2 unbounded).
 template <int G>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_force_f64(DevState D, int nblk,
-                                                                                              int remap)
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(3, 8))) void k_force_f64(DevState D)
 {
-    force_body<false, double, SUM_PLAIN, G>(D, xcd_block(blockIdx.x, nblk, remap));
+    force_body<false, double, SUM_PLAIN, G>(D, (int)blockIdx.x);
+    publish(D);
 }
 
 // ------------------------------------------------------ persistent passes
@@ -2261,12 +2336,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(5, 8))) voi
     DevState D, int nblk, int chunk, uint32_t* work)
 {
     SPHE_PERSISTENT_LOOP((force_body<false, float, SM, G>(D, b)))
+    publish(D);
 }
 
 template <int G>
 __global__ __launch_bounds__(512) void k_force_f64_pers(DevState D, int nblk, int chunk, uint32_t* work)
 {
     SPHE_PERSISTENT_LOOP((force_body<false, double, SUM_PLAIN, G>(D, b)))
+    publish(D);
 }
 
 // --------------------------------------------------------------- terrain
@@ -2277,7 +2354,7 @@ __global__ __launch_bounds__(512) void k_force_f64_pers(DevState D, int nblk, in
 // padding and keep their value.
 __device__ __forceinline__ void heights_quad(const DevState& D, int64_t t0)
 {
-    const SceneDev& S = D.scenes[D.tchunk_scene[t0 >> 6]];
+    const SceneDev& S = D.scenes[D.tchunk_scene[t0 >> 6]];  // a wave's cells may belong to four scenes
     const int64_t end = S.t_off + (int64_t)S.tnx * S.tnz;
     const float y0 = S.t_y0, hq = S.hq;
     if (t0 + 4 <= end) {
@@ -2333,7 +2410,7 @@ __global__ __launch_bounds__(256) void k_tcount(DevState D)
 {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= D.P) return;
-    const SceneDev& S = D.scenes[wave_scene(D.chunk_scene, p)];
+    const SceneDev& S = scene_ref(D, wave_scene(D.chunk_scene, p));
     if (S.erosion != 2) return;
     const int32_t tc = D.tcell[p];
     if (tc >= 0) atomicAdd(&D.tcnt[tc], 1u);
@@ -2344,7 +2421,7 @@ __global__ __launch_bounds__(256) void k_tscatter(DevState D)
 {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= D.P) return;
-    const SceneDev& S = D.scenes[wave_scene(D.chunk_scene, p)];
+    const SceneDev& S = scene_ref(D, wave_scene(D.chunk_scene, p));
     if (S.erosion != 2) return;
     const int32_t tc = D.tcell[p];
     if (tc < 0) return;
@@ -2386,7 +2463,7 @@ __global__ __launch_bounds__(64) void k_inspect(DevState D, const int32_t* __res
     }
     const int64_t slot = s32;
     const int l = (int)threadIdx.x;
-    const SceneDev& S = D.scenes[D.chunk_scene[slot >> 6]];
+    const SceneDev& S = scene_ref(D, wave_scene(D.chunk_scene, slot));
     const SceneConsts<T>& K = SceneSel<T>::get(S);
     const V4<T> pi = ((const V4<T>*)D.s_pos)[slot];
     const V4<T> vi = ((const V4<T>*)D.s_vel)[slot];
@@ -2412,7 +2489,8 @@ __global__ __launch_bounds__(64) void k_inspect(DevState D, const int32_t* __res
     if (l >= G) return;
     if (l == 0) acc.self_term(K, vi.w);
     if (listed) {
-        force_share<false, T, SM, G>(D, S, K, (uint32_t)slot, (uint32_t)slot, l, pi, vi, a_i, acc, false);
+        force_share<false, T, SM, G>(D, S, K, list_head<G>(D, (uint32_t)slot, (uint32_t)l), (uint32_t)slot,
+                                     (uint32_t)slot, l, pi, vi, a_i, acc, false);
     } else {
         force_share_walk<T, SM, G>(D, S, K, slot, l, pi, vi, a_i, acc, nbmax, count);
 #pragma unroll
@@ -2460,7 +2538,7 @@ __global__ __launch_bounds__(256) void k_idmap(DevState D, int32_t* __restrict__
 {
     const int64_t slot = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (slot >= D.P) return;
-    const SceneDev& S = D.scenes[wave_scene(D.chunk_scene, slot)];
+    const SceneDev& S = scene_ref(D, wave_scene(D.chunk_scene, slot));
     if (slot >= S.p_begin + S.n || S.idmap_off < 0) return;
     const int32_t id = D.u_id[slot];
     if (id < 0 || id >= S.idmap_len) return;
@@ -2543,7 +2621,8 @@ __global__ __launch_bounds__(256) void k_accel(DevState D, int scene, double* __
     const T a_i = ((const V4<T>*)D.posa)[slot].w;
     ForceAcc<T, SM> acc;
     if (l == 0) acc.self_term(K, vi.w);
-    force_share<false, T, SM, G>(D, S, K, (uint32_t)slot, wave_index((int)blockIdx.x) * (uint32_t)(SPHE_WAVE / G), l, pi,
+    force_share<false, T, SM, G>(D, S, K, list_head<G>(D, (uint32_t)slot, (uint32_t)l), (uint32_t)slot,
+                                 wave_index((int)blockIdx.x) * (uint32_t)(SPHE_WAVE / G), l, pi,
                                   vi, a_i, acc, false);
     acc.template merge<G>();
     if (l != 0) return;
@@ -2931,26 +3010,25 @@ static void launch_density_g(const DevState& D, int block, int remap, hipStream_
 }
 
 template <int G>
-static void launch_force_g(const DevState& D, int block, int remap, hipStream_t st, hipEvent_t e0, hipEvent_t e1)
+static void launch_force_g(const DevState& D, int block, hipStream_t st, hipEvent_t e0, hipEvent_t e1)
 {
     const int nblk = (int)grid_of(D.P * G, block);
     if (D.persistent) {
         if (D.precision == 2) {
-            klaunch_pers(k_force_f64_pers<G>, nblk, block, 0, D, st, e0, e1, D, nblk, remap, D.work);
+            klaunch_pers(k_force_f64_pers<G>, nblk, block, 0, D, st, e0, e1, D, nblk, 1, D.work);
             return;
         }
-#define CALL(T, SM) klaunch_pers(k_force_f32_pers<SM, G>, nblk, block, 0, D, st, e0, e1, D, nblk, remap, D.work)
+#define CALL(T, SM) klaunch_pers(k_force_f32_pers<SM, G>, nblk, block, 0, D, st, e0, e1, D, nblk, 1, D.work)
         SPHE_PREC_SWITCH(D.precision, CALL);
 #undef CALL
         return;
     }
     if (D.precision == 2) {
-        klaunch(k_force_f64<G>, nblk, block, st, e0, e1, D, nblk, remap);
+        klaunch(k_force_f64<G>, nblk, block, st, e0, e1, D);
         return;
     }
     const bool unit = D.h_unit != 0;
-#define CALL(T, SM) \
-    klaunch(unit ? k_force_f32<SM, G, G == 4> : k_force_f32<SM, G, false>, nblk, block, st, e0, e1, D, nblk, remap)
+#define CALL(T, SM) klaunch(unit ? k_force_f32<SM, G, G == 4> : k_force_f32<SM, G, false>, nblk, block, st, e0, e1, D)
     SPHE_PREC_SWITCH(D.precision, CALL);
 #undef CALL
 }
@@ -2967,15 +3045,14 @@ void sphe_launch_density(const DevState& D, int block, int remap, int lanes, hip
     }
 }
 
-void sphe_launch_force(const DevState& D, int block, int remap, int lanes, hipStream_t st, hipEvent_t e0,
-                       hipEvent_t e1)
+void sphe_launch_force(const DevState& D, int block, int lanes, hipStream_t st, hipEvent_t e0, hipEvent_t e1)
 {
     if (D.P == 0) return;
     switch (lanes) {
-    case 1: launch_force_g<1>(D, block, remap, st, e0, e1); break;
-    case 2: launch_force_g<2>(D, block, remap, st, e0, e1); break;
-    case 8: launch_force_g<8>(D, block, remap, st, e0, e1); break;
-    default: launch_force_g<4>(D, block, remap, st, e0, e1); break;
+    case 1: launch_force_g<1>(D, block, st, e0, e1); break;
+    case 2: launch_force_g<2>(D, block, st, e0, e1); break;
+    case 8: launch_force_g<8>(D, block, st, e0, e1); break;
+    default: launch_force_g<4>(D, block, st, e0, e1); break;
     }
 }
 

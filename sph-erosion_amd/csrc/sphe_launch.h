@@ -22,8 +22,8 @@ void sphe_launch_scatter(const DevState& D, hipStream_t st, hipEvent_t e0 = null
 void sphe_launch_reorder(const DevState& D, hipStream_t st, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 void sphe_launch_density(const DevState& D, int block, int remap, int lanes, hipStream_t st,
                          hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
-void sphe_launch_force(const DevState& D, int block, int remap, int lanes, hipStream_t st,
-                       hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
+void sphe_launch_force(const DevState& D, int block, int lanes, hipStream_t st, hipEvent_t e0 = nullptr,
+                       hipEvent_t e1 = nullptr);
 void sphe_launch_heights(const DevState& D, hipStream_t st, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 void sphe_launch_two_phase(const DevState& D, hipStream_t st, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 void sphe_launch_clear_status(const DevState& D, hipStream_t st);

@@ -118,9 +118,9 @@ struct sphe_ctx {
     std::map<std::string, std::pair<double, int>> prof;
     std::map<std::pair<int, int>, std::vector<float>> views;  // sphe_buffer snapshots by (scene, buffer)
 
-    int block = 128;
-    int fblock = 0;  // block size of the force pass (0: the density pass's)
-    int remap = 128;  // density: runs of 128 consecutive blocks per XCD (L2 locality); force: plain order
+    int block = 0;   // block size of the density and force passes (0: density_block's and force_block's choice)
+    int fblock = 0;  // block size of the force pass alone (0: as block)
+    int remap = 128;  // density: runs of 128 consecutive blocks per XCD (L2 locality); force: plain order (balance)
     int maxn = 256;  // neighbour-list capacity per particle (grown when a step overflows it)
     int ocap = 256;  // entries per overflow-pool chunk
     size_t mem_total = 0;  // the device's memory (bounds the neighbour lists)
@@ -848,8 +848,16 @@ struct Timed {
     }
 };
 
-// block size of the force pass: its own when set, else the density pass's
-int force_block(const sphe_ctx* c) { return c->fblock ? c->fblock : c->block; }
+// Block sizes of the density and force passes where none was set.  Nothing is
+// shared in a block but its place on a CU: one-wave blocks leave it wave by
+// wave.  Density, blocks of 64 / 128 / 256: 4,096 particles 10.1 / 13.0 / 12.0
+// us, 262,144 62.5 / 65.4 / 66.5, 700,001 126.7 / 129.2 / 132.3, but
+// 4,194,304 1,270 / 1,245 / 1,225 (four neighbouring waves share more of a
+// CU's L1).  Force, blocks of 64 / 128: 4,096 9.2 / 10.3, 48 uneven scenes 189 /
+// 203, 262,144 64.3 / 65.5, 4,194,304 1,318 / 1,337.
+const int64_t kDensityBigP = 1 << 21;
+int density_block(const sphe_ctx* c) { return c->block ? c->block : (c->D.P > kDensityBigP ? 256 : 64); }
+int force_block(const sphe_ctx* c) { return c->fblock ? c->fblock : (c->block ? c->block : 64); }
 
 bool any_erosion(const sphe_ctx* c, int mode)
 {
@@ -884,11 +892,11 @@ void launch_step(sphe_ctx* c, bool first)
     launch_sort(c, first);
     {
         Timed t(c, "density");
-        sphe_launch_density(D, c->block, c->remap, c->lanes, c->stream, t.a, t.b);
+        sphe_launch_density(D, density_block(c), c->remap, c->lanes, c->stream, t.a, t.b);
     }
     {
         Timed t(c, "force");
-        sphe_launch_force(D, force_block(c), 1, c->lanes, c->stream, t.a, t.b);  // plain XCD order: balance
+        sphe_launch_force(D, force_block(c), c->lanes, c->stream, t.a, t.b);
     }
     if (any_erosion(c, SPHE_EROSION_TWO_PHASE)) {
         Timed t(c, "two_phase");
@@ -901,8 +909,7 @@ std::string plan_signature(const sphe_ctx* c)
     // everything the captured kernels take by value (DevState) or as launch shape
     char b[384];
     snprintf(b, sizeof(b), "%d/%d/%d/%d/%d/%lld/%lld/%lld/%d/%d/%p/%p/%p/%d/%d/%d/%d/%lld/%d/%d/%d",
-             c->precision, c->block,
-             force_block(c), c->remap,
+             c->precision, density_block(c), force_block(c), c->remap,
              c->lanes, (long long)c->D.P, (long long)c->D.C, (long long)c->D.TC, (int)any_erosion(c, -1),
              (int)any_erosion(c, SPHE_EROSION_TWO_PHASE), (const void*)c->D.u_pos, (const void*)c->D.nbl,
              (const void*)c->D.pool, c->D.maxn, c->D.sub_log2, c->D.yz, c->D.ocap, (long long)c->D.pool_cap,
@@ -1175,7 +1182,7 @@ int sort_current(sphe_ctx* c)
         if (r) return r;
     }
     launch_sort(c, false);
-    sphe_launch_density(c->D, c->block, c->remap, c->lanes, c->stream);
+    sphe_launch_density(c->D, density_block(c), c->remap, c->lanes, c->stream);
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipStreamSynchronize(c->stream));
     c->counted = false;
@@ -2348,7 +2355,7 @@ int sphe_get_scan_tile(const sphe_ctx* c, int* log2_cells)
 int sphe_get_tuning(const sphe_ctx* c, int* block, int* remap)
 {
     if (!c) return SPHE_EARG;
-    if (block) *block = c->block;
+    if (block) *block = density_block(c);
     if (remap) *remap = c->remap;
     return SPHE_OK;
 }
@@ -2426,7 +2433,7 @@ int sphe_autotune(sphe_ctx* c, int steps_per_trial)
     if (r) return r;
     const bool prof = c->profiling;
     const auto saved_prof = c->prof;
-    int best_b = c->block, best_fb = force_block(c);
+    int best_b = density_block(c), best_fb = force_block(c);
     double best_d = 1e30, best_f = 1e30;
     // the block sizes only: the best XCD run length depends on how uneven the
     // state is (long runs win on uniform states and lose by up to a fifth on
@@ -2511,7 +2518,7 @@ int sphe_autotune_grid(sphe_ctx* c, int steps_per_trial)
     // what the choice depends on: the device, the kernels' variants, the
     // scenes' sizes and smoothing lengths (not the grid being tuned)
     std::string key = std::string(prop.gcnArchName) + "|" + std::to_string(c->precision) + "/" +
-                      std::to_string(c->lanes) + "/" + std::to_string(c->block) + "/" +
+                      std::to_string(c->lanes) + "/" + std::to_string(density_block(c)) + "/" +
                       std::to_string(force_block(c)) + "/" + std::to_string(c->D.P) + "/" +
                       std::to_string((int)any_erosion(c, -1));
     for (const Scene& s : c->scenes)
