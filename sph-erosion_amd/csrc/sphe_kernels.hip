@@ -783,73 +783,87 @@ __global__ __launch_bounds__(256) void k_scatter(DevState D)
 // first also writes the cell's slab offsets: for s = 1 .. 2^sub_log2 - 1 the
 // number of the cell's particles in slabs below s, 10 bits each from bit
 // 10 (s - 1); a cell of more than 1023 particles gets bit 31 instead.
-// A particle's rank is counted over its cell's (key, id) words: the block
-// first stages the words of the cells its 256 slots lie in (a window of at
-// most SPHE_REORDER_WINDOW slots) in LDS, with one coalesced pass, so each
-// word is read from memory about once; a block whose cells are larger ranks
-// from memory.
+// A particle's rank is counted over its cell's (key, id) words, staged in LDS by
+// the block: at once, without waiting for the cells' ranges, the words of its
+// own 256 slots and of SPHE_REORDER_SIDE on either side; where a cell reaches
+// further (a pile-up), the words of the cells its slots lie in (a window of at
+// most SPHE_REORDER_WINDOW slots); a block whose cells are larger still ranks
+// from memory.  The pass is a chain of latencies up to some 100,000 particles:
+// words, then cell ranges and the particle's state together, then the stores
+// (262,144 particles: 9.9 us with the window read after the ranges and the
+// state after the window, 8.0 now); bound by HBM beyond (100 bytes a particle:
+// 4.2M 99 us, now 79, 5.3 TB/s).
 #define SPHE_REORDER_WINDOW 2048
+#define SPHE_REORDER_SIDE 256
 template <typename T>
 __global__ __launch_bounds__(256) void k_reorder(DevState D)
 {
     __shared__ uint64_t wkid[SPHE_REORDER_WINDOW];
     __shared__ uint32_t wlo, whi;
-    const int64_t d = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    constexpr int SIDE = SPHE_REORDER_SIDE;
+    const int64_t base = (int64_t)blockIdx.x * 256;
+    const int64_t d = base + threadIdx.x;
     const bool live = d < D.P;
     const int sl = D.sub_log2;
-    uint64_t kid = 0;
-    int32_t src = 0, c = 0;
-    uint32_t s0 = 0, s1 = 0;
-    bool ok = false;
-    if (live) {
-        kid = D.tmp_kid[d];
-        src = D.tmp_src[d];
-        const int32_t fk = (int32_t)(kid >> 32);
-        c = fk >> sl;
-        ok = fk >= 0 && (int64_t)c < D.C;
-        if (ok) {
-            s0 = D.cells[c].x;
-            s1 = D.cells[(size_t)c + 1].x;
-            if ((int64_t)s1 > D.P) s1 = (uint32_t)D.P;
+    // slots before and after the block's, clamped to the array's (P > 0)
+    const int64_t before = base - SIDE + (int64_t)threadIdx.x, after = base + 256 + (int64_t)threadIdx.x;
+    const uint64_t kb = D.tmp_kid[before < 0 ? 0 : before], ka = D.tmp_kid[after < D.P ? after : D.P - 1];
+    const uint64_t kid = D.tmp_kid[live ? d : D.P - 1];
+    const int32_t src = D.tmp_src[live ? d : D.P - 1];
+    wkid[threadIdx.x] = kb;
+    wkid[SIDE + threadIdx.x] = kid;
+    wkid[SIDE + 256 + threadIdx.x] = ka;
+    const int32_t fk = (int32_t)(kid >> 32);
+    const int32_t c = fk >> sl;
+    const bool ok = live && fk >= 0 && (int64_t)c < D.C;
+    const uint32_t cc = ok ? (uint32_t)c : 0u;
+    // the particle's state, gathered while its rank is found (from a slot
+    // clamped into range: a bad src is reported below and never stored)
+    const uint32_t sc = (uint32_t)min(max(src, 0), (int32_t)(D.P - 1));
+    uint32_t s0 = D.cells[cc].x, s1 = D.cells[cc + 1u].x;
+    const V4<T> pv = at((const V4<T>*)D.u_pos, sc);
+    const V4<T> vv = at((const V4<T>*)D.u_vel, sc);
+    const int64_t sed = D.u_sed[sc];
+    if (!ok) s0 = s1 = 0u;
+    if ((int64_t)s1 > D.P) s1 = (uint32_t)D.P;
+    uint32_t w0 = (uint32_t)(base > SIDE ? base - SIDE : 0);
+    int shift = (int)(base - SIDE);  // slot of wkid[0]; negative in the first block
+    bool staged = true;
+    if (__syncthreads_or(s0 < s1 && (s0 < w0 || (int64_t)s1 > base + 256 + SIDE))) {
+        if (threadIdx.x == 0) {
+            wlo = ~0u;
+            whi = 0u;
         }
-    }
-    if (threadIdx.x == 0) {
-        wlo = ~0u;
-        whi = 0u;
-    }
-    __syncthreads();
-    {
-        // the block's window of cell slots: reduced over each wave, then one
-        // LDS atomic pair per wave
-        uint32_t lo = ok && s0 < s1 ? s0 : ~0u, hi = ok && s0 < s1 ? s1 : 0u;
+        __syncthreads();
+        {
+            // the block's window of cell slots: reduced over each wave, then
+            // one LDS atomic pair per wave
+            uint32_t lo = s0 < s1 ? s0 : ~0u, hi = s0 < s1 ? s1 : 0u;
 #pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) {
-            const uint32_t a = __shfl_xor(lo, o, 64), b = __shfl_xor(hi, o, 64);
-            lo = a < lo ? a : lo;
-            hi = b > hi ? b : hi;
+            for (int o = 32; o >= 1; o >>= 1) {
+                const uint32_t a = __shfl_xor(lo, o, 64), b = __shfl_xor(hi, o, 64);
+                lo = a < lo ? a : lo;
+                hi = b > hi ? b : hi;
+            }
+            if ((threadIdx.x & 63) == 0 && lo < hi) {
+                atomicMin(&wlo, lo);
+                atomicMax(&whi, hi);
+            }
         }
-        if ((threadIdx.x & 63) == 0 && lo < hi) {
-            atomicMin(&wlo, lo);
-            atomicMax(&whi, hi);
-        }
+        __syncthreads();
+        w0 = wlo;
+        const uint32_t w1 = whi;
+        staged = w0 < w1 && w1 - w0 <= (uint32_t)SPHE_REORDER_WINDOW;  // block-uniform
+        if (staged)
+            for (uint32_t j = w0 + threadIdx.x; j < w1; j += blockDim.x) wkid[j - w0] = D.tmp_kid[j];
+        __syncthreads();
+        shift = (int)w0;
     }
-    __syncthreads();
-    const uint32_t w0 = wlo, w1 = whi;
-    const bool staged = w0 < w1 && w1 - w0 <= (uint32_t)SPHE_REORDER_WINDOW;  // block-uniform
-    if (staged)
-        for (uint32_t j = w0 + threadIdx.x; j < w1; j += blockDim.x) wkid[j - w0] = D.tmp_kid[j];
-    __syncthreads();
     if (!live) return;
     if (!ok) {
         atomicOr(D.status, 2u);
         return;
     }
-    // the particle's state, gathered while its rank is found (from a slot
-    // clamped into range: a bad src is reported below and never stored)
-    const uint32_t sc = (uint32_t)min(max(src, 0), (int32_t)(D.P - 1));
-    const V4<T> pv = at((const V4<T>*)D.u_pos, sc);
-    const V4<T> vv = at((const V4<T>*)D.u_vel, sc);
-    const int64_t sed = D.u_sed[sc];
     const int32_t my = (int32_t)((uint32_t)kid ^ 0x80000000u);
     // one count field per slab boundary: a particle in slab k adds 1 to the
     // fields of the boundaries s > k
@@ -857,19 +871,21 @@ __global__ __launch_bounds__(256) void k_reorder(DevState D)
     const uint32_t smask = (1u << sl) - 1u;
     uint32_t rank = 0, below = 0;
     auto take = [&](uint32_t j, uint64_t o) {
-        rank += (o < kid || (o == kid && D.tmp_src[j] < src)) ? 1u : 0u;
+        rank += o < kid ? 1u : 0u;
+        if (__builtin_expect(o == kid && j != (uint32_t)d, 0)) rank += D.tmp_src[j] < src ? 1u : 0u;
         below += fields & (~0u << (10u * ((uint32_t)(o >> 32) & smask)));
     };
     uint32_t j = s0;
     if (staged) {
         for (; j + 3 < s1; j += 4) {
-            const uint64_t o0 = wkid[j - w0], o1 = wkid[j + 1 - w0], o2 = wkid[j + 2 - w0], o3 = wkid[j + 3 - w0];
+            const uint64_t* w = wkid + ((int)j - shift);
+            const uint64_t o0 = w[0], o1 = w[1], o2 = w[2], o3 = w[3];
             take(j, o0);
             take(j + 1, o1);
             take(j + 2, o2);
             take(j + 3, o3);
         }
-        for (; j < s1; ++j) take(j, wkid[j - w0]);
+        for (; j < s1; ++j) take(j, wkid[(int)j - shift]);
     } else {
         for (; j + 1 < s1; j += 2) {  // two loads in flight
             const uint64_t o0 = D.tmp_kid[j], o1 = D.tmp_kid[j + 1];

@@ -179,3 +179,16 @@ def test_small_and_large_reads(precision):
     ctx.set_particles(sids[1], ctx.positions(sids[1])[::-1].copy())
     ctx.step(1)
     check()
+
+
+@pytest.mark.parametrize("cluster", [1, 255, 256, 257, 300, 512, 513, 1400, 2048, 2100])
+def test_reorder_windows_bit_exact_twin(cluster):
+    """A cell of `cluster` particles among scattered ones, met at several
+    offsets of the blocks of 256 slots: ranked from the block's own words and
+    256 on either side, from its cells' words, or from memory."""
+    h = 0.0457
+    rng = np.random.default_rng(cluster)
+    pos = np.concatenate([rng.uniform(-0.19, 0.0, (300 + 37 * (cluster % 5), 3)),
+                          0.005 + rng.uniform(0.0, 0.01 * h, (cluster, 3)), rng.uniform(0.06, 0.19, (200, 3))])
+    pos = pos[rng.permutation(len(pos))]
+    _compare(_params(h, 0.2, dt=1e-9), pos, 2, sphe.FP32, 1, 1)
