@@ -103,9 +103,7 @@ struct DevState {
     int32_t yz;
     int32_t h_unit;  // every scene's smoothing length is at most 1
     int64_t* vol; float* height;
-    int64_t* dq; int32_t* tcell;        // two-phase erosion records
-    uint32_t* tcnt; uint32_t* tstart; uint32_t* tpartial; int64_t ntpartial;
-    int64_t* tdq;                       // two-phase: deltas grouped by terrain cell
+    int64_t* tsum;                      // two-phase erosion: a step's volume change of each terrain cell
     uint32_t* status;
     double* red;                        // reduction scratch
     int64_t nred;

@@ -8,9 +8,6 @@
 // e0 / e1 (optional): profiling events that take the start of the first and
 // the end of the last kernel a launcher issues.
 void sphe_launch_hash(const DevState& D, hipStream_t st, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
-// Exclusive prefix of n counts; with zero_counts the counts are reset.
-void sphe_launch_scan(uint32_t* cnt, uint32_t* start, int64_t n, uint32_t* partial, bool zero_counts,
-                      hipStream_t st);
 // The particle scan: counts -> cell records, the pool's claim counter reset;
 // with heights also the terrain heights, in its first launch; with first the
 // status word is cleared.

@@ -553,13 +553,7 @@ int build_layout(sphe_ctx* c)
     DALLOC(D.tfill, (size_t)D.npartial * 4);
     DALLOC(D.vol, (size_t)TC * 8);
     DALLOC(D.height, (size_t)TC * 4);
-    DALLOC(D.dq, Pn * 8);
-    DALLOC(D.tcell, Pn * 4);
-    DALLOC(D.tcnt, (size_t)(TC + 1) * 4);
-    DALLOC(D.tstart, (size_t)(TC + 1) * 4);
-    D.ntpartial = sphe_scan_partials(TC + 1);
-    DALLOC(D.tpartial, (size_t)D.ntpartial * 4);
-    DALLOC(D.tdq, Pn * 8);
+    DALLOC(D.tsum, (size_t)TC * 8);
     D.maxn = c->maxn;
     DALLOC(D.nbl, Pn * (size_t)D.maxn * 4);
     DALLOC(D.nbc, Pn * 4);
@@ -604,11 +598,11 @@ int build_layout(sphe_ctx* c)
     HIPCHK(c, hipMemsetAsync(D.tocc, 0, (size_t)D.npartial * 4, c->stream));
     HIPCHK(c, hipMemsetAsync(D.tfill, 0xFF, (size_t)D.npartial * 4, c->stream));  // no tile known filled
     HIPCHK(c, hipMemsetAsync(D.cells, 0, (size_t)(C + 2) * 8, c->stream));
-    HIPCHK(c, hipMemsetAsync(D.tcnt, 0, (size_t)(TC + 1) * 4, c->stream));
     HIPCHK(c, hipMemsetAsync(D.status, 0, 64, c->stream));
     HIPCHK(c, hipMemsetAsync(D.ovf, 0, 64, c->stream));
     HIPCHK(c, hipMemsetAsync(D.ptop, 0, 64, c->stream));
     if (TC > 0) HIPCHK(c, hipMemsetAsync(D.vol, 0, (size_t)TC * 8, c->stream));
+    if (TC > 0) HIPCHK(c, hipMemsetAsync(D.tsum, 0, (size_t)TC * 8, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     clear_published(c);  // no overflow published for the new lists
     c->layout_valid = true;

@@ -10,6 +10,7 @@ import pytest
 import oracle as O
 import sphe
 from gpu_common import orc_scene_from
+from sphe import scenes
 
 pytestmark = pytest.mark.gpu
 
@@ -192,3 +193,31 @@ def test_reorder_windows_bit_exact_twin(cluster):
                           0.005 + rng.uniform(0.0, 0.01 * h, (cluster, 3)), rng.uniform(0.06, 0.19, (200, 3))])
     pos = pos[rng.permutation(len(pos))]
     _compare(_params(h, 0.2, dt=1e-9), pos, 2, sphe.FP32, 1, 1)
+
+
+@pytest.mark.parametrize("precision", [sphe.FP32, sphe.FP64])
+@pytest.mark.parametrize("sizes", [(64,), (63, 65, 2), (128, 64, 192)])
+def test_two_phase_sums_in_mixed_batches(sizes, precision):
+    """Scenes without erosion, with atomic and with two-phase erosion in one
+    context, over terrains of odd and even sizes: every scene's terrain,
+    sediment and state are those of the scene alone with atomic erosion (or
+    without), and no sum of an earlier step is left over."""
+    batch = sphe.Context(precision)
+    want, ids = [], []
+    for k, T in enumerate(sizes):
+        for mode in (sphe.EROSION_TWO_PHASE, sphe.EROSION_ATOMIC, sphe.EROSION_OFF):
+            sc = scenes.dam_break_scene(50 + k, 900 + 131 * k, 0.3, T, erosion=mode, steps=4)
+            ids.append(batch.add_synthetic(sc))
+            alone = scenes.dam_break_scene(50 + k, 900 + 131 * k, 0.3, T, steps=4,
+                                           erosion=min(mode, sphe.EROSION_ATOMIC))
+            ctx = sphe.Context(precision)
+            sid = ctx.add_synthetic(alone)
+            ctx.step(19)
+            ctx.step(1)
+            want.append((ctx.terrain_volume_fx(sid), ctx.sediment_fx(sid)) + ctx.state_f64(sid))
+    batch.step(19)
+    batch.step(1)
+    assert any((w[1] != 0).any() for w in want)
+    for sid, w in zip(ids, want):
+        got = (batch.terrain_volume_fx(sid), batch.sediment_fx(sid)) + batch.state_f64(sid)
+        assert all(np.array_equal(a, b) for a, b in zip(got, w))
