@@ -382,7 +382,7 @@ def summarize_profiles(base, workload, steps):
 
     def short(n):
         m = re.search(r"(k_[a-z0-9_]+)", n)
-        return m.group(1) if m else n[:40]
+        return m.group(1).replace("_quad", "") if m else n[:40]  # density for four lanes: k_density_quad
 
     def rows(name, sql):
         db = os.path.join(base, name, "run_results.db")

@@ -300,14 +300,15 @@ int sphe_kernel_bytes(sphe_ctx* ctx, const char* kernel, double* bytes);
 
 /* ---- tuning ------------------------------------------------------------ */
 
-/* Launch parameters: block size of the neighbour kernels (default 128) and
+/* Launch parameters: block size of the neighbour kernels (until one is set, 64,
+ * above 2^21 particle slots 256 for density and 128 for force) and
  * the density pass's XCD mapping: blocks go to the 8 XCDs in runs of
  * xcd_remap consecutive blocks (default 128: neighbouring cells share an
  * XCD's L2; 0 or 1: plain round-robin order).  The force pass always uses
  * the plain order, which keeps the XCDs balanced when neighbour counts vary
  * across the domain.  sphe_set_tuning sets the block size of both neighbour
  * passes; sphe_set_force_block then gives the force pass its own (0: the
- * density pass's), and sphe_get_force_block reads the one in effect.
+ * block of sphe_set_tuning), and the getters read the sizes in effect.
  * sphe_autotune runs the step with block sizes {64, 128, 256, 512}, times
  * the density and force passes of each trial with the profiling events, and
  * keeps each pass's fastest, with the run as set.  No parameter here

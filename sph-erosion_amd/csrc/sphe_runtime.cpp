@@ -844,14 +844,21 @@ struct Timed {
 
 // Block sizes of the density and force passes where none was set.  Nothing is
 // shared in a block but its place on a CU: one-wave blocks leave it wave by
-// wave.  Density, blocks of 64 / 128 / 256: 4,096 particles 10.1 / 13.0 / 12.0
-// us, 262,144 62.5 / 65.4 / 66.5, 700,001 126.7 / 129.2 / 132.3, but
-// 4,194,304 1,270 / 1,245 / 1,225 (four neighbouring waves share more of a
-// CU's L1).  Force, blocks of 64 / 128: 4,096 9.2 / 10.3, 48 uneven scenes 189 /
-// 203, 262,144 64.3 / 65.5, 4,194,304 1,318 / 1,337.
-const int64_t kDensityBigP = 1 << 21;
-int density_block(const sphe_ctx* c) { return c->block ? c->block : (c->D.P > kDensityBigP ? 256 : 64); }
-int force_block(const sphe_ctx* c) { return c->fblock ? c->fblock : (c->block ? c->block : 64); }
+// wave, while in larger ones neighbouring waves share more of a CU's L1, which
+// is what counts on the largest contexts.  Blocks of 64 / 128 / 256, us:
+//   density   4,096 particles 9.7 / 10.4 / 11.7, 262,144 61.7 / 63.7 / 69.5, 700,001
+//             129 / 130 / 132, 1.5M 343 / 341 / 345; 2.5M 660 / 654 / 652, 4.2M 1,282 /
+//             1,254 / 1,255, 256 scenes of 4.6M in all 810 / 796 / 781
+//   force     4,096 7.9 / 8.2 / 9.3, 48 uneven scenes 150 / 162 / 181, 262,144 56.7 /
+//             57.0 / 59.0, 1.5M 388 / 385 / 389; 4.2M 1,227 / 1,230 / 1,255, 256 scenes 754 /
+//             740 / 727
+const int64_t kManySlots = 1 << 21;
+int density_block(const sphe_ctx* c) { return c->block ? c->block : (c->D.P > kManySlots ? 256 : 64); }
+int force_block(const sphe_ctx* c)
+{
+    if (c->fblock) return c->fblock;
+    return c->block ? c->block : (c->D.P > kManySlots ? 128 : 64);
+}
 
 bool any_erosion(const sphe_ctx* c, int mode)
 {
