@@ -2,8 +2,8 @@
 //
 // One step (all scenes of a context at once), reference Erosion/fluid_system.h
 // FluidSystemSPH::Run (:104-183) + advance (:306-353):
-//   scan      counts -> cell starts (1 to 3 kernels; tiles no particle counted
-//             into are not read)
+//   scan      counts -> cell starts (one or two kernels; tiles no particle
+//             counted into are not read)
 //   scatter   each particle to its cell segment (arrival order); resets
 //             its cell's count for the next step
 //   reorder   rank inside the cell by (x slab, particle id) -> canonical
@@ -468,12 +468,26 @@ __device__ __forceinline__ int32_t position_key(const DevState& D, const SceneDe
     return (int32_t)((key << D.sub_log2) | sub);
 }
 
-// Counts a particle of that key into its cell: its rank of arrival.
+// Word of scan tile t's total, and the tile of word w.
+__device__ __forceinline__ uint32_t tile_word(int tlog, uint32_t t) { return ((t & ((1u << tlog) - 1u)) << 5) | (t >> tlog); }
+__device__ __forceinline__ uint32_t word_tile(int tlog, uint32_t w) { return ((w & 31u) << tlog) | (w >> 5); }
+
+// Counts a particle of that key into its scan tile and its cell: its rank of
+// arrival in the cell.  The lanes that count here together are mostly
+// neighbours of one tile, which takes one atomic of the wave then (with the
+// totals in tile order, and so on a few lines, the force pass took 77 us instead
+// of 57 for 262,144 particles, and 289 instead of 155 for 48 uneven scenes).
 __device__ __forceinline__ uint32_t count_key(const DevState& D, int32_t key)
 {
-    const int32_t cell = key >> D.sub_log2;
-    D.tocc[cell >> D.scan_log2] = 1u;
-    return atomicAdd(&D.cnt[cell], 1u);
+    const int32_t cell = key >> D.sub_log2, tile = cell >> D.scan_log2;
+    const uint32_t rank = atomicAdd(&D.cnt[cell], 1u);
+    const int32_t t0 = __builtin_amdgcn_readfirstlane(tile);
+    const uint64_t same = __builtin_amdgcn_ballot_w64(tile == t0);
+    const bool leads =
+        __builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0u)) == 0u;
+    if (tile != t0 || leads)
+        atomicAdd(&D.total[tile_word(D.tlog, (uint32_t)tile)], tile != t0 ? 1u : (uint32_t)__popcll(same));
+    return rank;
 }
 
 template <typename T>
@@ -489,8 +503,7 @@ __device__ __forceinline__ void count_pad(const DevState& D, const SceneDev& S, 
 {
     const int64_t key = S.cell_off + S.ncell;
     D.key[slot] = (int32_t)(key << D.sub_log2);
-    D.arank[slot] = atomicAdd(&D.cnt[key], 1u);
-    D.tocc[key >> D.scan_log2] = 1u;
+    D.arank[slot] = count_key(D, (int32_t)(key << D.sub_log2));
 }
 
 // ------------------------------------------------------------------ sort
@@ -564,34 +577,13 @@ __device__ __forceinline__ void store4(uint2* __restrict__ p, int64_t i, int64_t
     }
 }
 
-// Total of count tile `tile` into partial[tile].  occ: the tile flags; an
-// unflagged tile's counts are all zero.
-template <int ITEMS>
-__device__ __forceinline__ void scan_reduce_tile(const uint32_t* __restrict__ in, int64_t n,
-                                                 uint32_t* __restrict__ partial, const uint32_t* __restrict__ occ,
-                                                 int tile, uint32_t* lds)
-{
-    if (occ[tile] == 0u) {
-        if (threadIdx.x == 0) partial[tile] = 0u;
-        return;
-    }
-    uint4 v[ITEMS / 4];
-    load_tile<ITEMS>(in, tile, n, v);
-    uint32_t s = 0;
-#pragma unroll
-    for (int c = 0; c < ITEMS / 4; ++c) s += (v[c].x + v[c].y) + (v[c].z + v[c].w);
-    s = wave_total(s);
-    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) partial[tile] = (lds[0] + lds[1]) + (lds[2] + lds[3]);
-}
-
-// Exclusive prefix of the n tile totals, in place, by one block of 1,024
+// Exclusive prefix of the n tile totals by one block of 1,024
 // threads: chunks of 16,384 totals, 16 consecutive ones per thread, one block
 // scan per chunk and the running total carried to the next chunk.  Linear in
 // the number of tiles; each scan-down block then reads its tile's prefix
 // with one load.
-__global__ __launch_bounds__(1024) void k_scan_tiles(uint32_t* __restrict__ partial, int64_t n)
+__global__ __launch_bounds__(1024) void k_scan_tiles(const uint32_t* __restrict__ total, int tlog,
+                                                     uint32_t* __restrict__ pre, int64_t n)
 {
     constexpr int ITEMS = 16;
     __shared__ uint32_t lds[16];
@@ -601,7 +593,7 @@ __global__ __launch_bounds__(1024) void k_scan_tiles(uint32_t* __restrict__ part
         const int64_t base = c0 + (int64_t)threadIdx.x * ITEMS;
         uint32_t v[ITEMS];
 #pragma unroll
-        for (int i = 0; i < ITEMS; ++i) v[i] = base + i < n ? partial[base + i] : 0u;
+        for (int i = 0; i < ITEMS; ++i) v[i] = base + i < n ? total[tile_word(tlog, (uint32_t)(base + i))] : 0u;
         uint32_t s = 0;
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i) s += v[i];
@@ -624,39 +616,37 @@ __global__ __launch_bounds__(1024) void k_scan_tiles(uint32_t* __restrict__ part
         }
 #pragma unroll
         for (int i = 0; i < ITEMS; ++i)
-            if (base + i < n) partial[base + i] = v[i];
+            if (base + i < n) pre[base + i] = v[i];
         carry += tot;
         __syncthreads();  // the wave totals of the next chunk reuse lds
     }
 }
 
 // Where a tile's prefix (the total of the tiles before it) comes from: a word
-// that k_scan_tiles left; the tiles' totals, added here; the counts before the
-// tile, added here, with no pass over the tiles before this one.  A launch
-// costs 4.5 us, so for few tiles the last two are faster although every block
-// repeats the sum: up to SCAN_SUM_TILES tiles a block adds 4 words a thread on
-// average at the limit, which its loads hide; up to SCAN_COUNT_TILES it reads
-// at most 256 KB of counts from L2.  Three launches against these: 12.8 -> 4.8
-// us on a grid of 2,900 cells and 13.2 -> 7.3 us on one of 39,000 (one launch),
-// 19.8 -> 13.4 us on 6.7M cells (two).  Runs of consecutive lines instead of
-// each thread's own 64 or 128 bytes: 57 -> 40 us on 16.7M cells (three).
-enum { SCAN_PREFIX, SCAN_SUMS, SCAN_COUNTS };
+// that k_scan_tiles left, or the tiles' totals, added here by every block: up
+// to SCAN_SUM_TILES tiles, at most 8 loads a thread, while a launch costs 4 us.  The totals themselves are counted
+// with the particles (count_key; a pass over the counts for them took a launch:
+// 13.2 -> 7.3 us on 6.7M cells, 19.6 -> 13.8 for 96 scenes with their terrain
+// heights, 40 -> 34 on 16.7M cells; for few tiles every block added the counts
+// before its tile: 5.6 -> 4.2 us on 39,000 cells).  Runs of consecutive lines instead
+// of each thread's own 64 or 128 bytes: 57 -> 40 us on 16.7M cells, before that.
+enum { SCAN_PREFIX, SCAN_SUMS };
 #define SPHE_SCAN_SUM_TILES 4096
-#define SPHE_SCAN_COUNT_TILES 16
 
 // start = exclusive prefix of the counts of one tile (each cell's first scatter
-// resets its count for the next arrivals).  occ: the tile flags; an unflagged
-// tile's counts are not read (all zero), and the block clears its tile's flag
-// once read.  fill: per tile, the value all of an empty tile's starts hold
-// since the tile was last written empty (~0: not known); an empty tile whose
-// prefix equals it is not written again.
+// resets its count, and the scatter the tiles' totals, for the next arrivals).
+// A tile whose total is 0 holds only zero counts, which are not read.  fill:
+// per tile, the value all of an empty tile's starts hold since the tile was
+// last written empty (~0: not known); an empty tile whose prefix equals it is
+// not written again.
 template <int ITEMS, int FROM>
 __device__ __forceinline__ void scan_down_tile(const uint32_t* __restrict__ cnt, uint2* __restrict__ start, int64_t n,
-                                               const uint32_t* __restrict__ partial, uint32_t* __restrict__ occ,
+                                               const uint32_t* __restrict__ total, int tlog,
+                                               const uint32_t* __restrict__ tpre,
                                                uint32_t* __restrict__ fill, int tile, uint32_t* lds)
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const bool empty = occ[tile] == 0u;  // block-uniform
+    const bool empty = total[tile_word(tlog, (uint32_t)tile)] == 0u;  // block-uniform
     const uint32_t filled = fill[tile];
     uint4 v[ITEMS / 4];
     if (empty) {
@@ -667,18 +657,16 @@ __device__ __forceinline__ void scan_down_tile(const uint32_t* __restrict__ cnt,
     }
     uint32_t pre = 0;  // this thread's share of the prefix
     if constexpr (FROM == SCAN_PREFIX) {
-        pre = threadIdx.x == 0 ? partial[tile] : 0u;
-    } else if constexpr (FROM == SCAN_SUMS) {
-#pragma unroll 4
-        for (int i = (int)threadIdx.x; i < tile; i += 256) pre += partial[i];
+        pre = threadIdx.x == 0 ? tpre[tile] : 0u;
     } else {
-        // whole tiles, all of a tile's loads in flight
-        for (int k = 0; k < tile; ++k) {
-            uint4 q[ITEMS / 4];
-#pragma unroll
-            for (int c = 0; c < ITEMS / 4; ++c) q[c] = *(const uint4*)(cnt + tile_cell<ITEMS>(k, c));
-#pragma unroll
-            for (int c = 0; c < ITEMS / 4; ++c) pre += (q[c].x + q[c].y) + (q[c].z + q[c].w);
+        // in the order of the words, so that they are read as lines
+#pragma unroll 2
+        for (uint32_t w = threadIdx.x * 4u; w < (32u << tlog); w += 1024u) {
+            const uint4 q = *(const uint4*)(total + w);
+            pre += word_tile(tlog, w) < (uint32_t)tile ? q.x : 0u;
+            pre += word_tile(tlog, w + 1u) < (uint32_t)tile ? q.y : 0u;
+            pre += word_tile(tlog, w + 2u) < (uint32_t)tile ? q.z : 0u;
+            pre += word_tile(tlog, w + 3u) < (uint32_t)tile ? q.w : 0u;
         }
     }
     // sums over the wave of each chunk, then of the waves before
@@ -712,9 +700,8 @@ __device__ __forceinline__ void scan_down_tile(const uint32_t* __restrict__ cnt,
             store4(start, tile_cell<ITEMS>(tile, c), n, o);
         }
     }
-    // every thread read the flag and the fill word before the barrier
+    // every thread read the fill word before the barrier
     if (threadIdx.x == 0) {
-        if (!empty) occ[tile] = 0u;
         const uint32_t nf = empty ? ptot : ~0u;
         if (nf != filled) fill[tile] = nf;
     }
@@ -723,6 +710,8 @@ __device__ __forceinline__ void scan_down_tile(const uint32_t* __restrict__ cnt,
 __global__ __launch_bounds__(256) void k_scatter(DevState D)
 {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    // the tiles' totals are used up
+    for (int64_t w = p; w < (32ll << D.tlog); w += (int64_t)gridDim.x * blockDim.x) D.total[w] = 0u;
     if (p >= D.P) return;
     const int32_t key = D.key[p];  // cell key << sub_log2 | slab
     const int32_t c = key >> D.sub_log2;
@@ -2363,23 +2352,14 @@ __device__ __forceinline__ bool heights_block(const DevState& D, int nscan)
     return true;
 }
 
-template <int ITEMS>
-__global__ __launch_bounds__(256) void k_scan_reduce_cells(DevState D, int nscan, int first)
-{
-    __shared__ uint32_t lds[4];
-    if (first && blockIdx.x == 0 && threadIdx.x == 0) *D.status = 0u;
-    if (heights_block(D, nscan)) return;  // block-uniform: no barrier is skipped by part of a block
-    scan_reduce_tile<ITEMS>(D.cnt, D.C + 1, D.partial, D.tocc, (int)blockIdx.x, lds);
-}
-
 template <int ITEMS, int FROM>
 __global__ __launch_bounds__(256) void k_scan_cells(DevState D, int nscan, int first)
 {
     __shared__ uint32_t lds[8];
     if (first && blockIdx.x == 0 && threadIdx.x == 0) *D.status = 0u;
-    if (FROM == SCAN_COUNTS && heights_block(D, nscan)) return;
+    if (heights_block(D, nscan)) return;  // block-uniform: no barrier is skipped by part of a block
     if (blockIdx.x == 0 && threadIdx.x == 0) *D.ptop = (unsigned long long)D.pool_origin;  // the pool's claims
-    scan_down_tile<ITEMS, FROM>(D.cnt, D.cells, D.C + 1, D.partial, D.tocc, D.tfill, (int)blockIdx.x, lds);
+    scan_down_tile<ITEMS, FROM>(D.cnt, D.cells, D.C + 1, D.total, D.tlog, D.tpre, D.tfill, (int)blockIdx.x, lds);
 }
 
 // Two-phase erosion, second phase: what the force pass summed up for each
@@ -2887,15 +2867,12 @@ static void launch_scan_cells_t(const DevState& D, bool heights, int first, hipS
 {
     const int nb = (int)((D.C + 1 + 256 * ITEMS - 1) / (256 * ITEMS));
     const int nh = heights ? (int)grid_of(D.TC / 4, 256) : 0;  // TC: a multiple of 64
-    if (nb <= SPHE_SCAN_COUNT_TILES) {
-        klaunch(k_scan_cells<ITEMS, SCAN_COUNTS>, nb + nh, 256, st, e0, e1, D, nb, first);
+    if (nb <= SPHE_SCAN_SUM_TILES) {
+        klaunch(k_scan_cells<ITEMS, SCAN_SUMS>, nb + nh, 256, st, e0, e1, D, nb, first);
         return;
     }
-    const bool sums = nb <= SPHE_SCAN_SUM_TILES;
-    klaunch(k_scan_reduce_cells<ITEMS>, nb + nh, 256, st, e0, nullptr, D, nb, first);
-    if (!sums) klaunch(k_scan_tiles, 1, 1024, st, nullptr, nullptr, D.partial, (int64_t)nb);
-    klaunch(sums ? k_scan_cells<ITEMS, SCAN_SUMS> : k_scan_cells<ITEMS, SCAN_PREFIX>, nb, 256, st, nullptr, e1, D, nb,
-            0);
+    klaunch(k_scan_tiles, 1, 1024, st, e0, nullptr, (const uint32_t*)D.total, D.tlog, D.tpre, (int64_t)nb);
+    klaunch(k_scan_cells<ITEMS, SCAN_PREFIX>, nb + nh, 256, st, nullptr, e1, D, nb, first);
 }
 
 void sphe_launch_scan_cells(const DevState& D, bool heights, bool first, hipStream_t st, hipEvent_t e0, hipEvent_t e1)

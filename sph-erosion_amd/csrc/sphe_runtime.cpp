@@ -475,6 +475,17 @@ void clear_published(sphe_ctx* c)
     for (int k = 0; k < 4; ++k) h[k] = 0u;
 }
 
+// log2 of the cache lines that the totals of the scan's tiles are spread over
+// (32 words a line; at least 64 lines, so that few tiles have one each).
+int tile_log(int64_t tiles)
+{
+    int t = 6;
+    while ((32ll << t) < tiles) ++t;
+    return t;
+}
+
+int64_t scan_tiles(int64_t C, int log2_cells) { return (C + 1 + (1ll << log2_cells) - 1) >> log2_cells; }
+
 int build_layout(sphe_ctx* c)
 {
     free_device(c);
@@ -548,8 +559,9 @@ int build_layout(sphe_ctx* c)
     D.scan_log2 = c->scan_log2;
     while (D.sub_log2 > 0 && (C << D.sub_log2) > INT32_MAX) --D.sub_log2;  // keys are int32
     D.npartial = sphe_scan_partials(C + 1);
-    DALLOC(D.partial, (size_t)D.npartial * 4);
-    DALLOC(D.tocc, (size_t)D.npartial * 4);
+    D.tlog = tile_log(scan_tiles(C, D.scan_log2));
+    DALLOC(D.total, (size_t)(32ll << tile_log(D.npartial)) * 4);  // room for every tile size
+    DALLOC(D.tpre, (size_t)D.npartial * 4);
     DALLOC(D.tfill, (size_t)D.npartial * 4);
     DALLOC(D.vol, (size_t)TC * 8);
     DALLOC(D.height, (size_t)TC * 4);
@@ -595,7 +607,7 @@ int build_layout(sphe_ctx* c)
     HIPCHK(c, hipMemcpyAsync(cs, hcs.data(), hcs.size() * 4, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipMemcpyAsync(tcs, htcs.data(), htcs.size() * 4, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipMemsetAsync(D.cnt, 0, (size_t)(C + 1) * 4, c->stream));
-    HIPCHK(c, hipMemsetAsync(D.tocc, 0, (size_t)D.npartial * 4, c->stream));
+    HIPCHK(c, hipMemsetAsync(D.total, 0, (size_t)(32ll << D.tlog) * 4, c->stream));
     HIPCHK(c, hipMemsetAsync(D.tfill, 0xFF, (size_t)D.npartial * 4, c->stream));  // no tile known filled
     HIPCHK(c, hipMemsetAsync(D.cells, 0, (size_t)(C + 2) * 8, c->stream));
     HIPCHK(c, hipMemsetAsync(D.status, 0, 64, c->stream));
@@ -960,6 +972,7 @@ int ensure_graph(sphe_ctx* c, int k, bool first, hipGraphExec_t* exec)
 int recount(sphe_ctx* c)
 {
     HIPCHK(c, hipMemsetAsync(c->D.cnt, 0, (size_t)(c->D.C + 1) * 4, c->stream));
+    HIPCHK(c, hipMemsetAsync(c->D.total, 0, (size_t)(32ll << c->D.tlog) * 4, c->stream));
     {
         Timed t(c, "hash");
         sphe_launch_hash(c->D, c->stream, t.a, t.b);
@@ -2322,12 +2335,13 @@ int sphe_set_scan_tile(sphe_ctx* c, int log2_cells)
         return fail(c, SPHE_EARG, "scan tile must be 2^%d .. 2^%d cells", SPHE_SCAN_LOG2_MIN, SPHE_SCAN_LOG2_MAX);
     c->scan_log2 = log2_cells;
     if (!c->layout_valid || c->D.scan_log2 == log2_cells) return SPHE_OK;
-    // the tile flags and fill words describe tiles of the old size: every
-    // tile is read and written by the next scan, which sets them up again
-    HIPCHK(c, hipMemsetAsync(c->D.tocc, 0x01, (size_t)c->D.npartial * 4, c->stream));
+    // the tiles' totals and fill words are those of the old size: the next step
+    // counts again, and its scan writes every tile
     HIPCHK(c, hipMemsetAsync(c->D.tfill, 0xFF, (size_t)c->D.npartial * 4, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     c->D.scan_log2 = log2_cells;
+    c->D.tlog = tile_log(scan_tiles(c->D.C, log2_cells));
+    c->counted = false;
     return SPHE_OK;
 }
 

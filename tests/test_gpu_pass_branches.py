@@ -221,3 +221,28 @@ def test_two_phase_sums_in_mixed_batches(sizes, precision):
     for sid, w in zip(ids, want):
         got = (batch.terrain_volume_fx(sid), batch.sediment_fx(sid)) + batch.state_f64(sid)
         assert all(np.array_equal(a, b) for a, b in zip(got, w))
+
+
+@pytest.mark.parametrize("graph", [True, False])
+def test_scan_tile_changed_between_steps(graph):
+    """The tiles' totals, counted by the step before for the old tile size, are
+    counted again for the new one: the states stay those of an unchanged
+    context bit for bit."""
+    rng = np.random.default_rng(12)
+    pos = rng.uniform(-0.9, 0.9, (3000, 3)).astype(np.float32)
+    pos[:2000] *= 0.2
+    ctxs = []
+    for _ in range(2):
+        ctx = sphe.Context()
+        ctx.use_graph(graph)
+        sid = ctx.add_scene(_params(0.0457, 1.0))
+        ctx.set_particles(sid, pos)
+        ctx.step(2)
+        ctxs.append(ctx)
+    for log2 in (11, 13, 12, 11):
+        ctxs[0].set_scan_tile(log2)
+        for ctx in ctxs:
+            ctx.step(3)
+        assert ctxs[0].status() == 0
+        a, b = ctxs[0].state_f64(sid), ctxs[1].state_f64(sid)
+        assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
