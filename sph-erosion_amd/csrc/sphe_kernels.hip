@@ -2,7 +2,7 @@
 //
 // One step (all scenes of a context at once), reference Erosion/fluid_system.h
 // FluidSystemSPH::Run (:104-183) + advance (:306-353):
-//   scan      counts -> cell starts (one or two kernels; tiles no particle
+//   scan      counts -> cell starts (one to three kernels; tiles no particle
 //             counted into are not read)
 //   scatter   each particle to its cell segment (arrival order); resets
 //             its cell's count for the next step
@@ -473,14 +473,19 @@ __device__ __forceinline__ uint32_t tile_word(int tlog, uint32_t t) { return ((t
 __device__ __forceinline__ uint32_t word_tile(int tlog, uint32_t w) { return ((w & 31u) << tlog) | (w >> 5); }
 
 // Counts a particle of that key into its scan tile and its cell: its rank of
-// arrival in the cell.  The lanes that count here together are mostly
-// neighbours of one tile, which takes one atomic of the wave then (with the
+// arrival in the cell.  In the largest contexts (D.totals 0) the tile is only
+// marked.  The lanes that count here together are mostly neighbours of one
+// tile, which takes one atomic of the wave then (with the
 // totals in tile order, and so on a few lines, the force pass took 77 us instead
 // of 57 for 262,144 particles, and 289 instead of 155 for 48 uneven scenes).
 __device__ __forceinline__ uint32_t count_key(const DevState& D, int32_t key)
 {
     const int32_t cell = key >> D.sub_log2, tile = cell >> D.scan_log2;
     const uint32_t rank = atomicAdd(&D.cnt[cell], 1u);
+    if (!D.totals) {
+        D.total[tile_word(D.tlog, (uint32_t)tile)] = 1u;
+        return rank;
+    }
     const int32_t t0 = __builtin_amdgcn_readfirstlane(tile);
     const uint64_t same = __builtin_amdgcn_ballot_w64(tile == t0);
     const bool leads =
@@ -2352,6 +2357,25 @@ __device__ __forceinline__ bool heights_block(const DevState& D, int nscan)
     return true;
 }
 
+// The totals of the marked tiles, where they were not counted with the
+// particles.
+template <int ITEMS>
+__global__ __launch_bounds__(256) void k_scan_reduce_cells(DevState D)
+{
+    __shared__ uint32_t lds[4];
+    uint32_t* const total = D.total + tile_word(D.tlog, blockIdx.x);
+    if (*total == 0u) return;  // block-uniform; its writer is this block alone, after the barrier
+    uint4 v[ITEMS / 4];
+    load_tile<ITEMS>(D.cnt, (int64_t)blockIdx.x, D.C + 1, v);
+    uint32_t s = 0;
+#pragma unroll
+    for (int c = 0; c < ITEMS / 4; ++c) s += (v[c].x + v[c].y) + (v[c].z + v[c].w);
+    s = wave_total(s);
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) *total = (lds[0] + lds[1]) + (lds[2] + lds[3]);
+}
+
 template <int ITEMS, int FROM>
 __global__ __launch_bounds__(256) void k_scan_cells(DevState D, int nscan, int first)
 {
@@ -2867,11 +2891,12 @@ static void launch_scan_cells_t(const DevState& D, bool heights, int first, hipS
 {
     const int nb = (int)((D.C + 1 + 256 * ITEMS - 1) / (256 * ITEMS));
     const int nh = heights ? (int)grid_of(D.TC / 4, 256) : 0;  // TC: a multiple of 64
+    if (!D.totals) klaunch(k_scan_reduce_cells<ITEMS>, nb, 256, st, e0, nullptr, D);
     if (nb <= SPHE_SCAN_SUM_TILES) {
-        klaunch(k_scan_cells<ITEMS, SCAN_SUMS>, nb + nh, 256, st, e0, e1, D, nb, first);
+        klaunch(k_scan_cells<ITEMS, SCAN_SUMS>, nb + nh, 256, st, D.totals ? e0 : nullptr, e1, D, nb, first);
         return;
     }
-    klaunch(k_scan_tiles, 1, 1024, st, e0, nullptr, (const uint32_t*)D.total, D.tlog, D.tpre, (int64_t)nb);
+    klaunch(k_scan_tiles, 1, 1024, st, D.totals ? e0 : nullptr, nullptr, (const uint32_t*)D.total, D.tlog, D.tpre, (int64_t)nb);
     klaunch(k_scan_cells<ITEMS, SCAN_PREFIX>, nb + nh, 256, st, nullptr, e1, D, nb, first);
 }
 

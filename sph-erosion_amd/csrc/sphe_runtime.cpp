@@ -475,6 +475,10 @@ void clear_published(sphe_ctx* c)
     for (int k = 0; k < 4; ++k) h[k] = 0u;
 }
 
+// Contexts of more slots take other block sizes and another scan (density_block,
+// build_layout).
+const int64_t kManySlots = 1 << 21;
+
 // log2 of the cache lines that the totals of the scan's tiles are spread over
 // (32 words a line; at least 64 lines, so that few tiles have one each).
 int tile_log(int64_t tiles)
@@ -560,6 +564,10 @@ int build_layout(sphe_ctx* c)
     while (D.sub_log2 > 0 && (C << D.sub_log2) > INT32_MAX) --D.sub_log2;  // keys are int32
     D.npartial = sphe_scan_partials(C + 1);
     D.tlog = tile_log(scan_tiles(C, D.scan_log2));
+    // above 2^21 slots the atomics on the totals cost the force pass more than
+    // the launch that adds them up (13.95M particles: force 4.37 ms against
+    // 4.15, the scan 6 us less; 4.2M: 1,243 us against 1,236, 6 us less)
+    D.totals = P <= kManySlots;
     DALLOC(D.total, (size_t)(32ll << tile_log(D.npartial)) * 4);  // room for every tile size
     DALLOC(D.tpre, (size_t)D.npartial * 4);
     DALLOC(D.tfill, (size_t)D.npartial * 4);
@@ -864,7 +872,6 @@ struct Timed {
 //   force     4,096 7.9 / 8.2 / 9.3, 48 uneven scenes 150 / 162 / 181, 262,144 56.7 /
 //             57.0 / 59.0, 1.5M 388 / 385 / 389; 4.2M 1,227 / 1,230 / 1,255, 256 scenes 754 /
 //             740 / 727
-const int64_t kManySlots = 1 << 21;
 int density_block(const sphe_ctx* c) { return c->block ? c->block : (c->D.P > kManySlots ? 256 : 64); }
 int force_block(const sphe_ctx* c)
 {
