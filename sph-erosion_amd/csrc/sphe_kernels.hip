@@ -632,8 +632,8 @@ __global__ __launch_bounds__(1024) void k_scan_tiles(const uint32_t* __restrict_
 // to SCAN_SUM_TILES tiles, at most 8 loads a thread, while a launch costs 4 us.  The totals themselves are counted
 // with the particles (count_key; a pass over the counts for them took a launch:
 // 13.2 -> 7.3 us on 6.7M cells, 19.6 -> 13.8 for 96 scenes with their terrain
-// heights, 40 -> 34 on 16.7M cells; for few tiles every block added the counts
-// before its tile: 5.6 -> 4.2 us on 39,000 cells).  Runs of consecutive lines instead
+// heights; for few tiles every block added the counts before its tile: 5.6 ->
+// 4.2 us on 39,000 cells), except in the largest contexts (build_layout).  Runs of consecutive lines instead
 // of each thread's own 64 or 128 bytes: 57 -> 40 us on 16.7M cells, before that.
 enum { SCAN_PREFIX, SCAN_SUMS };
 #define SPHE_SCAN_SUM_TILES 4096
