@@ -1455,6 +1455,10 @@ __device__ __forceinline__ void density_quad(const DevState& D, int b)
     if (slot >= hi) return;  // padding: whole groups leave together
     const V4<T> pi = pos[slot];
     {
+        // A stream that ends with a segment is looked up once more, past its end
+        // and past the marks: none there, so that look-up stays at the last row.
+        *lds_at<lds_u32>(marks + SPHE_SEG / 8 + 4u * (uint32_t)l) = 0u;
+        static_assert(QUAD_MARKS == SPHE_SEG / 8 + 16, "one 4-byte store a lane");
         clear_marks();
         constexpr int NR = YZ == 1 ? 3 : 7;  // the planes' rows l, then the fifth rows
         uint32_t j0[NR], len[NR];

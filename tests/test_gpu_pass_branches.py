@@ -246,3 +246,29 @@ def test_scan_tile_changed_between_steps(graph):
         assert ctxs[0].status() == 0
         a, b = ctxs[0].state_f64(sid), ctxs[1].state_f64(sid)
         assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
+
+
+@pytest.mark.parametrize("block", [64, 256, 512])
+@pytest.mark.parametrize("yz", [1, 2])
+@pytest.mark.parametrize("n", [256, 512, 768, 1024])
+def test_streams_that_end_with_a_segment(n, yz, block):
+    """Every particle is a candidate of every other, so all streams end with a
+    segment of row marks, the ones of a block's last group too: the look-up past
+    their end finds no marks, and the sums and lists are the twin's."""
+    h = 0.0457
+    rng = np.random.default_rng(n + yz)
+    pos = (rng.uniform(0.0, 0.4 * h, (n, 3)) + 0.013).astype(np.float32)
+    p = _params(h, 0.2)
+    ctx = sphe.Context()
+    ctx.set_yz_split(yz)
+    ctx.set_tuning(block, 1)
+    sid = ctx.add_scene(p)
+    ctx.set_particles(sid, pos)
+    ctx.step(1)
+    gp, gv = ctx.state_f64(sid)
+    osc = orc_scene_from(p)
+    osc.yz = yz
+    st = O.orc_step(osc, pos.astype(np.float64), np.zeros((n, 3)), np.zeros(n, np.int64),
+                    np.arange(n, dtype=np.int32), real=4, comp=1)
+    assert np.array_equal(gp, st["pos"]) and np.array_equal(gv, st["vel"])
+    assert np.array_equal(ctx.density(sid).astype(np.float64), st["rho"])
