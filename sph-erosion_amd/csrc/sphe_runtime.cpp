@@ -2398,12 +2398,12 @@ int sphe_restore_state(sphe_ctx* c)
     if (!c) return SPHE_EARG;
     if (!c->has_saved) return fail(c, SPHE_ESTATE, "no saved state");
     if (c->saved.size() != c->scenes.size()) return fail(c, SPHE_ESTATE, "scenes were added after the state was saved");
+    // the layout holds for these ids (the id maps) and terrain sizes
     bool same = true;
-    for (size_t i = 0; i < c->scenes.size(); ++i)
-        same = same && c->scenes[i].ids.size() == c->saved[i].ids.size() &&
-               c->scenes[i].vol.size() == c->saved[i].vol.size();
+    for (size_t i = 0; i < c->scenes.size() && same; ++i)
+        same = c->scenes[i].ids == c->saved[i].ids && c->scenes[i].vol.size() == c->saved[i].vol.size();
     if (!same) {
-        int r = begin_host_edit(c);  // particle or terrain sizes changed: new layout
+        int r = begin_host_edit(c);  // other particles or terrain sizes: new layout
         if (r) return r;
     }
     for (size_t i = 0; i < c->scenes.size(); ++i) {

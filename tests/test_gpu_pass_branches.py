@@ -272,3 +272,47 @@ def test_streams_that_end_with_a_segment(n, yz, block):
                     np.arange(n, dtype=np.int32), real=4, comp=1)
     assert np.array_equal(gp, st["pos"]) and np.array_equal(gv, st["vel"])
     assert np.array_equal(ctx.density(sid).astype(np.float64), st["rho"])
+
+
+@pytest.mark.parametrize("precision", [sphe.FP32, sphe.FP64])
+@pytest.mark.parametrize("n", [600, 22000])
+@pytest.mark.parametrize("saved,other", [("sparse", "dense"), ("dense", "sparse"), ("sparse", "shifted")])
+def test_restored_state_with_other_ids(saved, other, n, precision):
+    """A state restored over the same number of particles of other ids reads as
+    in a context that never held those: positions, velocities and densities
+    (22,000: past the staging buffer), records, absent ids refused."""
+    ids = {"sparse": 2 * np.arange(n, dtype=np.int32), "dense": np.arange(n, dtype=np.int32)}
+    ids["shifted"] = ids["sparse"] + 1
+    rng = np.random.default_rng(n)
+    pos = rng.uniform(-0.3, 0.3, (n, 3)).astype(np.float32)
+    ctxs = []
+    for replaced in (True, False):
+        ctx = sphe.Context(precision)
+        sid = ctx.add_scene(_params(0.0457, 0.4))
+        ctx.set_particles(sid, pos, ids=ids[saved])
+        if replaced:
+            ctx.save_state()
+            ctx.set_particles(sid, pos[::-1].copy(), ids=ids[other])
+            ctx.step(1)
+            ctx.positions(sid)
+            ctx.particle(sid, int(ids[other][3]))
+            ctx.restore_state()
+        ctx.step(1)
+        ctxs.append(ctx)
+
+    def reads(ctx):
+        yield ctx.positions(sid)
+        yield ctx.velocities(sid)
+        yield ctx.density(sid)
+        yield ctx.read(sid, sphe.BUF_ID)
+        yield from ctx.state_f64(sid)
+    for got, want in zip(reads(ctxs[0]), reads(ctxs[1])):
+        assert np.array_equal(got, want)
+    present = set(ids[saved].tolist())
+    for i in (0, 1, 2, 3, n - 1, n, 2 * n - 2, 2 * n - 1, 2 * n):
+        if i in present:
+            assert bytes(ctxs[0].particle(sid, i)) == bytes(ctxs[1].particle(sid, i))
+        else:
+            for ctx in ctxs:
+                with pytest.raises(sphe.SpheError):
+                    ctx.particle(sid, i)
