@@ -799,7 +799,8 @@ int upload_table(sphe_ctx* c, bool force)
         HIPCHK(c, hipMemcpyAsync((void*)c->D.scenes, c->table.data(), t.size() * sizeof(SceneDev),
                                  hipMemcpyHostToDevice, c->stream));
     c->table_uploaded = true;
-    ++c->epoch;  // new constants: a kept sort of the state no longer holds
+    c->lists_valid = false;  // an inspection under new constants walks for the neighbours they give
+    ++c->epoch;              // new constants: a kept sort of the state no longer holds
     return SPHE_OK;
 }
 

@@ -316,3 +316,30 @@ def test_restored_state_with_other_ids(saved, other, n, precision):
             for ctx in ctxs:
                 with pytest.raises(sphe.SpheError):
                     ctx.particle(sid, i)
+
+
+@pytest.mark.parametrize("precision", [sphe.FP32, sphe.FP64])
+@pytest.mark.parametrize("change", [dict(h=0.0447), dict(h=0.0463), dict(mass=0.021)])
+def test_inspection_after_a_change_of_parameters(change, precision):
+    """Parameters that reach the device between a step and an inspection (here
+    with the mass bookkeeping) make the record one of the new parameters over
+    the neighbours they give, whether or not the step's lists are still there."""
+    rng = np.random.default_rng(5)
+    pos = rng.uniform(-0.15, 0.15, (2500, 3)).astype(np.float32)
+    recs = []
+    for renewed in (False, True):
+        ctx = sphe.Context(precision)
+        sid = ctx.add_scene(_params(0.0457, 0.2))
+        ctx.set_particles(sid, pos)
+        ctx.step(1)
+        prm = ctx.get_params(sid)
+        for k, v in change.items():
+            setattr(prm, k, v)
+        ctx.set_params(sid, prm)
+        ctx.mass(sid)
+        if renewed:
+            ctx.set_list_capacity(1024)
+        recs.append([bytes(ctx.particle(sid, i)) for i in range(0, 2500, 50)])
+    assert recs[0] == recs[1]
+    ctx.step(1)
+    ctx.particle(sid, 0)
