@@ -300,9 +300,10 @@ int sphe_kernel_bytes(sphe_ctx* ctx, const char* kernel, double* bytes);
 
 /* ---- tuning ------------------------------------------------------------ */
 
-/* Launch parameters: block size of the neighbour kernels (until one is set, 64,
- * above 2^21 particle slots 256 for density and 128 for force) and
- * the density pass's XCD mapping: blocks go to the 8 XCDs in runs of
+/* Launch parameters: block size of the neighbour kernels (until one is set, 64;
+ * 256 in persistent mode; above 2^21 particle slots 128 for force, and 256 for
+ * density with 4 lanes a particle and a y/z split of 1 or 2) and the
+ * density pass's XCD mapping: blocks go to the 8 XCDs in runs of
  * xcd_remap consecutive blocks (default 128: neighbouring cells share an
  * XCD's L2; 0 or 1: plain round-robin order).  The force pass always uses
  * the plain order, which keeps the XCDs balanced when neighbour counts vary

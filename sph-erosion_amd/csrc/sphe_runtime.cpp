@@ -872,12 +872,27 @@ struct Timed {
 //             1,254 / 1,255, 256 scenes of 4.6M in all 810 / 796 / 781
 //   force     4,096 7.9 / 8.2 / 9.3, 48 uneven scenes 150 / 162 / 181, 262,144 56.7 /
 //             57.0 / 59.0, 1.5M 388 / 385 / 389; 4.2M 1,227 / 1,230 / 1,255, 256 scenes 754 /
-//             740 / 727
-int density_block(const sphe_ctx* c) { return c->block ? c->block : (c->D.P > kManySlots ? 256 : 64); }
+//             740 / 727: 128 lies between the two, within 2% of the better one on both
+// The density kernel of the other lane counts and of thirds of cells takes 64 at
+// every size (2.5M: one lane 1,776 / 2,133 / 2,134, two 993 / 1,025 / 1,211, eight
+// 737 / 746 / 747, thirds 1,016 / 1,037 / 1,152).  A persistent launch has as many
+// blocks as are resident, which take their work from eight queues, an atomic and
+// a barrier each time: more and smaller blocks only queue longer (4,096 particles:
+// density 97 / 95 / 92, force 47 / 46 / 45; 262,144: 399 / 242 / 168, 318 / 168 / 106;
+// 2.5M: 2,539 / 1,426 / 938, 2,528 / 1,456 / 911; with one lane a particle 324 / 294 /
+// 294 and 257 / 246 / 262 on the 262,144).
+int density_block(const sphe_ctx* c)
+{
+    if (c->block) return c->block;
+    if (c->persistent) return 256;
+    return c->D.P > kManySlots && c->lanes == 4 && c->yz <= 2 ? 256 : 64;
+}
 int force_block(const sphe_ctx* c)
 {
     if (c->fblock) return c->fblock;
-    return c->block ? c->block : (c->D.P > kManySlots ? 128 : 64);
+    if (c->block) return c->block;
+    if (c->persistent) return 256;
+    return c->D.P > kManySlots ? 128 : 64;
 }
 
 bool any_erosion(const sphe_ctx* c, int mode)

@@ -343,3 +343,25 @@ def test_inspection_after_a_change_of_parameters(change, precision):
     assert recs[0] == recs[1]
     ctx.step(1)
     ctx.particle(sid, 0)
+
+
+@pytest.mark.parametrize("n,lanes,split,persistent,density,force", [
+    (1000, 4, 2, False, 64, 64), (1000, 1, 2, False, 64, 64), (1000, 4, 3, False, 64, 64),
+    (1000, 4, 2, True, 256, 256), (1000, 8, 1, True, 256, 256),
+    (2 ** 21, 4, 2, False, 64, 64), (2 ** 21 + 1, 4, 2, False, 256, 128), (2 ** 21 + 1, 4, 3, False, 64, 128),
+    (2 ** 21 + 1, 2, 1, False, 64, 128), (2 ** 21 + 1, 4, 1, True, 256, 256)])
+def test_block_sizes_by_kernel_and_size(n, lanes, split, persistent, density, force):
+    """The block sizes in effect until some are set, by the kernels that serve
+    the context; one that is set is taken for all."""
+    ctx = sphe.Context()
+    ctx.set_yz_split(split)
+    ctx.set_lanes(lanes)
+    ctx.set_persistent(persistent)
+    sid = ctx.add_scene(_params(0.0457, 2.0))
+    ctx.set_particles(sid, np.linspace(-1.9, 1.9, 3 * n, dtype=np.float32).reshape(n, 3))
+    ctx.mass(sid)  # builds the layout; a line of this many particles is not stepped
+    assert (ctx.get_tuning()[0], ctx.get_force_block()) == (density, force)
+    ctx.set_tuning(512, 1)
+    assert (ctx.get_tuning()[0], ctx.get_force_block()) == (512, 512)
+    ctx.set_force_block(128)
+    assert (ctx.get_tuning()[0], ctx.get_force_block()) == (512, 128)
