@@ -366,10 +366,12 @@ int sphe_set_persistent(sphe_ctx* ctx, int on);
 int sphe_get_persistent(const sphe_ctx* ctx, int* on);
 /* Steps per captured graph launch of a long sphe_step call (1..4096,
  * default 32); the remaining steps of a call run one at a time, or as one
- * sequence from the second call with that remainder on.  The host reads the
- * list-overflow words between launches, so longer sequences grow the lists
- * later.  Results do not depend on it.  No counterpart in the reference (one
- * Run per frame, fluid_system.h:104-183). */
+ * sequence from the second call with that remainder on, for the first few
+ * remainders that come again (ten sequences in all under one launch plan) and
+ * not in calls before which the neighbour counts past the lists still rose.
+ * The host reads the list-overflow words between launches, so longer sequences
+ * grow the lists later.  Results do not depend on it.  No counterpart in the
+ * reference (one Run per frame, fluid_system.h:104-183). */
 int sphe_set_sequence_steps(sphe_ctx* ctx, int steps);
 int sphe_get_sequence_steps(const sphe_ctx* ctx, int* steps);
 /* Cells per scan tile of the sort's prefix sum: 2^log2_cells, 11..13

@@ -97,6 +97,8 @@ struct sphe_ctx {
     // calls by the length of what their whole sequences left over, under the
     // current plan: a length that comes again gets a sequence of its own
     std::map<int, int> rest_seen;
+    uint32_t ovf_seen = 0;  // the largest overflowing count published before the last call
+    bool grew = false;      // the lists grew since that call began
     // the list-overflow word as the last step sequence published it: host
     // memory mapped for the device (h_ovf_dev), written by a kernel at the
     // end of every sequence and read by the host without a stream wait
@@ -1109,6 +1111,7 @@ int grow_lists(sphe_ctx* c)
     HIPCHK(c, hipMemsetAsync(c->D.ovf, 0, 8, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     clear_published(c);
+    c->grew = true;
     return SPHE_OK;
 }
 
@@ -1118,12 +1121,13 @@ int grow_lists(sphe_ctx* c)
 const int kInFlight = 2;
 
 // Whether the `rest` steps that a call's whole sequences leave over run as one
-// captured sequence: a single step always, more from the second call with that
-// rest on, for up to kMaxSequences sequences in all (else one step at a time,
-// launched directly).  Between two one-step graphs the device idles for 13 us
-// (a tenth of a step of 100,000 particles) and between two direct steps for
-// 10; a capture costs the host about as much per step, once, which a call that
-// never comes again would not win back.
+// captured sequence: a call of a single step always, any other rest from the
+// second call with it on, for up to kMaxSequences sequences of a plan (none is
+// given up for another), else one step at a time, launched directly.  Between
+// two one-step graphs the device idles for 13 us (a tenth of a step of 100,000
+// particles) and between two direct steps for 10; a capture costs the host
+// about as much per step, once, which a call that never comes again would not
+// win back.
 const size_t kMaxSequences = 10;
 bool rest_as_sequence(sphe_ctx* c, int rest, bool first)
 {
@@ -1152,7 +1156,16 @@ int do_steps(sphe_ctx* c, int nsteps)
     const int rest = nsteps % c->seq_steps;
     const bool several = nsteps > c->seq_steps;
     if (graph) check_plan(c);
-    const bool rest_seq = graph && rest_as_sequence(c, rest, !several);
+    // while the largest count past the lists rises from call to call, or after
+    // a call in which they grew, lists may soon be too short: the rest goes one
+    // step at a time then, so that they grow two steps late and not a sequence
+    // late (a column of 110,592 falling onto its terrain, calls of 16 steps: 104
+    // -> 92 us a step in all, 570 -> 220 in the slowest call)
+    const uint32_t ovf = *(volatile uint32_t*)c->h_ovf;
+    const bool rising = ovf > c->ovf_seen || c->grew;
+    c->ovf_seen = ovf;
+    c->grew = false;
+    const bool rest_seq = graph && (rest == 1 || !rising) && rest_as_sequence(c, rest, !several);
     if (graph && several) sphe_launch_clear_status(c->D, c->stream);
     bool first = !(graph && several);
     for (int done = 0; done < nsteps;) {

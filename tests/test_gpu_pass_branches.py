@@ -365,3 +365,44 @@ def test_block_sizes_by_kernel_and_size(n, lanes, split, persistent, density, fo
     assert (ctx.get_tuning()[0], ctx.get_force_block()) == (512, 512)
     ctx.set_force_block(128)
     assert (ctx.get_tuning()[0], ctx.get_force_block()) == (512, 128)
+
+
+def test_lists_grow_within_a_call_while_counts_rise():
+    """A cluster that contracts (no forces): its counts pass the lists' 32
+    entries in the first call of 16 steps and list and overflow chunk (64) in
+    the second, more than two steps before its end.  The lists have grown when
+    the second call is done, as they do one step at a time."""
+    g = np.array([(a, b, c) for a in range(6) for b in range(6) for c in range(6)]) - 2.5
+    jitter = np.random.default_rng(21).uniform(-0.05, 0.05, g.shape)
+    cluster = (g + jitter) * 0.0235
+    # far neighbours, so that the pool has a chunk for every particle of the cluster
+    k = np.arange(2048)
+    far = np.stack([k // 256 * 0.07, k // 16 % 16 * 0.07, k % 16 * 0.07], 1) + (0.3, -0.5, -0.5)
+    pos = np.concatenate([cluster, far]).astype(np.float32)
+    vel = np.zeros_like(pos)
+    vel[:216] = -0.01 * pos[:216] / 1e-3
+    p = sphe.default_params(h=0.0457, mass=0.02, dt=1e-3, box_half=1.0, box_center=(0.0, 0.0, 0.0), stiffness=0.0,
+                            visc=0.0, surf_tens=0.0, gravity=(0.0, 0.0, 0.0))
+
+    def context():
+        ctx = sphe.Context()
+        ctx.set_list_capacity(32)
+        sid = ctx.add_scene(p)
+        ctx.set_particles(sid, pos, vel)
+        return ctx, sid
+    single, sid = context()
+    most = []
+    for _ in range(32):
+        single.step(1)
+        single.sync()
+        most.append(int(single.debug_neighbours(sid, csr=False)[0].max()) - 1)  # at the end of the step
+    assert most[0] <= 32 < most[14] and max(most[:15]) <= 64 < min(most[27:])
+    ctx, sid = context()
+    ctx.step(16)
+    ctx.sync()
+    assert ctx.get_list_capacity() == 32
+    ctx.step(16)
+    ctx.sync()
+    assert ctx.get_list_capacity() > 64
+    for a, b in zip(ctx.state_f64(sid), single.state_f64(sid)):
+        assert np.array_equal(a, b)
