@@ -2498,14 +2498,15 @@ __global__ __launch_bounds__(256) void k_fill_i32(int32_t* __restrict__ p, int64
     if (i < n) p[i] = v;
 }
 
-// id -> slot of the current state, for the scenes with a map.  UNIQUE: every
-// entry of the map belongs to one particle; otherwise the map was cleared to
-// INT32_MAX first, and duplicate ids keep their lowest slot.
+// id -> slot of the current state, for the scenes with a map among those at
+// slots p0 .. p1-1 (p0 a multiple of 64).  UNIQUE: every entry of the map
+// belongs to one particle; otherwise the map was cleared to INT32_MAX first,
+// and duplicate ids keep their lowest slot.
 template <bool UNIQUE>
-__global__ __launch_bounds__(256) void k_idmap(DevState D, int32_t* __restrict__ map)
+__global__ __launch_bounds__(256) void k_idmap(DevState D, int64_t p0, int64_t p1, int32_t* __restrict__ map)
 {
-    const int64_t slot = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (slot >= D.P) return;
+    const int64_t slot = p0 + (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (slot >= p1) return;
     const SceneDev& S = scene_ref(D, wave_scene(D.chunk_scene, slot));
     if (slot >= S.p_begin + S.n || S.idmap_off < 0) return;
     const int32_t id = D.u_id[slot];
@@ -3051,14 +3052,15 @@ void sphe_launch_inspect(const DevState& D, const int32_t* slotp, int lanes, boo
     }
 }
 
-void sphe_launch_idmap(const DevState& D, int32_t* map, int64_t len, bool unique, hipStream_t st)
+void sphe_launch_idmap(const DevState& D, int64_t p0, int64_t p1, int32_t* map, int64_t m0, int64_t m1, bool unique,
+                       hipStream_t st)
 {
-    if (D.P == 0 || len == 0) return;
+    if (p1 <= p0 || m1 <= m0) return;
     if (unique) {
-        k_idmap<true><<<grid_of(D.P, 256), 256, 0, st>>>(D, map);
+        k_idmap<true><<<grid_of(p1 - p0, 256), 256, 0, st>>>(D, p0, p1, map);
     } else {
-        k_fill_i32<<<grid_of(len, 256), 256, 0, st>>>(map, len, INT32_MAX);
-        k_idmap<false><<<grid_of(D.P, 256), 256, 0, st>>>(D, map);
+        k_fill_i32<<<grid_of(m1 - m0, 256), 256, 0, st>>>(map + m0, m1 - m0, INT32_MAX);
+        k_idmap<false><<<grid_of(p1 - p0, 256), 256, 0, st>>>(D, p0, p1, map);
     }
 }
 

@@ -30,9 +30,11 @@ void sphe_launch_terrain_mesh(const float* H, int nx, int nz, float cell, float 
 // memory) into out[0 .. 28]; out[22] = -1 when *slotp names no slot.  lists:
 // the neighbour lists are still the last step's.
 void sphe_launch_inspect(const DevState& D, const int32_t* slotp, int lanes, bool lists, double* out, hipStream_t st);
-// id -> slot map of the current state for the scenes that have one; unique:
-// every entry belongs to exactly one particle.
-void sphe_launch_idmap(const DevState& D, int32_t* map, int64_t len, bool unique, hipStream_t st);
+// id -> slot map of the current state for those of the scenes at slots p0 ..
+// p1-1 (whole scenes) that have one, entries m0 .. m1-1; unique: every entry of
+// these belongs to exactly one particle.
+void sphe_launch_idmap(const DevState& D, int64_t p0, int64_t p1, int32_t* map, int64_t m0, int64_t m1, bool unique,
+                       hipStream_t st);
 // Positions (what 0) or velocities (1) of the n particles at slots p0 ..
 // p0+n-1, whose ids are 0 .. n-1, as 3 floats at out[3 id]; their last
 // densities (2) as one float at out[id].

@@ -406,3 +406,52 @@ def test_lists_grow_within_a_call_while_counts_rise():
     assert ctx.get_list_capacity() > 64
     for a, b in zip(ctx.state_f64(sid), single.state_f64(sid)):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("filler", [0, 2 ** 20])
+@pytest.mark.parametrize("precision", [sphe.FP32, sphe.FP64])
+def test_reads_of_single_scenes_of_a_batch(precision, filler):
+    """Scenes of a batch read and inspected one by one, in other orders after
+    each step, a scene again before and after another's edit: the values of the
+    scene alone.  Among them are one particle, a whole wave, sparse ids, ids
+    with a gap and double ids.  The first scene read after a step is mapped by
+    itself, the first three in a context of 2^20 particles more, the next one
+    with all others."""
+    rng = np.random.default_rng(31)
+    sizes = (1, 64, 700, 333, 65, 1000)
+    ids = [None, None, np.arange(700) * 7, np.r_[0:100, 140:373], np.r_[0:40, 20:45], None]
+    poss = [rng.uniform(-0.15, 0.15, (n, 3)).astype(np.float32) for n in sizes]
+
+    def add(ctx, k):
+        sid = ctx.add_scene(_params(0.0457, 0.2, dt=1e-4))
+        ctx.set_particles(sid, poss[k], ids=None if ids[k] is None else ids[k].astype(np.int32))
+        return sid
+    batch = sphe.Context(precision)
+    sids = [add(batch, k) for k in range(6)]
+    if filler:
+        o = batch.add_scene(_params(0.0457, 3.0))
+        batch.set_particles(o, rng.uniform(-2.9, 2.9, (filler, 3)).astype(np.float32))
+    alone = []
+    for k in range(6):
+        ctx = sphe.Context(precision)
+        alone.append((ctx, add(ctx, k)))
+
+    def compare(k):
+        ctx, sid = alone[k]
+        i = 0 if ids[k] is None else int(ids[k][len(ids[k]) // 2])
+        assert bytes(batch.particle(sids[k], i)) == bytes(ctx.particle(sid, i))
+        for which in (sphe.BUF_POS, sphe.BUF_VEL, sphe.BUF_DENSITY):
+            assert np.array_equal(batch.read(sids[k], which), ctx.read(sid, which))
+    for order in ((5, 0, 1, 2), (4, 3, 5, 4), (1, 2, 0, 5, 3)):
+        batch.step(2)
+        for ctx, _ in alone:
+            ctx.step(2)
+        for k in order:
+            compare(k)
+    for ctx, sid in ((batch, sids[1]), alone[1]):
+        ctx.set_particles(sid, poss[1][::-1].copy())
+        ctx.step(1)
+    for k in (0, 2, 3, 4, 5):
+        alone[k][0].step(1)
+    for k in (3, 1, 5, 2, 0, 4):
+        compare(k)
