@@ -55,6 +55,12 @@ struct Scene {
     bool ids_dense = false;                 // the ids are 0 .. n-1 (the device gathers in id order)
 };
 
+// Mapped host memory of a context: the published words, and beside them room
+// for reads of up to 16,128 bytes (1,344 positions); kStageBytes for reads past
+// those from the first of them on (that read takes some 25 us more).  Every
+// context holding kStageBytes from its creation would pin them for nothing
+// where it reads little or nothing.
+const size_t kMappedBytes = 16 * 1024, kWordBytes = 256;
 const size_t kStageBytes = 256 * 1024;
 
 struct ProfRec {
@@ -105,10 +111,13 @@ struct sphe_ctx {
     // end of every sequence and read by the host without a stream wait
     uint32_t* h_ovf = nullptr;
     uint32_t* h_ovf_dev = nullptr;
-    // what small reads come back through (kStageBytes after the words above):
-    // kernels write it, the host copies from it once the stream is done
+    // what small reads come back through: kernels write it, the host copies
+    // from it once the stream is done (stage_for)
     char* h_stage = nullptr;
     char* h_stage_dev = nullptr;
+    size_t stage_bytes = 0;
+    bool stage_tried = false;  // kStageBytes were asked for
+    void* h_big = nullptr;
     // completion of the last launches (one event per launch slot): before a
     // launch the host waits for the one kInFlight launches back, so the
     // overflow word it reads is at most that many launches old
@@ -1345,7 +1354,7 @@ int sphe_create(int precision, sphe_ctx** out)
         return SPHE_EHIP;
     }
     void* h = nullptr;
-    if (hipHostMalloc(&h, 256 + kStageBytes, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
+    if (hipHostMalloc(&h, kMappedBytes, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
         hipHostGetDevicePointer((void**)&c->h_ovf_dev, h, 0) != hipSuccess) {
         (void)hipGetLastError();
         if (h) (void)hipHostFree(h);
@@ -1354,8 +1363,9 @@ int sphe_create(int precision, sphe_ctx** out)
         return SPHE_EHIP;
     }
     c->h_ovf = (uint32_t*)h;
-    c->h_stage = (char*)h + 256;
-    c->h_stage_dev = (char*)c->h_ovf_dev + 256;
+    c->h_stage = (char*)h + kWordBytes;
+    c->h_stage_dev = (char*)c->h_ovf_dev + kWordBytes;
+    c->stage_bytes = kMappedBytes - kWordBytes;
     clear_published(c);  // pinned memory may come back holding an earlier owner's words
     for (hipEvent_t& e : c->seq_ev) {
         if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
@@ -1391,6 +1401,7 @@ int sphe_destroy(sphe_ctx* c)
     for (hipEvent_t e : c->seq_ev)
         if (e) (void)hipEventDestroy(e);
     if (c->h_ovf) (void)hipHostFree(c->h_ovf);
+    if (c->h_big) (void)hipHostFree(c->h_big);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
     return SPHE_OK;
@@ -1657,6 +1668,27 @@ static int ensure_idmap(sphe_ctx* c, Scene* s)
     return SPHE_OK;
 }
 
+// Whether a read of that many bytes can come through the mapped memory.
+static bool stage_for(sphe_ctx* c, size_t bytes)
+{
+    if (bytes <= c->stage_bytes) return true;
+    if (bytes > kStageBytes || c->stage_tried) return false;
+    c->stage_tried = true;
+    void* h = nullptr;
+    void* d = nullptr;
+    if (hipHostMalloc(&h, kStageBytes, hipHostMallocMapped | hipHostMallocCoherent) != hipSuccess ||
+        hipHostGetDevicePointer(&d, h, 0) != hipSuccess) {
+        (void)hipGetLastError();
+        if (h) (void)hipHostFree(h);
+        return false;
+    }
+    c->h_big = h;
+    c->h_stage = (char*)h;
+    c->h_stage_dev = (char*)d;
+    c->stage_bytes = kStageBytes;
+    return true;
+}
+
 int sphe_read_buffer(sphe_ctx* c, int scene, int which, void* out, size_t bytes)
 {
     SCENE_OR_FAIL(s, c, scene);
@@ -1672,7 +1704,7 @@ int sphe_read_buffer(sphe_ctx* c, int scene, int which, void* out, size_t bytes)
         // and copy 4 bytes per value, with no host sync of the rest
         const int what = which == SPHE_BUF_POS ? FEED_POS : (state ? FEED_VEL : FEED_RHO);
         const size_t nbytes = n * comps * 4;
-        if (nbytes <= kStageBytes && s->idmap_off >= 0) {
+        if (s->idmap_off >= 0 && stage_for(c, nbytes)) {
             int r = ensure_device(c);
             if (!r) r = ensure_idmap(c, s);
             if (r) return r;

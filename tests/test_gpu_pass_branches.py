@@ -455,3 +455,27 @@ def test_reads_of_single_scenes_of_a_batch(precision, filler):
         alone[k][0].step(1)
     for k in (3, 1, 5, 2, 0, 4):
         compare(k)
+
+
+@pytest.mark.parametrize("precision", [sphe.FP32, sphe.FP64])
+def test_reads_at_the_edges_of_the_mapped_memory(precision):
+    """Sizes on both sides of what a context holds from its creation (16,128
+    bytes: 1,344 positions, 4,032 densities) and of what the first larger read
+    takes, the small after the large ones: the state's own values; records
+    between them."""
+    rng = np.random.default_rng(9)
+    ctx = sphe.Context(precision)
+    sids = []
+    for n in (1344, 1345, 4032, 4033, 21845, 21846):
+        sids.append(ctx.add_scene(_params(0.0457, 0.5)))
+        ctx.set_particles(sids[-1], rng.uniform(-0.45, 0.45, (n, 3)).astype(np.float32))
+    for order in ((0, 2, 1, 3, 4, 5), (5, 4, 3, 2, 1, 0)):
+        ctx.step(1)
+        got = {}
+        for k in order:
+            got[k] = [ctx.density(sids[k]), ctx.positions(sids[k]), ctx.velocities(sids[k])]
+            p = ctx.particle(sids[k], 1000)
+            assert p.Density == got[k][0][1000] and list(p.Position) == got[k][1][1000].tolist()
+        for k in order:
+            gp, gv = ctx.state_f64(sids[k])
+            assert np.array_equal(got[k][1], gp.astype(np.float32)) and np.array_equal(got[k][2], gv.astype(np.float32))
