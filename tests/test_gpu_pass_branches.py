@@ -479,3 +479,45 @@ def test_reads_at_the_edges_of_the_mapped_memory(precision):
         for k in order:
             gp, gv = ctx.state_f64(sids[k])
             assert np.array_equal(got[k][1], gp.astype(np.float32)) and np.array_equal(got[k][2], gv.astype(np.float32))
+
+
+@pytest.mark.parametrize("tiles", [4096, 4097])
+def test_marked_tiles_give_the_counted_ones_steps(tiles):
+    """Above 2^21 slots the tiles are only marked and their totals added up by
+    the scan: a scene of 2^21 - 64 particles, and a small one, step to the same
+    bits in such a context (of exactly that many tiles at first, so one launch
+    less or more) as alone, where the totals are counted; the tile size changes
+    between steps."""
+    h = 0.0457
+    n = 2 ** 21 - 64
+    k = np.arange(n)
+    rng = np.random.default_rng(4)
+    far = (np.stack([k >> 14, k >> 7 & 127, k & 127], 1) * 0.045 - 2.85).astype(np.float32)
+    near = rng.uniform(-0.12, 0.12, (2000, 3)).astype(np.float32)
+
+    def add(ctx, half, pos):
+        sid = ctx.add_scene(_params(h, half, dt=1e-4))
+        ctx.set_particles(sid, pos)
+        return sid
+    alone = []
+    for half, pos in ((2.9, far), (0.2, near)):
+        ctx = sphe.Context()
+        alone.append((ctx, add(ctx, half, pos)))
+    both = sphe.Context()
+    both.set_scan_tile(11)
+    sids = [add(both, 2.9, far), add(both, 0.2, near)]
+    left = 2048 * tiles - (_cells(_params(h, 2.9)) + 1) - (_cells(_params(h, 0.2)) + 1) - 1
+    for half in (0.4, 0.2, 0.1, 0.05, 0.01):
+        c = _cells(_params(h, half)) + 1
+        while left >= 2048 and c <= left:
+            left -= c
+            add(both, half, np.float32(0.4 * half) * np.array([[1, 1, 1], [-1, 1, 1], [1, -1, 1]], np.float32))
+    assert 0 <= left < 2048  # the last tile is partly filled
+    for log2 in (11, 12, 13, 11):
+        both.set_scan_tile(log2)
+        for ctx in [both] + [c for c, _ in alone]:
+            ctx.step(2)
+    assert both.status() == 0
+    for sid, (ctx, other) in zip(sids, alone):
+        for which in (sphe.BUF_POS, sphe.BUF_VEL, sphe.BUF_DENSITY):
+            assert np.array_equal(both.read(sid, which), ctx.read(other, which))
