@@ -82,11 +82,12 @@ struct DevState {
     int32_t* key; uint32_t* arank;      // cell key << sub_log2 | x slab, arrival rank in the cell
     uint64_t* tmp_kid; int32_t* tmp_src;  // scatter output: (key, id) packed, previous slot
     // counts per cell; and totals per scan tile of 2^scan_log2 cells, counted
-    // with them (totals; else marked and added up by the scan) and reset by the scatter (the scan reads the counts of tiles
-    // with any).  Neighbouring tiles' totals lie in different cache lines, 32
-    // words each, 2^tlog lines: waves that count at the same time are in
-    // neighbouring tiles, and atomics on one line wait for each other (tile_word).
-    // tpre: the totals' prefix in tile order, where there are many tiles.
+    // with them (totals; else marked, and added up by the scan) and reset when
+    // the scan is done with them (it reads the counts of tiles with any).
+    // Neighbouring tiles' totals lie in different cache lines, 32 words each,
+    // 2^tlog lines: waves that count at the same time are in neighbouring tiles,
+    // and atomics on one line wait for each other (tile_word).  tpre: the totals'
+    // prefix in tile order, at the same words, where there are many tiles.
     uint32_t* cnt; uint32_t* total; uint32_t* tpre; int64_t npartial;
     int32_t tlog, totals;
     // one word per scan tile of cells: the value every start of the tile

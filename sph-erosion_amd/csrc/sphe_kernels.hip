@@ -582,54 +582,68 @@ __device__ __forceinline__ void store4(uint2* __restrict__ p, int64_t i, int64_t
     }
 }
 
-// Exclusive prefix of the n tile totals by one block of 1,024
-// threads: chunks of 16,384 totals, 16 consecutive ones per thread, one block
-// scan per chunk and the running total carried to the next chunk.  Linear in
-// the number of tiles; each scan-down block then reads its tile's prefix
-// with one load.
+// Exclusive prefix, in tile order, of the 32 2^tlog words of the tiles' totals,
+// word by word (tile_word's order), by one block of 1,024 threads.  A line has
+// one tile of each of 32 runs of 2^tlog tiles: thread (q, g) adds up the words
+// 4 q .. 4 q + 3 of its 2^tlog / 128 consecutive lines, a scan over the 32 runs'
+// 128 sums each gives where it starts, and a second pass over its lines leaves
+// the prefixes.  So lines are read and written whole (scan of 1,000 particles in
+// 360M cells, 88,000 tiles: 63 us; 129 with 16 consecutive tiles to a thread,
+// each from a line of its own).  tlog >= 8.
 __global__ __launch_bounds__(1024) void k_scan_tiles(const uint32_t* __restrict__ total, int tlog,
-                                                     uint32_t* __restrict__ pre, int64_t n)
+                                                     uint32_t* __restrict__ pre)
 {
-    constexpr int ITEMS = 16;
-    __shared__ uint32_t lds[16];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    uint32_t carry = 0;
-    for (int64_t c0 = 0; c0 < n; c0 += 1024 * ITEMS) {
-        const int64_t base = c0 + (int64_t)threadIdx.x * ITEMS;
-        uint32_t v[ITEMS];
+    __shared__ __attribute__((aligned(16))) uint32_t sums[32 * 128];
+    __shared__ uint32_t waves[16];
+    const int q = threadIdx.x & 7, g = threadIdx.x >> 3, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lines = 1 << (tlog - 7);  // at least 2
+    const uint4* src = (const uint4*)total + ((int64_t)g * lines * 8 + q);
+    uint4* dst = (uint4*)pre + ((int64_t)g * lines * 8 + q);
+    // calls f(line, words) for the thread's lines, eight or two loads in flight
+    auto each = [&](auto&& f) {
+        auto run = [&](auto count) {
+            constexpr int U = decltype(count)::value;
+            for (int i = 0; i < lines; i += U) {
+                uint4 v[U];
 #pragma unroll
-        for (int i = 0; i < ITEMS; ++i) v[i] = base + i < n ? total[tile_word(tlog, (uint32_t)(base + i))] : 0u;
-        uint32_t s = 0;
+                for (int u = 0; u < U; ++u) v[u] = src[(i + u) * 8];
 #pragma unroll
-        for (int i = 0; i < ITEMS; ++i) s += v[i];
-        const uint32_t x = wave_sums(s);  // over the wave, then the 16 wave totals
-        if (lane == 63) lds[wave] = x;
-        __syncthreads();
-        uint32_t before = 0, tot = 0;
+                for (int u = 0; u < U; ++u) f(i + u, v[u]);
+            }
+        };
+        if (lines >= 8) run(std::integral_constant<int, 8>());
+        else run(std::integral_constant<int, 2>());
+    };
+    uint4 s = make_uint4(0u, 0u, 0u, 0u);
+    each([&](int, const uint4& v) { s = make_uint4(s.x + v.x, s.y + v.y, s.z + v.z, s.w + v.w); });
+    uint32_t* const mine = sums + 4 * q * 128 + g;
+    mine[0] = s.x;
+    mine[128] = s.y;
+    mine[256] = s.z;
+    mine[384] = s.w;
+    __syncthreads();
+    uint4 t = ((const uint4*)sums)[threadIdx.x];
+    const uint32_t all = (t.x + t.y) + (t.z + t.w);
+    const uint32_t x = wave_sums(all);  // over the wave, then the 16 wave totals
+    if (lane == 63) waves[wave] = x;
+    __syncthreads();
+    uint32_t at = x - all;
 #pragma unroll
-        for (int k = 0; k < 16; ++k) {
-            const uint32_t t = lds[k];
-            if (k < wave) before += t;
-            tot += t;
-        }
-        uint32_t run = carry + before + (x - s);
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i) {
-            const uint32_t c = v[i];
-            v[i] = run;
-            run += c;
-        }
-#pragma unroll
-        for (int i = 0; i < ITEMS; ++i)
-            if (base + i < n) pre[base + i] = v[i];
-        carry += tot;
-        __syncthreads();  // the wave totals of the next chunk reuse lds
-    }
+    for (int k = 0; k < 16; ++k) at += k < wave ? waves[k] : 0u;
+    t = make_uint4(at, at + t.x, at + t.x + t.y, at + t.x + t.y + t.z);
+    ((uint4*)sums)[threadIdx.x] = t;
+    __syncthreads();
+    uint4 r = make_uint4(mine[0], mine[128], mine[256], mine[384]);
+    each([&](int i, const uint4& v) {
+        dst[i * 8] = r;
+        r = make_uint4(r.x + v.x, r.y + v.y, r.z + v.z, r.w + v.w);
+    });
 }
 
 // Where a tile's prefix (the total of the tiles before it) comes from: a word
 // that k_scan_tiles left, or the tiles' totals, added here by every block: up
-// to SCAN_SUM_TILES tiles, at most 8 loads a thread, while a launch costs 4 us.  The totals themselves are counted
+// to SCAN_SUM_TILES tiles, at most four loads a thread, while a launch costs 4
+// us.  The totals themselves are counted
 // with the particles (count_key; a pass over the counts for them took a launch:
 // 13.2 -> 7.3 us on 6.7M cells, 19.6 -> 13.8 for 96 scenes with their terrain
 // heights; for few tiles every block added the counts before its tile: 5.6 ->
@@ -637,16 +651,22 @@ __global__ __launch_bounds__(1024) void k_scan_tiles(const uint32_t* __restrict_
 // of each thread's own 64 or 128 bytes: 57 -> 40 us on 16.7M cells, before that.
 enum { SCAN_PREFIX, SCAN_SUMS };
 #define SPHE_SCAN_SUM_TILES 4096
+__host__ __device__ inline int64_t scan_tiles(const DevState& D)
+{
+    return (D.C + 1 + (1ll << D.scan_log2) - 1) >> D.scan_log2;
+}
+__host__ __device__ inline bool scan_sums(const DevState& D) { return scan_tiles(D) <= SPHE_SCAN_SUM_TILES; }
 
 // start = exclusive prefix of the counts of one tile (each cell's first scatter
-// resets its count, and the scatter the tiles' totals, for the next arrivals).
+// resets its count for the next arrivals; the tile's total is reset here where
+// no other block reads it, else by the scatter: scan_sums).
 // A tile whose total is 0 holds only zero counts, which are not read.  fill:
 // per tile, the value all of an empty tile's starts hold since the tile was
 // last written empty (~0: not known); an empty tile whose prefix equals it is
 // not written again.
 template <int ITEMS, int FROM>
 __device__ __forceinline__ void scan_down_tile(const uint32_t* __restrict__ cnt, uint2* __restrict__ start, int64_t n,
-                                               const uint32_t* __restrict__ total, int tlog,
+                                               uint32_t* __restrict__ total, int tlog,
                                                const uint32_t* __restrict__ tpre,
                                                uint32_t* __restrict__ fill, int tile, uint32_t* lds)
 {
@@ -662,7 +682,7 @@ __device__ __forceinline__ void scan_down_tile(const uint32_t* __restrict__ cnt,
     }
     uint32_t pre = 0;  // this thread's share of the prefix
     if constexpr (FROM == SCAN_PREFIX) {
-        pre = threadIdx.x == 0 ? tpre[tile] : 0u;
+        pre = threadIdx.x == 0 ? tpre[tile_word(tlog, (uint32_t)tile)] : 0u;
     } else {
         // in the order of the words, so that they are read as lines
 #pragma unroll 2
@@ -705,10 +725,11 @@ __device__ __forceinline__ void scan_down_tile(const uint32_t* __restrict__ cnt,
             store4(start, tile_cell<ITEMS>(tile, c), n, o);
         }
     }
-    // every thread read the fill word before the barrier
+    // every thread read the total and the fill word before the barrier
     if (threadIdx.x == 0) {
         const uint32_t nf = empty ? ptot : ~0u;
         if (nf != filled) fill[tile] = nf;
+        if (FROM == SCAN_PREFIX && !empty) total[tile_word(tlog, (uint32_t)tile)] = 0u;
     }
 }
 
@@ -716,7 +737,8 @@ __global__ __launch_bounds__(256) void k_scatter(DevState D)
 {
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     // the tiles' totals are used up
-    for (int64_t w = p; w < (32ll << D.tlog); w += (int64_t)gridDim.x * blockDim.x) D.total[w] = 0u;
+    if (scan_sums(D))
+        for (int64_t w = p; w < (32ll << D.tlog); w += (int64_t)gridDim.x * blockDim.x) D.total[w] = 0u;
     if (p >= D.P) return;
     const int32_t key = D.key[p];  // cell key << sub_log2 | slab
     const int32_t c = key >> D.sub_log2;
@@ -2894,14 +2916,15 @@ void sphe_launch_hash(const DevState& D, hipStream_t st, hipEvent_t e0, hipEvent
 template <int ITEMS>
 static void launch_scan_cells_t(const DevState& D, bool heights, int first, hipStream_t st, hipEvent_t e0, hipEvent_t e1)
 {
-    const int nb = (int)((D.C + 1 + 256 * ITEMS - 1) / (256 * ITEMS));
+    const int nb = (int)scan_tiles(D);
     const int nh = heights ? (int)grid_of(D.TC / 4, 256) : 0;  // TC: a multiple of 64
     if (!D.totals) klaunch(k_scan_reduce_cells<ITEMS>, nb, 256, st, e0, nullptr, D);
-    if (nb <= SPHE_SCAN_SUM_TILES) {
+    if (scan_sums(D)) {
         klaunch(k_scan_cells<ITEMS, SCAN_SUMS>, nb + nh, 256, st, D.totals ? e0 : nullptr, e1, D, nb, first);
         return;
     }
-    klaunch(k_scan_tiles, 1, 1024, st, D.totals ? e0 : nullptr, nullptr, (const uint32_t*)D.total, D.tlog, D.tpre, (int64_t)nb);
+    klaunch(k_scan_tiles, 1, 1024, st, D.totals ? e0 : nullptr, nullptr, (const uint32_t*)D.total, D.tlog,
+            D.tpre);
     klaunch(k_scan_cells<ITEMS, SCAN_PREFIX>, nb + nh, 256, st, nullptr, e1, D, nb, first);
 }
 

@@ -590,7 +590,7 @@ int build_layout(sphe_ctx* c)
     // 4.15, the scan 6 us less; 4.2M: 1,243 us against 1,236, 6 us less)
     D.totals = P <= kManySlots;
     DALLOC(D.total, (size_t)(32ll << tile_log(D.npartial)) * 4);  // room for every tile size
-    DALLOC(D.tpre, (size_t)D.npartial * 4);
+    DALLOC(D.tpre, (size_t)(32ll << tile_log(D.npartial)) * 4);
     DALLOC(D.tfill, (size_t)D.npartial * 4);
     DALLOC(D.vol, (size_t)TC * 8);
     DALLOC(D.height, (size_t)TC * 4);

@@ -521,3 +521,44 @@ def test_marked_tiles_give_the_counted_ones_steps(tiles):
     for sid, (ctx, other) in zip(sids, alone):
         for which in (sphe.BUF_POS, sphe.BUF_VEL, sphe.BUF_DENSITY):
             assert np.array_equal(both.read(sid, which), ctx.read(other, which))
+
+
+@pytest.mark.parametrize("tiles", [4097, 8192, 8193, 16385, 40000])
+def test_prefix_of_many_tiles(tiles):
+    """More than 4,096 tiles get their prefixes from a launch of its own, which
+    reads the totals by lines: 2 lines a thread up to 8,192 tiles, 4 to 16,384,
+    then 8 and more.  The same scene over the first cells, the last ones and some
+    between steps to the bits of the scene alone, while far tiles fill and empty."""
+    h = 0.0457
+    p = _params(h, 0.2, dt=1e-4)
+    pos = np.random.default_rng(11).uniform(-0.12, 0.12, (2000, 3)).astype(np.float32)
+    three = np.array([[1, 1, 1], [-1, 1, 1], [1, -1, 1]], np.float32)
+
+    def probe(ctx):
+        sid = ctx.add_scene(p)
+        ctx.set_particles(sid, pos)
+        return sid
+    alone = sphe.Context()
+    s0 = probe(alone)
+    ctx = sphe.Context()
+    ctx.set_scan_tile(11)
+    cells = {half: _cells(_params(h, half)) + 1 for half in (2.9, 1.0, 0.4, 0.2, 0.1, 0.05, 0.01)}
+    sids = [probe(ctx)]
+    left = 2048 * tiles - 1 - 4 * cells[0.2]
+    for half in sorted(cells, reverse=True):
+        while left >= 2048 and cells[half] <= left:
+            left -= cells[half]
+            o = ctx.add_scene(_params(h, half, dt=1e-4))
+            ctx.set_particles(o, np.float32(0.4 * half) * three)
+            if len(sids) < 3 and left < 2048 * tiles // (1 + len(sids)):
+                sids.append(probe(ctx))
+    while len(sids) < 4:
+        sids.append(probe(ctx))
+    assert 0 <= left < 2048  # the last tile is partly filled
+    for k in (1, 5):
+        ctx.step(k)
+        alone.step(k)
+        for sid in sids:
+            for which in (sphe.BUF_POS, sphe.BUF_VEL, sphe.BUF_DENSITY):
+                assert np.array_equal(ctx.read(sid, which), alone.read(s0, which))
+    assert ctx.status() == 0
