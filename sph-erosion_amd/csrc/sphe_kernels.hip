@@ -473,8 +473,8 @@ __device__ __forceinline__ uint32_t tile_word(int tlog, uint32_t t) { return ((t
 __device__ __forceinline__ uint32_t word_tile(int tlog, uint32_t w) { return ((w & 31u) << tlog) | (w >> 5); }
 
 // Counts a particle of that key into its scan tile and its cell: its rank of
-// arrival in the cell.  In the largest contexts (D.totals 0) the tile is only
-// marked.  The lanes that count here together are mostly neighbours of one
+// arrival in the cell.  In the largest contexts and those of many particles a
+// tile (D.totals 0) the tile is only marked.  The lanes that count here together are mostly neighbours of one
 // tile, which takes one atomic of the wave then (with the
 // totals in tile order, and so on a few lines, the force pass took 77 us instead
 // of 57 for 262,144 particles, and 289 instead of 155 for 48 uneven scenes).
@@ -647,7 +647,7 @@ __global__ __launch_bounds__(1024) void k_scan_tiles(const uint32_t* __restrict_
 // with the particles (count_key; a pass over the counts for them took a launch:
 // 13.2 -> 7.3 us on 6.7M cells, 19.6 -> 13.8 for 96 scenes with their terrain
 // heights; for few tiles every block added the counts before its tile: 5.6 ->
-// 4.2 us on 39,000 cells), except in the largest contexts (build_layout).  Runs of consecutive lines instead
+// 4.2 us on 39,000 cells), except where the atomics cost more (count_totals).  Runs of consecutive lines instead
 // of each thread's own 64 or 128 bytes: 57 -> 40 us on 16.7M cells, before that.
 enum { SCAN_PREFIX, SCAN_SUMS };
 #define SPHE_SCAN_SUM_TILES 4096

@@ -511,6 +511,18 @@ int tile_log(int64_t tiles)
 
 int64_t scan_tiles(int64_t C, int log2_cells) { return (C + 1 + (1ll << log2_cells) - 1) >> log2_cells; }
 
+// Whether the particles are counted into the scan's tiles (one atomic a wave
+// and tile, and no launch to add the totals up), or only mark them.  Many waves
+// to a tile queue for its word, many slots for the memory system.  Counted /
+// marked, us a step:
+//   1 tile    4,000 particles 27.6 / 28.0, 8,000 34.0 / 31.7, 32,000 91.7 / 79.1
+//   2 tiles   4,000 24.5 / 25.7, 8,000 27.5 / 27.4, 16,000 33.8 / 31.0, 64,000 98.8 / 79.6
+//   6 tiles   8,000 23.5 / 25.0, 16,000 27.1 / 27.7, 32,000 36.0 / 33.4, 128,000 121 / 102
+// so up to 4,096 particles a tile; and above 2^21 slots the force pass loses
+// more than the launch takes (13.95M particles: 4.37 ms against 4.15, the scan
+// 6 us less; 4.2M: 1,243 us against 1,236, 6 us less).
+bool count_totals(int64_t P, int64_t tiles) { return P <= kManySlots && P <= 4096 * tiles; }
+
 int build_layout(sphe_ctx* c)
 {
     free_device(c);
@@ -585,10 +597,7 @@ int build_layout(sphe_ctx* c)
     while (D.sub_log2 > 0 && (C << D.sub_log2) > INT32_MAX) --D.sub_log2;  // keys are int32
     D.npartial = sphe_scan_partials(C + 1);
     D.tlog = tile_log(scan_tiles(C, D.scan_log2));
-    // above 2^21 slots the atomics on the totals cost the force pass more than
-    // the launch that adds them up (13.95M particles: force 4.37 ms against
-    // 4.15, the scan 6 us less; 4.2M: 1,243 us against 1,236, 6 us less)
-    D.totals = P <= kManySlots;
+    D.totals = count_totals(P, scan_tiles(C, D.scan_log2));
     DALLOC(D.total, (size_t)(32ll << tile_log(D.npartial)) * 4);  // room for every tile size
     DALLOC(D.tpre, (size_t)(32ll << tile_log(D.npartial)) * 4);
     DALLOC(D.tfill, (size_t)D.npartial * 4);
@@ -964,12 +973,12 @@ std::string plan_signature(const sphe_ctx* c)
 {
     // everything the captured kernels take by value (DevState) or as launch shape
     char b[384];
-    snprintf(b, sizeof(b), "%d/%d/%d/%d/%d/%lld/%lld/%lld/%d/%d/%p/%p/%p/%d/%d/%d/%d/%lld/%d/%d/%d",
+    snprintf(b, sizeof(b), "%d/%d/%d/%d/%d/%lld/%lld/%lld/%d/%d/%p/%p/%p/%d/%d/%d/%d/%lld/%d/%d/%d/%d",
              c->precision, density_block(c), force_block(c), c->remap,
              c->lanes, (long long)c->D.P, (long long)c->D.C, (long long)c->D.TC, (int)any_erosion(c, -1),
              (int)any_erosion(c, SPHE_EROSION_TWO_PHASE), (const void*)c->D.u_pos, (const void*)c->D.nbl,
              (const void*)c->D.pool, c->D.maxn, c->D.sub_log2, c->D.yz, c->D.ocap, (long long)c->D.pool_cap,
-             c->D.scan_log2, c->D.persistent, c->D.h_unit);
+             c->D.scan_log2, c->D.totals, c->D.persistent, c->D.h_unit);
     return b;
 }
 
@@ -2431,6 +2440,7 @@ int sphe_set_scan_tile(sphe_ctx* c, int log2_cells)
     HIPCHK(c, hipStreamSynchronize(c->stream));
     c->D.scan_log2 = log2_cells;
     c->D.tlog = tile_log(scan_tiles(c->D.C, log2_cells));
+    c->D.totals = count_totals(c->D.P, scan_tiles(c->D.C, log2_cells));
     c->counted = false;
     return SPHE_OK;
 }

@@ -562,3 +562,28 @@ def test_prefix_of_many_tiles(tiles):
             for which in (sphe.BUF_POS, sphe.BUF_VEL, sphe.BUF_DENSITY):
                 assert np.array_equal(ctx.read(sid, which), alone.read(s0, which))
     assert ctx.status() == 0
+
+
+@pytest.mark.parametrize("precision", [sphe.FP32, sphe.FP64])
+@pytest.mark.parametrize("n", [4096, 4097, 8192, 8193, 20000])
+def test_many_particles_a_tile(n, precision):
+    """More than 4,096 particles to a scan tile only mark it: a scene over one or
+    two tiles steps to the same bits as beside an empty scene of many tiles,
+    where the particles are counted; the tile size changes between steps."""
+    h = 0.0457
+    pos = np.random.default_rng(n).uniform(-0.19, 0.19, (n, 3)).astype(np.float32)
+    ctxs = []
+    for wide in (False, True):
+        ctx = sphe.Context(precision)
+        sid = ctx.add_scene(_params(h, 0.2, dt=1e-5))
+        ctx.set_particles(sid, pos)
+        if wide:
+            ctx.add_scene(_params(h, 1.0))
+        ctxs.append(ctx)
+    for log2 in (12, 11, 13, 12):
+        for ctx in ctxs:
+            ctx.set_scan_tile(log2)
+            ctx.step(3)
+    for a, b in zip(ctxs[0].state_f64(sid), ctxs[1].state_f64(sid)):
+        assert np.array_equal(a, b)
+    assert ctxs[0].status() == 0
