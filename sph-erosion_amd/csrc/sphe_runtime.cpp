@@ -204,6 +204,31 @@ int fail(sphe_ctx* c, int code, const char* fmt, ...)
         if (e_ != hipSuccess) return fail((ctx), SPHE_EHIP, "%s: %s", #expr, hipGetErrorString(e_)); \
     } while (0)
 
+// Copies between host and device through the context's own stream: one on the
+// legacy stream fails, and breaks the capture, while another thread's context
+// captures a step sequence.
+struct Copies {
+    sphe_ctx* c;
+    hipError_t e = hipSuccess;
+    void add(void* dst, const void* src, size_t bytes, hipMemcpyKind kind)
+    {
+        if (e == hipSuccess && bytes > 0) e = hipMemcpyAsync(dst, src, bytes, kind, c->stream);
+    }
+    // waits for all of them, whether or not one failed: the host memory is free then
+    hipError_t done()
+    {
+        const hipError_t w = hipStreamSynchronize(c->stream);
+        return e == hipSuccess ? w : e;
+    }
+};
+
+hipError_t copy_now(sphe_ctx* c, void* dst, const void* src, size_t bytes, hipMemcpyKind kind)
+{
+    Copies q{c};
+    q.add(dst, src, bytes, kind);
+    return q.done();
+}
+
 inline int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 
 // hipMalloc that leaves no error behind when it fails: the runtime keeps a
@@ -696,10 +721,12 @@ int upload_t(sphe_ctx* c)
         std::vector<int32_t> id;
         pack_particles<T>(s, s.p_cap, p4, v4, sd, id);
         const size_t off = (size_t)s.p_begin;
-        HIPCHK(c, hipMemcpy((T*)D.u_pos + 4 * off, p4.data(), p4.size() * sizeof(T), hipMemcpyHostToDevice));
-        HIPCHK(c, hipMemcpy((T*)D.u_vel + 4 * off, v4.data(), v4.size() * sizeof(T), hipMemcpyHostToDevice));
-        HIPCHK(c, hipMemcpy(D.u_sed + off, sd.data(), sd.size() * 8, hipMemcpyHostToDevice));
-        HIPCHK(c, hipMemcpy(D.u_id + off, id.data(), id.size() * 4, hipMemcpyHostToDevice));
+        Copies q{c};
+        q.add((T*)D.u_pos + 4 * off, p4.data(), p4.size() * sizeof(T), hipMemcpyHostToDevice);
+        q.add((T*)D.u_vel + 4 * off, v4.data(), v4.size() * sizeof(T), hipMemcpyHostToDevice);
+        q.add(D.u_sed + off, sd.data(), sd.size() * 8, hipMemcpyHostToDevice);
+        q.add(D.u_id + off, id.data(), id.size() * 4, hipMemcpyHostToDevice);
+        HIPCHK(c, q.done());
     }
     return SPHE_OK;
 }
@@ -708,15 +735,13 @@ int upload_table(sphe_ctx* c, bool force);
 
 int upload(sphe_ctx* c)
 {
-    HIPCHK(c, hipStreamSynchronize(c->stream));
     int r = c->precision == SPHE_FP64 ? upload_t<double>(c) : upload_t<float>(c);
     if (r) return r;
     DevState& D = c->D;
-    for (const Scene& s : c->scenes) {
-        const size_t nt = (size_t)s.tnx * s.tnz;
-        if (nt == 0) continue;
-        HIPCHK(c, hipMemcpy(D.vol + s.t_off, s.vol.data(), nt * 8, hipMemcpyHostToDevice));
-    }
+    Copies q{c};
+    for (const Scene& s : c->scenes)
+        q.add(D.vol + s.t_off, s.vol.data(), (size_t)s.tnx * s.tnz * 8, hipMemcpyHostToDevice);
+    HIPCHK(c, q.done());
     r = upload_table(c, true);
     if (r) return r;
     sphe_launch_heights(D, c->stream);
@@ -742,10 +767,12 @@ int download_t(sphe_ctx* c)
         std::vector<int64_t> sd(n);
         std::vector<int32_t> id(n);
         const size_t off = (size_t)s.p_begin;
-        HIPCHK(c, hipMemcpy(p4.data(), (T*)D.u_pos + 4 * off, p4.size() * sizeof(T), hipMemcpyDeviceToHost));
-        HIPCHK(c, hipMemcpy(v4.data(), (T*)D.u_vel + 4 * off, v4.size() * sizeof(T), hipMemcpyDeviceToHost));
-        HIPCHK(c, hipMemcpy(sd.data(), D.u_sed + off, n * 8, hipMemcpyDeviceToHost));
-        HIPCHK(c, hipMemcpy(id.data(), D.u_id + off, n * 4, hipMemcpyDeviceToHost));
+        Copies q{c};
+        q.add(p4.data(), (T*)D.u_pos + 4 * off, p4.size() * sizeof(T), hipMemcpyDeviceToHost);
+        q.add(v4.data(), (T*)D.u_vel + 4 * off, v4.size() * sizeof(T), hipMemcpyDeviceToHost);
+        q.add(sd.data(), D.u_sed + off, n * 8, hipMemcpyDeviceToHost);
+        q.add(id.data(), D.u_id + off, n * 4, hipMemcpyDeviceToHost);
+        HIPCHK(c, q.done());
         for (size_t i = 0; i < n; ++i) {
             for (int a = 0; a < 3; ++a) {
                 s.pos[3 * i + a] = (double)p4[4 * i + a];
@@ -762,14 +789,12 @@ int download_t(sphe_ctx* c)
 int sync_to_host(sphe_ctx* c)
 {
     if (c->host_valid) return SPHE_OK;
-    HIPCHK(c, hipStreamSynchronize(c->stream));
     int r = c->precision == SPHE_FP64 ? download_t<double>(c) : download_t<float>(c);
     if (r) return r;
-    for (Scene& s : c->scenes) {
-        const size_t nt = (size_t)s.tnx * s.tnz;
-        if (nt == 0) continue;
-        HIPCHK(c, hipMemcpy(s.vol.data(), c->D.vol + s.t_off, nt * 8, hipMemcpyDeviceToHost));
-    }
+    Copies q{c};
+    for (Scene& s : c->scenes)
+        q.add(s.vol.data(), c->D.vol + s.t_off, (size_t)s.tnx * s.tnz * 8, hipMemcpyDeviceToHost);
+    HIPCHK(c, q.done());
     c->host_valid = true;
     return SPHE_OK;
 }
@@ -1118,8 +1143,8 @@ int grow_lists(sphe_ctx* c)
     HIPCHK(c, hipStreamSynchronize(c->stream));
     uint32_t w[2] = {0, 0};
     unsigned long long claimed = 0;
-    HIPCHK(c, hipMemcpy(w, c->D.ovf, 8, hipMemcpyDeviceToHost));
-    HIPCHK(c, hipMemcpy(&claimed, c->D.ptop, 8, hipMemcpyDeviceToHost));
+    HIPCHK(c, copy_now(c, w, c->D.ovf, 8, hipMemcpyDeviceToHost));
+    HIPCHK(c, copy_now(c, &claimed, c->D.ptop, 8, hipMemcpyDeviceToHost));
     const int64_t need = std::max<int64_t>(w[0], seen);
     const int64_t fails = std::max<int64_t>(w[1], failed);
     auto up = [](int64_t x, int64_t m) { return (x + m - 1) / m * m; };
@@ -1612,15 +1637,14 @@ static int read_rho(sphe_ctx* c, Scene& s, std::vector<double>& rho)
     const size_t n = s.ids.size();
     rho.assign(n, 0.0);
     if (!c->stepped || n == 0) return SPHE_OK;
-    HIPCHK(c, hipStreamSynchronize(c->stream));
     std::vector<int32_t> id(n);
-    HIPCHK(c, hipMemcpy(id.data(), c->D.s_id + s.p_begin, n * 4, hipMemcpyDeviceToHost));
+    HIPCHK(c, copy_now(c, id.data(), c->D.s_id + s.p_begin, n * 4, hipMemcpyDeviceToHost));
     std::vector<double> r(n);
     if (c->precision == SPHE_FP64) {
-        HIPCHK(c, hipMemcpy(r.data(), (double*)c->D.rho + s.p_begin, n * 8, hipMemcpyDeviceToHost));
+        HIPCHK(c, copy_now(c, r.data(), (double*)c->D.rho + s.p_begin, n * 8, hipMemcpyDeviceToHost));
     } else {
         std::vector<float> rf(n);
-        HIPCHK(c, hipMemcpy(rf.data(), (float*)c->D.rho + s.p_begin, n * 4, hipMemcpyDeviceToHost));
+        HIPCHK(c, copy_now(c, rf.data(), (float*)c->D.rho + s.p_begin, n * 4, hipMemcpyDeviceToHost));
         for (size_t i = 0; i < n; ++i) r[i] = rf[i];
     }
     std::vector<size_t> perm(n);
@@ -1664,8 +1688,8 @@ static int ensure_idmap(sphe_ctx* c, Scene* s)
 {
     if (s->idmap_state == c->state_no || c->idmap_all == c->state_no) return SPHE_OK;
     if (c->idmap_single <= c->D.P >> 19) {
-        sphe_launch_idmap(c->D, s->p_begin, s->p_begin + s->p_cap, c->d_idmap, s->idmap_off, s->idmap_off + s->idmap_len,
-                          s->ids_dense, c->stream);
+        sphe_launch_idmap(c->D, s->p_begin, s->p_begin + s->p_cap, c->d_idmap, s->idmap_off,
+                          s->idmap_off + s->idmap_len, s->ids_dense, c->stream);
         HIPCHK(c, hipGetLastError());
         s->idmap_state = c->state_no;
         ++c->idmap_single;
@@ -1959,8 +1983,7 @@ int sphe_terrain_heights(sphe_ctx* c, int scene, float* out, size_t count)
     int r = ensure_device(c);
     if (!r) r = ensure_heights(c);
     if (r) return r;
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    HIPCHK(c, hipMemcpy(out, c->D.height + s->t_off, nt * 4, hipMemcpyDeviceToHost));
+    HIPCHK(c, copy_now(c, out, c->D.height + s->t_off, nt * 4, hipMemcpyDeviceToHost));
     return SPHE_OK;
 }
 
@@ -2012,7 +2035,7 @@ int sphe_terrain_mesh(sphe_ctx* c, int scene, float* verts, size_t* nverts, uint
             float* d = nullptr;
             int r = mesh_on_device(c, s, &d);
             if (r) return r;
-            HIPCHK(c, hipMemcpy(verts, d, nv * 4, hipMemcpyDeviceToHost));
+            HIPCHK(c, copy_now(c, verts, d, nv * 4, hipMemcpyDeviceToHost));
         }
         *nverts = nv;
     }
@@ -2778,7 +2801,7 @@ int sphe_debug_neighbours(sphe_ctx* c, int scene, int32_t* counts, const int64_t
     const size_t n = s->ids.size();
     if (n == 0) return SPHE_OK;
     std::vector<int32_t> sid(n), cnt(n);
-    HIPCHK(c, hipMemcpy(sid.data(), c->D.s_id + s->p_begin, n * 4, hipMemcpyDeviceToHost));
+    HIPCHK(c, copy_now(c, sid.data(), c->D.s_id + s->p_begin, n * 4, hipMemcpyDeviceToHost));
     int32_t* dcnt = nullptr;
     HIPCHK(c, try_malloc(&dcnt, n * 4));
     sphe_launch_neighbours(c->D, scene, nullptr, dcnt, nullptr, c->stream);
@@ -2802,7 +2825,7 @@ int sphe_debug_neighbours(sphe_ctx* c, int scene, int32_t* counts, const int64_t
     int32_t* didx = nullptr;
     e = try_malloc(&doff, (n + 1) * 8);
     if (e == hipSuccess) e = try_malloc(&didx, (size_t)std::max<int64_t>(1, soff[n]) * 4);
-    if (e == hipSuccess) e = hipMemcpy(doff, soff.data(), (n + 1) * 8, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = copy_now(c, doff, soff.data(), (n + 1) * 8, hipMemcpyHostToDevice);
     std::vector<int32_t> hidx((size_t)soff[n]);
     if (e == hipSuccess) {
         sphe_launch_neighbours(c->D, scene, doff, dcnt, didx, c->stream);

@@ -587,3 +587,45 @@ def test_many_particles_a_tile(n, precision):
     for a, b in zip(ctxs[0].state_f64(sid), ctxs[1].state_f64(sid)):
         assert np.array_equal(a, b)
     assert ctxs[0].status() == 0
+
+
+def test_contexts_of_several_threads():
+    """Threads with a context each, that capture sequences of new lengths while
+    others upload, download, grow their lists and inspect: no call fails and
+    every state is that of the same calls in one thread."""
+    import threading
+
+    def work(i):
+        ctx = sphe.Context()
+        ctx.set_list_capacity(32)
+        sid = ctx.add_synthetic(scenes.dam_break_scene(60 + i, 1500 + 100 * i, 0.3, 64))
+        out = []
+        ctx.step(20)
+        ctx.save_state()
+        for k in (3, 4, 5, 3, 4, 5, 40, 7, 40, 7, 9, 9):
+            ctx.step(k)
+            out += ctx.state_f64(sid)
+            ctx.particle(sid, 5)
+            out.append(ctx.terrain_heights(sid))
+            if k == 7:
+                ctx.set_particles(sid, ctx.positions(sid), ctx.velocities(sid))
+            if k == 40:
+                ctx.restore_state()
+        return out
+    want = [work(i) for i in range(6)]
+    for _ in range(4):
+        got, failed = [None] * 6, []
+
+        def run(i):
+            try:
+                got[i] = work(i)
+            except Exception as e:  # noqa: BLE001  (reported below)
+                failed.append(e)
+        threads = [threading.Thread(target=run, args=(i,)) for i in range(6)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert not failed, failed
+        for a, b in zip(got, want):
+            assert all(np.array_equal(x, y) for x, y in zip(a, b))
