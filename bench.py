@@ -382,7 +382,7 @@ def summarize_profiles(base, workload, steps):
 
     def short(n):
         m = re.search(r"(k_[a-z0-9_]+)", n)
-        return m.group(1).replace("_quad", "") if m else n[:40]  # density for four lanes: k_density_quad
+        return m.group(1) if m else n[:40]
 
     def rows(name, sql):
         db = os.path.join(base, name, "run_results.db")
@@ -432,13 +432,14 @@ def summarize_profiles(base, workload, steps):
         hbm = (f * fscale + w * wscale) * 1024 if f is not None and w is not None else None
         lines.append(f"| {k} | {len(v)} | {wnd:.1f} | {rep:.1f} | {100 * sum(v) / total:.1f} | {f or 0:.0f} | "
                      f"{w or 0:.0f} | {(hbm or 0) / 1e6:.1f} | {(vi / wv) if vi and wv else 0:.0f} | {wv or 0:.0f} |")
-        key = k.replace("k_", "").replace("_f32", "").replace("_count", "")
+        # the pass's name in the bench line (density for four lanes: k_density_quad)
+        key = k.replace("k_", "").replace("_f32", "").replace("_count", "").replace("_quad", "")
         out[key] = dict(hbm_bytes=hbm, valu_insts=vi, waves=wv, avg_us_replay=rep, avg_us_window=wnd)
         if k in stall:
             out[key]["stall"] = {c: mean(win(x)) for c, x in stall[k].items()}
     lines += ["", "Stall counters per launch (wave-cycles summed over the device; GRBM_GUI_ACTIVE summed over "
                   "the XCDs):", ""]
-    for k in ("k_force_f32", "k_density", "k_reorder"):
+    for k in ("k_force_f32", "k_density_quad", "k_density", "k_reorder"):
         for src in (stall, sq):
             if k in src:
                 lines.append(f"- {k}: " + ", ".join(f"{c} {mean(win(x)):.3e}" for c, x in sorted(src[k].items())))

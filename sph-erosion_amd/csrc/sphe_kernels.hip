@@ -474,10 +474,11 @@ __device__ __forceinline__ uint32_t word_tile(int tlog, uint32_t w) { return ((w
 
 // Counts a particle of that key into its scan tile and its cell: its rank of
 // arrival in the cell.  In the largest contexts and those of many particles a
-// tile (D.totals 0) the tile is only marked.  The lanes that count here together are mostly neighbours of one
-// tile, which takes one atomic of the wave then (with the
-// totals in tile order, and so on a few lines, the force pass took 77 us instead
-// of 57 for 262,144 particles, and 289 instead of 155 for 48 uneven scenes).
+// tile (D.totals 0) the tile is only marked.  The lanes that count here together
+// are mostly neighbours of one tile, which takes one atomic of the wave then
+// (with the totals in tile order, and so on a few lines, the force pass took 77
+// us instead of 57 for 262,144 particles, and 289 instead of 155 for 48 uneven
+// scenes).
 __device__ __forceinline__ uint32_t count_key(const DevState& D, int32_t key)
 {
     const int32_t cell = key >> D.sub_log2, tile = cell >> D.scan_log2;
@@ -643,12 +644,11 @@ __global__ __launch_bounds__(1024) void k_scan_tiles(const uint32_t* __restrict_
 // Where a tile's prefix (the total of the tiles before it) comes from: a word
 // that k_scan_tiles left, or the tiles' totals, added here by every block: up
 // to SCAN_SUM_TILES tiles, at most four loads a thread, while a launch costs 4
-// us.  The totals themselves are counted
-// with the particles (count_key; a pass over the counts for them took a launch:
-// 13.2 -> 7.3 us on 6.7M cells, 19.6 -> 13.8 for 96 scenes with their terrain
-// heights; for few tiles every block added the counts before its tile: 5.6 ->
-// 4.2 us on 39,000 cells), except where the atomics cost more (count_totals).  Runs of consecutive lines instead
-// of each thread's own 64 or 128 bytes: 57 -> 40 us on 16.7M cells, before that.
+// us.  The totals themselves are counted with the particles (count_key; a pass
+// over the counts for them took a launch: 13.2 -> 7.3 us on 6.7M cells, 19.6 ->
+// 13.8 for 96 scenes with their terrain heights; for few tiles every block added
+// the counts before its tile: 5.6 -> 4.2 us on 39,000 cells), except where the
+// atomics cost more (count_totals).
 enum { SCAN_PREFIX, SCAN_SUMS };
 #define SPHE_SCAN_SUM_TILES 4096
 __host__ __device__ inline int64_t scan_tiles(const DevState& D)
@@ -2370,11 +2370,11 @@ __global__ __launch_bounds__(256) void k_heights(DevState D)
     if (t0 < D.TC) heights_quad(D, t0);
 }
 
-// The particle scan's kernels.  Blocks past the nscan tiles of the first one
-// launched compute terrain heights (both need only the force pass done): from
-// the volumes the last force pass eroded, before this step's samples them.
-// first: the first step of a call, whose status word starts from 0 (later
-// kernels of the step set its bits).
+// The particle scan's kernels.  Blocks past the nscan tiles of the last one
+// launched (k_scan_cells) compute terrain heights: from the volumes the last
+// force pass eroded, before this step's samples them.  first: the first step of
+// a call, whose status word starts from 0 there (the scan's earlier launches set
+// no bits; later kernels of the step do).
 __device__ __forceinline__ bool heights_block(const DevState& D, int nscan)
 {
     if ((int)blockIdx.x < nscan) return false;

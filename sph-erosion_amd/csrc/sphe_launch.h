@@ -8,9 +8,9 @@
 // e0 / e1 (optional): profiling events that take the start of the first and
 // the end of the last kernel a launcher issues.
 void sphe_launch_hash(const DevState& D, hipStream_t st, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
-// The particle scan: counts -> cell records, the pool's claim counter reset;
-// with heights also the terrain heights, in its first launch; with first the
-// status word is cleared.
+// The particle scan: counts -> cell records, the pool's claim counter reset; in
+// its last launch also the terrain heights (heights), and the status word is
+// cleared (first), so that no launch of it before may set a status bit.
 void sphe_launch_scan_cells(const DevState& D, bool heights, bool first, hipStream_t st, hipEvent_t e0 = nullptr,
                             hipEvent_t e1 = nullptr);
 // tiles of n counts at the smallest tile size (the size of the per-tile arrays)

@@ -962,7 +962,7 @@ void launch_sort(sphe_ctx* c, bool first)
     {
         Timed t(c, "scan");
         // with erosion the terrain heights of the last force pass are computed
-        // in the scan's first launch (this step's force pass samples them)
+        // in the scan's last launch (this step's force pass samples them)
         sphe_launch_scan_cells(D, any_erosion(c, -1) && D.TC > 0, first, c->stream, t.a, t.b);
     }
     {
